@@ -249,6 +249,37 @@ int pkv_paged_attention_prefill_append(
     float scale, int dtype,
     hipStream_t stream);
 
+/* Both calls above with a workspace, so that a batch of few query rows behind long
+ * contexts (prompts whose prefix is cached, chunks of a lone prompt) can cut its contexts
+ * into runs computed by separate workgroups. k_new / v_new / slots NULL: attention only;
+ * else the append of pkv_paged_attention_prefill_append. host_context_lens /
+ * host_query_lens: the lengths in HOST memory, int64 [num_seqs], read during the call;
+ * they only decide whether and how to split (a context longer than told is still attended
+ * to whole); NULL means no split. workspace: at least
+ * pkv_paged_attention_prefill_workspace_bytes() bytes for the same sizes and lengths, else
+ * (or NULL) the batch is not split. Its first 256 KiB are never touched and the rest needs
+ * no initialisation, so one buffer can serve this call and the decode calls on a stream;
+ * calls that overlap in time need distinct workspaces. */
+int64_t pkv_paged_attention_prefill_workspace_bytes(int64_t num_seqs, int64_t num_heads, int64_t num_kv_heads,
+                                                    int64_t head_dim, int64_t num_tokens,
+                                                    const int64_t* host_context_lens,
+                                                    const int64_t* host_query_lens);
+int pkv_paged_attention_prefill_split(
+    void* out, int64_t out_stride_t, int64_t out_stride_h,
+    const void* query, int64_t q_stride_t, int64_t q_stride_h,
+    void* k_pool, void* v_pool,
+    int64_t pool_stride_block, int64_t pool_stride_slot, int64_t pool_stride_head,
+    int64_t num_blocks, int64_t block_size, int64_t num_kv_heads, int64_t head_dim,
+    const void* k_new, const void* v_new, int64_t new_stride_t, int64_t new_stride_h,
+    const int64_t* slots,
+    const int64_t* block_tables, int64_t table_stride, int64_t table_width,
+    const int64_t* context_lens, const int64_t* query_start_loc,
+    int64_t num_seqs, int64_t num_heads, int64_t num_tokens, int64_t max_query_len,
+    const int64_t* host_context_lens, const int64_t* host_query_lens,
+    float scale, int dtype,
+    void* workspace, int64_t workspace_bytes,
+    hipStream_t stream);
+
 /* ------------------------------------------------------------------ KV append
  * Scatter this pass's new K/V rows into their pool slots. Replaces
  * `_PagedCache.update` (inference_server/core/paged_executor.py:116-125):

@@ -54,6 +54,9 @@ int fill_common(AttnParams& p, const char* what, void* out, int64_t out_st, int6
     p.group = (int)(num_heads / num_kv_heads);
     p.scale_log2 = scale * kLog2e;
     p.scale = scale;
+    p.block_shift = block_size & (block_size - 1) ? -1 : 63 - __builtin_clzll((unsigned long long)block_size);
+    p.splits = 1;
+    p.split_tiles = 0x7fffffff;
     return PKV_OK;
 }
 
@@ -164,18 +167,25 @@ int decode_impl(void* out, int64_t out_stride_t, int64_t out_stride_h, const voi
         p.ws_o = (float*)((char*)workspace + w.cnt_bytes + w.mfma_pfx_bytes + w.mfma_ml_bytes);
     }
 
+    // 16-bit shapes without a decode kernel (block sizes other than 16, other head_dims and
+    // groups) run as one-token prompts on the prefill MFMA kernel, their contexts split into
+    // the workspace's partials (never more than one per 256 tokens).
+    const bool streams = decode_streams(p, dtype);
     if (app) {
-        // The streaming kernel writes the rows itself (4-byte copies: even strides and
-        // 4-byte aligned sources); any other kernel gets the append launch first.
-        const bool fuse = decode_streams(p, dtype) && app->st % 2 == 0 && app->sh % 2 == 0 &&
-                          ((uintptr_t)app->k_new | (uintptr_t)app->v_new) % 4 == 0;
-        if (fuse) {
-            p.app_k = app->k_new;
-            p.app_v = app->v_new;
-            p.app_st = app->st;
-            p.app_sh = app->sh;
-            p.app_slots = app->slots;
-        } else {
+        p.app_k = app->k_new;
+        p.app_v = app->v_new;
+        p.app_st = app->st;
+        p.app_sh = app->sh;
+        p.app_slots = app->slots;
+        // The streaming kernels write the rows themselves (4-byte copies: even strides and
+        // 4-byte aligned sources), and so does the prefill kernel (16-byte rows); any other
+        // kernel gets the append launch first.
+        const bool fuse = streams ? app->st % 2 == 0 && app->sh % 2 == 0 &&
+                                        ((uintptr_t)app->k_new | (uintptr_t)app->v_new) % 4 == 0
+                                  : prefill_tuned(p, dtype);
+        if (!fuse) {
+            p.app_k = p.app_v = nullptr;
+            p.app_slots = nullptr;
             rc = pkv_kv_append(const_cast<void*>(k_pool), const_cast<void*>(v_pool), pool_stride_block,
                                pool_stride_slot, pool_stride_head, num_blocks, block_size, num_kv_heads, head_dim,
                                app->k_new, app->v_new, app->st, app->sh, app->slots, num_seqs, dtype, stream);
@@ -192,9 +202,24 @@ int decode_impl(void* out, int64_t out_stride_t, int64_t out_stride_h, const voi
         p.ws_ml = (float*)((char*)workspace + w.cnt_bytes);
         p.ws_o = (float*)((char*)workspace + w.cnt_bytes + w.ml_bytes);
     }
-    rc = launch_decode_attention(p, dtype, stream);
+    rc = streams || dtype == PKV_FLOAT32 ? launch_decode_attention(p, dtype, stream) : PKV_EUNSUPPORTED;
     if (rc != PKV_EUNSUPPORTED) return rc;
     clear_error();
+    if (prefill_tuned(p, dtype)) {
+        if (w.max_parts > 1) {
+            const SplitPlan plan = prefill_split_plan(num_seqs, num_heads, num_kv_heads, head_dim, num_seqs, nullptr,
+                                                      nullptr, max_context_len);
+            if (plan.splits > 1 && plan.splits <= w.max_parts) {
+                p.splits = plan.splits;
+                p.split_tiles = plan.split_tiles;
+                p.split_items = plan.items;
+            }
+        }
+        if (p.splits == 1 || prefill_tuned(p, dtype)) return launch_prefill_attention(p, dtype, stream);
+        p.splits = 1;                              // the split grid is too large: unsplit
+        p.split_tiles = 0x7fffffff;
+        return launch_prefill_attention(p, dtype, stream);
+    }
     if (dtype == PKV_FLOAT32) {
         rc = launch_f32_attention(p, stream);
         if (rc != PKV_EUNSUPPORTED) return rc;
@@ -306,7 +331,8 @@ int prefill_impl(void* out, int64_t out_stride_t, int64_t out_stride_h, const vo
                  int64_t num_kv_heads, int64_t head_dim, const int64_t* block_tables, int64_t table_stride,
                  int64_t table_width, const int64_t* context_lens, const int64_t* query_start_loc,
                  int64_t num_seqs, int64_t num_heads, int64_t num_tokens, int64_t max_query_len, float scale,
-                 int dtype, const DecodeAppend* app, hipStream_t stream) {
+                 int dtype, const DecodeAppend* app, const int64_t* host_ctx, const int64_t* host_qlen, void* workspace,
+                 int64_t workspace_bytes, hipStream_t stream) {
     AttnParams p;
     int rc = fill_common(p, "paged_attention_prefill", out, out_stride_t, out_stride_h, query, q_stride_t,
                          q_stride_h, k_pool, v_pool, pool_stride_block, pool_stride_slot, pool_stride_head,
@@ -337,6 +363,24 @@ int prefill_impl(void* out, int64_t out_stride_t, int64_t out_stride_h, const vo
                                pool_stride_slot, pool_stride_head, num_blocks, block_size, num_kv_heads, head_dim,
                                app->k_new, app->v_new, app->st, app->sh, app->slots, num_tokens, dtype, stream);
             if (rc) return rc;
+        }
+    }
+    if (workspace && host_ctx && host_qlen && prefill_tuned(p, dtype)) {
+        const SplitPlan plan = prefill_split_plan(num_seqs, num_heads, num_kv_heads, head_dim, num_tokens, host_ctx,
+                                                  host_qlen, 0);
+        if (plan.splits > 1 && kMergeCounterBytes + plan.total() <= workspace_bytes) {
+            p.splits = plan.splits;
+            p.split_tiles = plan.split_tiles;
+            p.split_items = plan.items;
+            if (prefill_tuned(p, dtype)) {
+                char* base = (char*)workspace + kMergeCounterBytes;
+                p.ws_rows = (int*)base;
+                p.ws_ml = (float*)(base + plan.rows_bytes);
+                p.ws_o = (float*)(base + plan.rows_bytes + plan.ml_bytes);
+            } else {                               // the split grid is too large: unsplit
+                p.splits = 1;
+                p.split_tiles = 0x7fffffff;
+            }
         }
     }
     rc = launch_prefill_attention(p, dtype, stream);
@@ -375,7 +419,7 @@ extern "C" int pkv_paged_attention_prefill(
     return prefill_impl(out, out_stride_t, out_stride_h, query, q_stride_t, q_stride_h, k_pool, v_pool,
                         pool_stride_block, pool_stride_slot, pool_stride_head, num_blocks, block_size, num_kv_heads,
                         head_dim, block_tables, table_stride, table_width, context_lens, query_start_loc, num_seqs,
-                        num_heads, num_tokens, max_query_len, scale, dtype, nullptr, stream);
+                        num_heads, num_tokens, max_query_len, scale, dtype, nullptr, nullptr, nullptr, nullptr, 0, stream);
 }
 
 extern "C" int pkv_paged_attention_prefill_append(
@@ -393,5 +437,39 @@ extern "C" int pkv_paged_attention_prefill_append(
     return prefill_impl(out, out_stride_t, out_stride_h, query, q_stride_t, q_stride_h, k_pool, v_pool,
                         pool_stride_block, pool_stride_slot, pool_stride_head, num_blocks, block_size, num_kv_heads,
                         head_dim, block_tables, table_stride, table_width, context_lens, query_start_loc, num_seqs,
-                        num_heads, num_tokens, max_query_len, scale, dtype, &app, stream);
+                        num_heads, num_tokens, max_query_len, scale, dtype, &app, nullptr, nullptr, nullptr, 0, stream);
+}
+
+extern "C" int64_t pkv_paged_attention_prefill_workspace_bytes(int64_t num_seqs, int64_t num_heads,
+                                                               int64_t num_kv_heads, int64_t head_dim,
+                                                               int64_t num_tokens,
+                                                               const int64_t* host_context_lens,
+                                                               const int64_t* host_query_lens) {
+    if (num_seqs <= 0 || num_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 || num_heads % num_kv_heads ||
+        !host_context_lens || !host_query_lens)
+        return 0;
+    const SplitPlan plan = prefill_split_plan(num_seqs, num_heads, num_kv_heads, head_dim, num_tokens,
+                                              host_context_lens, host_query_lens, 0);
+    return plan.splits > 1 ? kMergeCounterBytes + plan.total() : 0;
+}
+
+extern "C" int pkv_paged_attention_prefill_split(
+    void* out, int64_t out_stride_t, int64_t out_stride_h, const void* query, int64_t q_stride_t,
+    int64_t q_stride_h, void* k_pool, void* v_pool, int64_t pool_stride_block, int64_t pool_stride_slot,
+    int64_t pool_stride_head, int64_t num_blocks, int64_t block_size, int64_t num_kv_heads, int64_t head_dim,
+    const void* k_new, const void* v_new, int64_t new_stride_t, int64_t new_stride_h, const int64_t* slots,
+    const int64_t* block_tables, int64_t table_stride, int64_t table_width, const int64_t* context_lens,
+    const int64_t* query_start_loc, int64_t num_seqs, int64_t num_heads, int64_t num_tokens, int64_t max_query_len,
+    const int64_t* host_context_lens, const int64_t* host_query_lens, float scale, int dtype, void* workspace,
+    int64_t workspace_bytes, hipStream_t stream) {
+    clear_error();
+    const bool append = k_new || v_new || slots;
+    if (append && num_tokens > 0 && (!k_new || !v_new || !slots))
+        return fail(PKV_EINVAL, "paged_attention_prefill_split: null pointer");
+    const DecodeAppend app{k_new, v_new, new_stride_t, new_stride_h, slots};
+    return prefill_impl(out, out_stride_t, out_stride_h, query, q_stride_t, q_stride_h, k_pool, v_pool,
+                        pool_stride_block, pool_stride_slot, pool_stride_head, num_blocks, block_size, num_kv_heads,
+                        head_dim, block_tables, table_stride, table_width, context_lens, query_start_loc, num_seqs,
+                        num_heads, num_tokens, max_query_len, scale, dtype, append ? &app : nullptr, host_context_lens,
+                        host_query_lens, workspace, workspace_bytes, stream);
 }

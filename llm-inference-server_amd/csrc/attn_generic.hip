@@ -6,9 +6,9 @@
 // at :288) — and walks that token's keys 0..q_pos through the block table with an
 // online softmax in fp32. Lanes split head_dim (lane d, d+64, ...), so each key row
 // is one coalesced load and the score is one wave reduction. This path exists for
-// shapes the tuned kernels do not cover (block sizes 4/6, head_dim 8/12 in the unit
-// tests, fp32 prefill); the tuned decode and MFMA prefill kernels take every
-// production shape.
+// shapes the tuned kernels do not cover: in 16 bits, head_dims that are no multiple of 16
+// or outside 32..128, block sizes that are no power of two or below 8, and unaligned
+// rows; in fp32 what the fp32 kernels decline.
 #include "attention.h"
 
 namespace pkv {

@@ -1,13 +1,15 @@
-// Paged prefill / chunked-prefill attention on MFMA (gfx950), fp16/bf16, block
-// size 16, head_dim 64/128, GQA group 1/2/4/8. Other shapes take the generic kernel.
+// Paged prefill / chunked-prefill attention on MFMA (gfx950), fp16/bf16, head_dim a
+// multiple of 16 from 32 to 128, any GQA group, block sizes that are powers of two from 8
+// up; decode batches whose shape the decode kernels do not take run here too (one query
+// token per sequence). Other shapes take the generic kernel.
 //
 // Prefill is compute-bound (config 4 chunks: ~926 flop per byte touched), so the
 // contraction runs on v_mfma_f32_32x32x16_{bf16,f16}. The formulation is chosen so
 // the softmax needs almost no cross-lane traffic:
 //
-//  * S^T = K · Q^T per 32-key x 32-query tile: A = K rows (from LDS), B = Q^T
+//  * S^T = K · Q^T per 32-key x 32-row tile: A = K rows (from LDS), B = Q^T
 //    (registers, loaded once). MFMA result register r of lane l holds
-//    S^T[key 8*(r/4) + 4*(l/32) + r%4][query l%32], so every lane owns ONE query's
+//    S^T[key 8*(r/4) + 4*(l/32) + r%4][row l%32], so every lane owns ONE query row's
 //    column: row max / row sum are lane-local over 32 values plus one permlane32 swap
 //    with the lane holding the other half of the keys.
 //  * P^T feeds the P·V MFMA as its B operand straight from the S^T accumulator
@@ -20,18 +22,29 @@
 //  * V^T: the 64-key V tile is staged row-major like K and read through gfx950's
 //    transposing LDS load (ds_read_b64_tr_b16): two 8-byte reads per MFMA give each
 //    lane its 8 keys of one head_dim column.
-//  * Work unit: one workgroup = (sequence, KV head, 32-query tile) x 4 waves. With a
-//    GQA group of G >= 4 the waves are 4 query heads of one KV head and share every
-//    staged K/V tile (G = 8 uses two workgroups); with G < 4 they are 4/G consecutive
-//    query tiles x G heads. K/V tiles are 64 keys (4 blocks) walked through the block
-//    table up to the causal bound of the workgroup's last query.
+//  * Work unit: one workgroup = (sequence, KV head, 128 query rows) x 4 waves of 32 rows.
+//    A query row is one (token, query head of the KV head's group) pair, row f of a
+//    sequence = token f / G, head f % G, so the rows of every group size (3 and 6
+//    included) fill the tile and all share the staged K/V tiles: 64 keys walked through
+//    the block table up to the causal bound of the workgroup's last token. A wave whose
+//    own rows end before a tile skips its products and only stages.
+//  * Split contexts: a batch of few query rows behind long contexts (cached prefixes,
+//    chunks of a lone prompt, decode rows) makes too few workgroups to fill the GPU and
+//    each walks its context serially, so the launch cuts the contexts into runs of
+//    split_tiles tiles, one workgroup each, whose (max, denominator, unnormalised output)
+//    go to the workspace in fp32 and are merged by prefill_merge_kernel. Measured, calls
+//    through the Python entry: 12 prompts of 8-61 tokens behind 0.6-7.5k, 32/8 heads, bf16,
+//    190 -> 72 us; decode of 24 sequences of up to 3k tokens, 24/8 heads, block size 32, fp16
+//    (one wave per (token, head) before), 5,100 -> 38.6 us; 12 chunks of 24-190 tokens behind
+//    up to 1.5k, 32 heads x 80, block size 32, bf16, 5,970 -> 62 us. prefill_split_plan
+//    chooses.
 //  * Two waves per SIMD (registers capped at 256 per lane): with one, every MFMA ->
 //    softmax -> MFMA dependency and every load wait idles the matrix core; two
 //    workgroups per CU interleave (config 4 chunks: 311 -> 486 TFLOP/s).
 //  * XCD-aware order: the hardware hands workgroup L to XCD L % 8 and each XCD has its
-//    own L2. Work items are numbered query block fastest, then sequence, then KV head,
-//    and XCD x takes the x-th contiguous eighth, so the workgroups that re-read one
-//    sequence's K/V tiles share an L2 instead of fetching them from HBM once per XCD.
+//    own L2. Work items are numbered query block fastest, then split, then sequence, then
+//    KV head, and XCD x takes the x-th contiguous eighth, so the workgroups that re-read
+//    one sequence's K/V tiles share an L2 instead of fetching them from HBM once per XCD.
 //    Within a sequence the query blocks go last-first (longest causal range first).
 //  * Staging: K/V tiles move HBM -> LDS by DMA (global_load_lds_dwordx4), double
 //    buffered: tile t+1 streams into one buffer pair while tile t is computed from the
@@ -43,8 +56,11 @@
 //    take per-lane offsets computed once and carry the buffer and key-group part as
 //    immediates (config 4 chunks: 337 -> 328 us for the two together).
 //    Rows are unpadded with an XOR swizzle of their 16-byte chunks (lds_swizzle), which
-//    keeps the K and transposed V reads free of bank conflicts. The tile's 4 block ids
+//    keeps the K and transposed V reads free of bank conflicts. The tile's block ids
 //    come from one vector load issued a tile ahead, so no DMA waits on a table read.
+//  * Block sizes: a wave stages 16 keys per tile as two 8-key halves, each inside one
+//    block for any power of two >= 8. Block size 16 has instances of its own (one id per
+//    wave and tile, no shifts).
 //  * Online softmax in fp32, base-2 domain, with lazy rescaling (the running max is
 //    raised only when a tile exceeds it by more than 2^8); causal mask key <= query
 //    position, applied only on tiles that cross the workgroup's first query position,
@@ -59,7 +75,8 @@ namespace {
 
 constexpr int kBS = 16;
 constexpr int kKT = 64;          // keys per staged tile
-constexpr int kQT = 32;          // queries per wave task
+constexpr int kQT = 32;          // query rows per wave
+constexpr int kRows = 4 * kQT;   // query rows per workgroup
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -117,10 +134,14 @@ __device__ __forceinline__ uint2 lds_read_tr16(const uint16_t* ptr) {
 // D = 128 (16 chunks = 256 bytes per row, one bank sweep): slot c ^ (4 (r % 4) + r / 4 % 4).
 // D = 64 (8 chunks per 128-byte row, two rows per bank sweep): rows of one parity share
 // the sweep half, so the same two rules apply to each parity: c ^ (4 bit1 + 2 bit2 + bit3).
+// Other widths only meet the first rule: rows 4 apart start in the same banks at D = 32
+// and 96 (c ^ r / 4 % 4), rows 8 apart at 48, 80 and 112 (c ^ r / 8 % 2).
 template <int D>
 __device__ __forceinline__ int lds_swizzle(int r) {
     if constexpr (D == 128) return ((r & 3) << 2) | ((r >> 2) & 3);
-    else return (((r >> 1) & 1) << 2) | (((r >> 2) & 1) << 1) | ((r >> 3) & 1);
+    else if constexpr (D == 64) return (((r >> 1) & 1) << 2) | (((r >> 2) & 1) << 1) | ((r >> 3) & 1);
+    else if constexpr (D % 32 == 0) return (r >> 2) & 3;
+    else return (r >> 3) & 1;
 }
 
 // Softmax maxima are only raised when a tile's max exceeds the running one by more
@@ -153,32 +174,26 @@ __device__ __forceinline__ void dma16(const char* addr, uint32_t lds) {
                  : "memory");
 }
 
-// One whole live 16-row block of K and V by LDS DMA: the block bases are uniform (SGPR
-// pairs) and each lane adds its fixed 32-bit offset inside the block, so an issue costs
-// one address add instead of a 64-bit multiply-add and a select per instruction.
-template <int IPB, int RPI, int ROWB>
-__device__ __forceinline__ void dma_whole_block(const char* kb, const char* vb, const uint32_t* off,
-                                                uint16_t* sk, uint16_t* sv, int row0) {
-#pragma unroll
-    for (int j = 0; j < IPB; ++j) {
-        const int dst = (row0 + j * RPI) * ROWB;
-        dma16(kb, off[j], lds_u32((char*)sk + dst));
-        dma16(vb, off[j], lds_u32((char*)sv + dst));
-    }
+// Tiles per split of a workgroup with n_tiles key tiles: its splits are of even lengths.
+__device__ __forceinline__ int split_run(int n_tiles, int splits, int split_tiles) {
+    const int n = split_count(n_tiles, splits, split_tiles);
+    return (n_tiles + n - 1) / n;
 }
 
-template <typename T, int D, int G>
+template <typename T, int D, bool BS16>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void paged_prefill_kernel(
     const AttnParams p) {
-    constexpr int NH = G >= 4 ? 4 : G;        // query heads per workgroup
-    constexpr int NQT = 4 / NH;               // 32-query tiles per workgroup
-    constexpr int HGROUPS = G / NH;           // workgroups per KV head per query block
+    static_assert(D % 16 == 0 && D >= 32 && D <= 128, "head_dim");
     constexpr int DSTEPS = D / 16;            // QK^T contraction steps
-    constexpr int DTILES = D / 32;            // P·V output d tiles
+    constexpr int DTILES = (D + 31) / 32;     // P·V output d tiles (the last may be half a tile)
     constexpr int ROWB = D * 2;               // bytes per K/V row
-    constexpr int RPI = 1024 / ROWB;          // rows per DMA instruction (64 lanes x 16 B)
-    constexpr int IPB = kBS / RPI;            // DMA instructions per 16-row block, K or V
     constexpr int CPR = ROWB / 16;            // 16-byte chunks per row
+    // DMA instructions (64 lanes x 16 B) per 16-row block, K or V; the last one is partly
+    // masked where 16 rows are not whole instructions.
+    constexpr int IPB = (kBS * CPR + 63) / 64;
+    constexpr bool kWholeDma = kBS * CPR % 64 == 0;
+    // Rows of one instruction all in one 8-row half of the block: the half's base is uniform.
+    constexpr bool kHalfDma = 64 % CPR == 0 && 64 / CPR <= 8;
 
     // Two K/V tile buffers, distinct objects so the compiler can tell a DMA into one
     // from reads of the other (it waits on a pending LDS DMA only before reading the
@@ -188,79 +203,48 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
     __shared__ __attribute__((aligned(1024))) uint16_t s_k1[kKT * D];
     __shared__ __attribute__((aligned(1024))) uint16_t s_v1[kKT * D];
 
-    // XCD-ordered work item of this workgroup (the grid is padded to a multiple of 8).
-    const int64_t n_qb = (p.max_query_len + NQT * kQT - 1) / (NQT * kQT);
-    const int64_t n_items = n_qb * p.num_seqs * p.num_kv_heads * HGROUPS;
-    const int64_t per_xcd = (n_items + 7) / 8;
-    const int64_t item = (int64_t)(blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    if (item >= n_items) return;
-    // Query blocks of a sequence run last-first: the last block sees the most keys
-    // (causal), so the longest workgroups are dispatched first and the short ones fill
-    // the tail (config 4 chunks 335 -> 331 us).
-    const int qblock = (int)(n_qb - 1 - item % n_qb);
-    const int seq_slot = (int)((item / n_qb) % p.num_seqs);
-    const int hy = (int)(item / (n_qb * p.num_seqs));
-    const int kvh = hy / HGROUPS;
-    const int hgroup = hy % HGROUPS;
-    // Sequences longest first (prefill_seq, attention.h).
-    const PrefillSeq ps = prefill_seq(p, seq_slot, kBS);
-    const int seq = ps.seq;
-    const int64_t q_first = ps.q_first;
-    const int q_len = ps.q_len;
-    const int ctx = ps.ctx;
-    const int q0 = qblock * NQT * kQT;        // first query (within the sequence) of this workgroup
-    if (q0 >= q_len) return;
+    // This workgroup's work item (prefill_item, attention.h).
+    PrefillItem it;
+    if (!prefill_item<kRows, kKT>(p, BS16 ? kBS : p.block_size, it)) return;
+    const uint32_t G = (uint32_t)p.group;
+    const int kvh = it.kvh, split = it.split, seq = it.seq;
+    const int64_t q_first = it.q_first;
+    const int q_len = it.q_len;
+    const int ctx = it.ctx;
+    const int n_rows = q_len * (int)G;        // query rows of the sequence
+    const int row0 = it.row_tile * kRows;     // first row of this workgroup
     const int pos0 = ctx - q_len;             // position of query 0
-    const int q_last = (q0 + NQT * kQT < q_len ? q0 + NQT * kQT : q_len) - 1;
+    const int rows = n_rows - row0 < kRows ? n_rows - row0 : kRows;
+    const int q0 = (int)((uint32_t)row0 / G);                    // first and last token of this workgroup
+    const int q_last = (int)((uint32_t)(row0 + rows - 1) / G);
     const int kmax = pos0 + q_last + 1;       // keys [0, kmax) are visible to this workgroup
     if (kmax <= 0) return;
     const int first_pos = pos0 + q0;          // smallest query position in the workgroup
+    // This workgroup's run of key tiles.
+    const int n_tiles = (kmax + kKT - 1) / kKT;
+    int t_begin = 0, t_end = n_tiles, run = n_tiles;
+    if (it.splits > 1) {
+        run = split_run(n_tiles, it.splits, p.split_tiles);
+        t_begin = split * run;
+        if (t_begin >= n_tiles) return;
+        t_end = n_tiles - t_begin < run ? n_tiles : t_begin + run;
+    }
 
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int h = lane >> 5;                  // half of the wave
-    const int col = lane & 31;                // query column / MFMA row-col index
-    const int head = kvh * G + hgroup * NH + wave % NH;
-    const int qt = q0 + (wave / NH) * kQT;    // this wave's first query
-    const int my_q = qt + col;                // this lane's query (may be >= q_len: not stored)
+    const int col = lane & 31;                // query row of the wave / MFMA row-col index
+    // This lane's query row: token my_q, head my_head of the group. Rows past the last one
+    // repeat it (computed, not stored).
+    const int wrow = wave * kQT + col;
+    const bool my_live = wrow < rows;
+    const uint32_t my_row = (uint32_t)(row0 + (my_live ? wrow : rows - 1));
+    const int my_q = (int)(my_row / G);
+    const int my_head = kvh * (int)G + (int)(my_row - (uint32_t)my_q * G);
     const int my_pos = pos0 + my_q;
-
-    // Q^T B operand: lane supplies Q[query my_q][d = 16*step + 8*h .. +8].
-    u32x4 qfrag[DSTEPS];
-    {
-        const int qq = my_q < q_len ? my_q : q_len - 1;
-        const char* qrow = reinterpret_cast<const char*>(p.q) +
-                           ((q_first + qq) * p.q_st + (int64_t)head * p.q_sh) * (int64_t)sizeof(T);
-#pragma unroll
-        for (int s = 0; s < DSTEPS; ++s) {
-            const Vec16 v = load16(qrow + (s * 16 + h * 8) * (int)sizeof(T));
-            qfrag[s] = u32x4{v.w[0], v.w[1], v.w[2], v.w[3]};
-        }
-    }
-
-    // Fused KV append (p.app_k set): this workgroup's own query tokens' new K/V rows go
-    // to their pool slots (KV-head group 0 of the KV head writes them). Nothing in this
-    // launch reads those slots: every workgroup stages positions >= pos0 from the
-    // source rows instead (dma_tile), so no workgroup waits for another.
-    const bool fused = p.app_k != nullptr;
-    if (fused && hgroup == 0) {
-        constexpr int LPR = ROWB / 16;          // lanes per row, 16 bytes each
-        constexpr int RPW = 64 / LPR;           // rows per wave instruction
-        const int n_tok = q_len - q0 < NQT * kQT ? q_len - q0 : NQT * kQT;
-        const int64_t pool_slots = p.num_blocks * kBS;
-        for (int i = wave * RPW + lane / LPR; i < n_tok; i += 4 * RPW) {
-            const int64_t tok = q_first + q0 + i;
-            const int64_t slot = p.app_slots[tok];
-            if ((uint64_t)slot >= (uint64_t)pool_slots) continue;     // outside the pool: skipped
-            const int64_t src = (tok * p.app_st + (int64_t)kvh * p.app_sh) * (int64_t)sizeof(T) + (lane % LPR) * 16;
-            const int64_t dst = ((slot / kBS) * p.sb + (slot % kBS) * p.ss + (int64_t)kvh * p.sh) * (int64_t)sizeof(T) +
-                                (lane % LPR) * 16;
-            store16(reinterpret_cast<char*>(const_cast<void*>(p.k)) + dst,
-                    load16(reinterpret_cast<const char*>(p.app_k) + src));
-            store16(reinterpret_cast<char*>(const_cast<void*>(p.v)) + dst,
-                    load16(reinterpret_cast<const char*>(p.app_v) + src));
-        }
-    }
+    // Keys visible to this wave's rows (0: it has none, and only stages).
+    const int wave_rows = rows - wave * kQT < kQT ? rows - wave * kQT : kQT;
+    const int wave_kmax = wave_rows > 0 ? pos0 + (int)((uint32_t)(row0 + wave * kQT + wave_rows - 1) / G) + 1 : 0;
 
     f32x16 o[DTILES];
 #pragma unroll
@@ -273,32 +257,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
     const int64_t block_bytes = p.sb * (int64_t)sizeof(T);
     const int64_t slot_bytes = p.ss * (int64_t)sizeof(T);
 
-    // Block ids of 64-key tile kt: lane l holds entry 4 kt + l % 4, the index clamped to
-    // the last block with a visible key, so every lane loads a valid table entry without
-    // a branch (kmax <= context <= table width x 16). A block at or beyond kmax is staged
-    // by position, never from its id: dma_tile sends it to the redirect path.
-    const int nb_last = (kmax - 1) / kBS;
+    // Block ids of 64-key tile kt: lane l holds the block of the tile's 8-key half-group
+    // l % 8 (block size 16: of its 16-key group l % 4), the index clamped to the last block
+    // with a visible key, so every lane loads a valid table entry without a branch (kmax <=
+    // context <= table width x block size). A group at or beyond kmax is staged by
+    // position, never from its id: dma_tile sends it to the redirect path.
+    const int nb_last = BS16 ? (kmax - 1) / kBS : (kmax - 1) >> p.block_shift;
     auto tile_ids = [&](int kt) -> int64_t {
-        const int b = kt * (kKT / kBS) + (lane & 3);
+        const int b = BS16 ? kt * (kKT / kBS) + (lane & 3) : (kt * kKT + 8 * (lane & 7)) >> p.block_shift;
         return table[b < nb_last ? b : nb_last];
     };
     // Tile staging by LDS DMA (global_load_lds_dwordx4: lane i's 16 bytes land at the
-    // instruction's LDS base + 16 i, no registers involved). Wave w stages block w of
-    // the tile (16 rows) for K and V; instruction j covers rows 16 w + RPI j .. +RPI.
-    // Rows at or beyond kmax, and blocks whose id is outside the pool, are redirected
-    // to the tile's first row (a valid key): masked to -inf in S, so their finite V rows
-    // get probability 0.
-    const int dma_row = lane / CPR;           // row within the instruction's RPI rows
-    const int dma_slot = lane % CPR;          // physical 16-byte slot written by this lane
-    // This lane's byte offset inside a block for each of its DMA instructions (the row
-    // within the block and the swizzled source chunk), fixed for the whole kernel.
+    // instruction's LDS base + 16 i, no registers involved). Wave w stages keys 16 w ..
+    // 16 w + 15 of the tile for K and V; instruction j writes chunks 64 j .. 64 j + 63 of
+    // those 16 rows. Rows at or beyond kmax, and blocks whose id is outside the pool, are
+    // redirected to the tile's first row (a valid key): masked to -inf in S, so their
+    // finite V rows get probability 0.
+    // Row within the 16 and swizzled source chunk of this lane's instruction j.
+    auto dma_row = [&](int j) { return (64 * j + lane) / CPR; };
+    auto dma_chunk = [&](int j) { return (64 * j + lane) % CPR ^ lds_swizzle<D>((64 * j + lane) / CPR); };
+    // This lane's byte offset inside an 8-row half (inside the block at block size 16) for
+    // each of its DMA instructions, fixed for the whole kernel.
     uint32_t lane_off[IPB];
 #pragma unroll
-    for (int j = 0; j < IPB; ++j) {
-        const int r = wave * kBS + j * RPI + dma_row;
-        lane_off[j] = (uint32_t)((r % kBS) * slot_bytes) + (uint32_t)((dma_slot ^ lds_swizzle<D>(r)) * 16);
-    }
+    for (int j = 0; j < IPB; ++j)
+        lane_off[j] = (uint32_t)((BS16 ? dma_row(j) : dma_row(j) & 7) * slot_bytes) + (uint32_t)(dma_chunk(j) * 16);
     const bool offs_fit = kBS * slot_bytes + ROWB <= (int64_t)0xffffffff;
+    const bool fused = p.app_k != nullptr;
     // With a fused append, key positions >= pos0 (this pass's new tokens) come from the
     // source rows: key position j is packed token q_first + j - pos0.
     const int new_from = fused ? pos0 : 0x7fffffff;
@@ -308,14 +293,39 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
                              : nullptr;
     const int64_t new_row_bytes = p.app_st * (int64_t)sizeof(T);
     auto dma_tile = [&](int kt, int64_t ids, uint16_t* sk, uint16_t* sv) {
+        const int row0 = kt * kKT + wave * kBS;                       // first key of this wave's group
+        // Bytes from the pool head's base to the group's two 8-key halves.
         const int64_t id0 = readlane64(ids, 0);
-        const int64_t idw = readlane64(ids, wave);
-        const bool okw = (uint64_t)idw < (uint64_t)p.num_blocks;
-        const int row0 = kt * kKT + wave * kBS;                       // first key of this wave's block
+        int64_t idw, idw2, half0, half1;
+        if constexpr (BS16) {
+            idw = idw2 = readlane64(ids, wave);
+            half0 = idw * block_bytes;
+            half1 = half0 + 8 * slot_bytes;
+        } else {
+            idw = readlane64(ids, 2 * wave);
+            idw2 = readlane64(ids, 2 * wave + 1);
+            half0 = idw * block_bytes + (row0 & (p.block_size - 1)) * slot_bytes;
+            half1 = idw2 * block_bytes + ((row0 + 8) & (p.block_size - 1)) * slot_bytes;
+        }
+        const bool okw = ((uint64_t)idw < (uint64_t)p.num_blocks) & ((uint64_t)idw2 < (uint64_t)p.num_blocks);
         // The common case; one uniform branch (bitwise &: no short-circuit branches).
         if (okw & offs_fit & (row0 + kBS <= kmax) & (row0 + kBS <= new_from)) {
-            dma_whole_block<IPB, RPI, ROWB>(kbase + idw * block_bytes, vbase + idw * block_bytes, lane_off, sk, sv,
-                                            wave * kBS);
+#pragma unroll
+            for (int j = 0; j < IPB; ++j) {
+                const int dst = wave * kBS * ROWB + j * 1024;
+                if constexpr (BS16 && kWholeDma) {
+                    dma16(kbase + half0, lane_off[j], lds_u32((char*)sk + dst));
+                    dma16(vbase + half0, lane_off[j], lds_u32((char*)sv + dst));
+                } else if constexpr (kHalfDma) {
+                    const int64_t half = 64 * j / CPR < 8 ? half0 : half1;
+                    dma16(kbase + half, lane_off[j], lds_u32((char*)sk + dst));
+                    dma16(vbase + half, lane_off[j], lds_u32((char*)sv + dst));
+                } else if (kWholeDma || 64 * j + lane < kBS * CPR) {
+                    const int64_t off = (dma_row(j) < 8 ? half0 : half1) + lane_off[j];
+                    dma16(kbase + off, lds_u32((char*)sk + dst));
+                    dma16(vbase + off, lds_u32((char*)sv + dst));
+                }
+            }
             return;
         }
         // The redirect target, key kt * kKT: with a fused append it is a new row when it
@@ -329,32 +339,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
             ksafe = knew + o;
             vsafe = vnew + o;
         } else {
-            const int64_t o = (uint64_t)id0 < (uint64_t)p.num_blocks ? id0 * block_bytes : 0;
+            const int64_t o = (uint64_t)id0 < (uint64_t)p.num_blocks
+                                  ? id0 * block_bytes + (BS16 ? 0 : (key0 & (p.block_size - 1)) * slot_bytes)
+                                  : 0;
             ksafe = kbase + o;
             vsafe = vbase + o;
         }
 #pragma unroll
         for (int j = 0; j < IPB; ++j) {
-            const int r = wave * kBS + j * RPI + dma_row;
-            const int key = kt * kKT + r;
-            const int64_t chunk = (int64_t)((dma_slot ^ lds_swizzle<D>(r)) * 16);
+            const int r = dma_row(j);
+            const int key = row0 + r;
+            const int64_t chunk = (int64_t)(dma_chunk(j) * 16);
             const char* ks;
             const char* vs;
             if (key >= new_from && key < kmax) {                      // a new row: from the source
                 const int64_t off = (q_first + key - pos0) * new_row_bytes + chunk;
                 ks = knew + off;
                 vs = vnew + off;
-            } else if (okw && key < kmax) {
-                const int64_t off = idw * block_bytes + (int64_t)(r % kBS) * slot_bytes + chunk;
+            } else if ((uint64_t)(r < 8 ? idw : idw2) < (uint64_t)p.num_blocks && key < kmax) {
+                const int64_t off = (r < 8 ? half0 : half1) + (int64_t)(r & 7) * slot_bytes + chunk;
                 ks = kbase + off;
                 vs = vbase + off;
             } else {
                 ks = ksafe + chunk;
                 vs = vsafe + chunk;
             }
-            const int dst = (wave * kBS + j * RPI) * ROWB;
-            dma16(ks, lds_u32((char*)sk + dst));
-            dma16(vs, lds_u32((char*)sv + dst));
+            const int dst = wave * kBS * ROWB + j * 1024;
+            if (kWholeDma || 64 * j + lane < kBS * CPR) {
+                dma16(ks, lds_u32((char*)sk + dst));
+                dma16(vs, lds_u32((char*)sv + dst));
+            }
         }
     };
 
@@ -386,21 +400,83 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
     }
 #pragma unroll
     for (int t = 0; t < DTILES; ++t) {
-        voff_lo[t] = (uint32_t)((4 * (grp >> 1) + tr_key) * ROWB + v_byte + (((4 * t + v_cb) ^ v_lo_swz) << 4));
-        voff_hi[t] = (uint32_t)((4 * (grp >> 1) + tr_key + 8) * ROWB + v_byte + (((4 * t + v_cb) ^ v_hi_swz) << 4));
+        // Columns past head_dim (the last tile of 48, 80, 112) re-read the tile's first
+        // chunks: their products land in output rows that are never stored.
+        const int c = 4 * t + v_cb < CPR ? 4 * t + v_cb : 4 * t + (v_cb & 1);
+        voff_lo[t] = (uint32_t)((4 * (grp >> 1) + tr_key) * ROWB + v_byte + ((c ^ v_lo_swz) << 4));
+        voff_hi[t] = (uint32_t)((4 * (grp >> 1) + tr_key + 8) * ROWB + v_byte + ((c ^ v_hi_swz) << 4));
         asm volatile("" : "+v"(voff_lo[t]), "+v"(voff_hi[t]));
     }
 
-    const int n_tiles = (kmax + kKT - 1) / kKT;
-    int64_t ids = tile_ids(0);
-    dma_tile(0, ids, s_k0, s_v0);
-    ids = tile_ids(1);
+    // The first tile's block ids, then everything that needs no id, so that one memory
+    // round trip covers them all; the fused append's stores go out behind the first DMAs
+    // (in front of them, with its row loads behind the slot's, it held every workgroup up
+    // for 5.8 us on config 4 chunks).
+    int64_t ids = tile_ids(t_begin);
+    // Q^T B operand: lane supplies Q[query my_q][d = 16*step + 8*h .. +8].
+    u32x4 qfrag[DSTEPS];
+    {
+        const char* qrow = reinterpret_cast<const char*>(p.q) +
+                           ((q_first + my_q) * p.q_st + (int64_t)my_head * p.q_sh) * (int64_t)sizeof(T);
+#pragma unroll
+        for (int s = 0; s < DSTEPS; ++s) {
+            const Vec16 v = load16(qrow + (s * 16 + h * 8) * (int)sizeof(T));
+            qfrag[s] = u32x4{v.w[0], v.w[1], v.w[2], v.w[3]};
+        }
+    }
+
+    // Fused KV append (p.app_k set): the new K/V rows of the tokens whose first query row
+    // is this workgroup's go to their pool slots (the first split writes them). Nothing in
+    // this launch reads those slots: every workgroup stages positions >= pos0 from the
+    // source rows instead (dma_tile), so no workgroup waits for another.
+    constexpr int kAppend = 4;                // 16-byte pieces of K and V in flight per thread
+    const int tok_begin = (int)(((uint32_t)row0 + G - 1) / G);
+    const int n_pieces =
+        fused && split == 0 ? ((int)(((uint32_t)(row0 + rows) + G - 1) / G) - tok_begin) * CPR : 0;
+    Vec16 app_k[kAppend], app_v[kAppend];
+    int64_t app_slot[kAppend];
+    auto append_load = [&](int i0) {
+#pragma unroll
+        for (int j = 0; j < kAppend; ++j) {
+            const int i = i0 + j * 256 + (int)threadIdx.x;
+            app_slot[j] = -1;
+            if (i < n_pieces) {
+                const int64_t tok = q_first + tok_begin + i / CPR;
+                const int64_t src = (tok * p.app_st + (int64_t)kvh * p.app_sh) * (int64_t)sizeof(T) + (i % CPR) * 16;
+                app_slot[j] = p.app_slots[tok];
+                app_k[j] = load16(reinterpret_cast<const char*>(p.app_k) + src);
+                app_v[j] = load16(reinterpret_cast<const char*>(p.app_v) + src);
+            }
+        }
+    };
+    auto append_store = [&](int i0) {
+        const int bs = BS16 ? kBS : p.block_size;
+#pragma unroll
+        for (int j = 0; j < kAppend; ++j) {
+            const int64_t slot = app_slot[j];
+            if ((uint64_t)slot >= (uint64_t)(p.num_blocks * bs)) continue;     // outside the pool: skipped
+            const int64_t blk = BS16 ? slot / kBS : slot >> p.block_shift;
+            const int64_t dst = (blk * p.sb + (slot - blk * bs) * p.ss) * (int64_t)sizeof(T) +
+                                (i0 + j * 256 + (int)threadIdx.x) % CPR * 16;
+            store16(const_cast<char*>(kbase) + dst, app_k[j]);
+            store16(const_cast<char*>(vbase) + dst, app_v[j]);
+        }
+    };
+    if (n_pieces) append_load(0);
+    dma_tile(t_begin, ids, s_k0, s_v0);
+    ids = tile_ids(t_begin + 1);
+    for (int i0 = 0; i0 < n_pieces; i0 += kAppend * 256) {
+        if (i0) append_load(i0);
+        append_store(i0);
+    }
     // One tile: wait for this wave's DMA of tile kt, meet the other waves (their DMAs
     // have landed and they are done with tile kt-1, so its buffer is free), compute S^T,
     // start the DMA of tile kt+1 into the free buffer, then the softmax and P·V.
     auto tile = [&](int kt, const uint16_t* tile_k, const uint16_t* tile_v, uint16_t* nk, uint16_t* nv) {
         __builtin_amdgcn_s_waitcnt(0);
         lds_barrier();
+        // None of this wave's rows sees the tile: it only stages.
+        const bool sees = kt * kKT < wave_kmax;
 
         // ---- S^T for 64 keys: two 32-key MFMA tiles.
         // Both 32-key halves' K fragments first, then the two accumulators' MFMAs
@@ -409,7 +485,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
         // rather than holding these MFMAs back (config 4 chunks: 348.5 -> 341 us).
         __builtin_amdgcn_s_setprio(1);
         f32x16 st[2];
-        {
+        if (sees) {
             u32x4 kf[2][DSTEPS];
 #pragma unroll
             for (int half = 0; half < 2; ++half) {
@@ -432,10 +508,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
         // The next tile's DMA goes out after the S^T MFMAs (issued at the tile's top, it
         // delayed them: config 4 chunks 332 -> 325 us for the move, with the DMA still
         // visible to the compiler; 318 vs 310 us between the two places with it hidden).
-        if (kt + 1 < n_tiles) {
+        if (kt + 1 < t_end) {
             dma_tile(kt + 1, ids, nk, nv);
             ids = tile_ids(kt + 2);
         }
+        if (!sees) return;
         // ---- causal mask only on tiles that cross the workgroup's first query position.
         if (kt * kKT + kKT - 1 > first_pos) {
 #pragma unroll
@@ -498,73 +575,233 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
         }
     };
     // Two tiles per trip, so every buffer reference names a fixed array.
-    for (int kt = 0; kt < n_tiles; kt += 2) {
+    for (int kt = t_begin; kt < t_end; kt += 2) {
         tile(kt, s_k0, s_v0, s_k1, s_v1);
-        if (kt + 1 < n_tiles) tile(kt + 1, s_k1, s_v1, s_k0, s_v0);
+        if (kt + 1 < t_end) tile(kt + 1, s_k1, s_v1, s_k0, s_v0);
     }
 
-    // ---- normalise and store: lane holds query my_q, d = 32 t + 8 (r/4) + 4 h + r%4.
-    if (my_q < q_len) {
-        const float inv = 1.f / l_run;
-        T* orow = reinterpret_cast<T*>(p.out) + (q_first + my_q) * p.out_st + (int64_t)head * p.out_sh;
+    // ---- store: the lane holds d = 32 t + 8 (r/4) + 4 h + r%4 of its query row.
+    if (!my_live) return;
+    const int64_t tok = q_first + my_q;
+    if (run < n_tiles) {
+        // One of several splits: this row's partial, unnormalised.
+        const int64_t row = tok * p.num_heads + my_head;
+        const int64_t slot = row * p.splits + split;
+        float* po = p.ws_o + slot * D + 4 * h;
 #pragma unroll
         for (int t = 0; t < DTILES; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int d = 32 * t + 8 * i + 4 * h;
-                const uint32_t w0 = Mfma<T>::pack(o[t][4 * i] * inv, o[t][4 * i + 1] * inv);
-                const uint32_t w1 = Mfma<T>::pack(o[t][4 * i + 2] * inv, o[t][4 * i + 3] * inv);
-                *reinterpret_cast<uint2*>(orow + d) = make_uint2(w0, w1);
-            }
+            for (int i = 0; i < 4; ++i)
+                if (32 * t + 8 * i < D)
+                    *reinterpret_cast<float4*>(po + 32 * t + 8 * i) =
+                        make_float4(o[t][4 * i], o[t][4 * i + 1], o[t][4 * i + 2], o[t][4 * i + 3]);
+        if (h == 0) *reinterpret_cast<float2*>(p.ws_ml + slot * 2) = make_float2(m_run, l_run);
+        // Splits that hold a key this row sees (the merge reads only those).
+        if (p.ws_rows && h == 0 && split == 0) p.ws_rows[row] = my_pos / (run * kKT) + 1;
+        return;
     }
+    if (p.ws_rows && h == 0) p.ws_rows[tok * p.num_heads + my_head] = 0;   // finished here
+    const float inv = 1.f / l_run;
+    T* orow = reinterpret_cast<T*>(p.out) + tok * p.out_st + (int64_t)my_head * p.out_sh;
+#pragma unroll
+    for (int t = 0; t < DTILES; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (32 * t + 8 * i >= D) continue;
+            const int d = 32 * t + 8 * i + 4 * h;
+            const uint32_t w0 = Mfma<T>::pack(o[t][4 * i] * inv, o[t][4 * i + 1] * inv);
+            const uint32_t w1 = Mfma<T>::pack(o[t][4 * i + 2] * inv, o[t][4 * i + 3] * inv);
+            *reinterpret_cast<uint2*>(orow + d) = make_uint2(w0, w1);
+        }
 }
 
-// Workgroups of the MFMA kernel's flat grid for group size `group`: the work items
-// padded to a multiple of 8 (the kernel maps the grid to work items XCD by XCD and
-// retires the padding). -1 for a group the kernel has no instance of.
-int64_t prefill_workgroups(const AttnParams& p, int group) {
-    if (group != 1 && group != 2 && group != 4 && group != 8) return -1;
-    const int nh = group >= 4 ? 4 : group;
-    const int nqt = 4 / nh;
-    const int64_t items = ceil_div(p.max_query_len, nqt * kQT) * p.num_seqs * p.num_kv_heads * (group / nh);
+// Merge of the splits, launched after the kernel above on the same stream: D / 4 lanes per
+// query row (four head_dim elements each), log-sum-exp rule over the row's splits in key
+// order. Rows that one workgroup finished are marked 0 and skipped, as are tokens of no
+// sequence (rows the launch above never wrote: tokens past query_start_loc's end). Bound by
+// the latency of its two dependent loads and by workgroup launches, hence as many rows per
+// wave as fit.
+template <int D>
+constexpr int kMergeRows = 4 * (64 / (D / 4));   // query rows per 256-thread workgroup
+
+template <typename T, int D>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(const AttnParams p) {
+    constexpr int LPR = D / 4, RPW = 64 / LPR;
+    const int lane = lane_id();
+    if (lane >= RPW * LPR) return;
+    const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW + lane / LPR;
+    const int64_t end = p.qsl ? p.qsl[p.num_seqs] : p.num_tokens;
+    if (row >= end * p.num_heads) return;
+    const int64_t tok = row / p.num_heads;
+    int n;
+    if (p.qsl) {
+        n = p.ws_rows[row];
+    } else {
+        // A decode batch: the splits of the row's own context, none if it has only one.
+        const int64_t cap = p.table_width * p.block_size;
+        int64_t c = p.ctx_lens[tok];
+        c = c < cap ? c : cap;
+        const int tiles = (int)((c + kKT - 1) / kKT);
+        const int run = split_run(tiles, p.splits, p.split_tiles);
+        n = run > 0 && run < tiles ? (tiles + run - 1) / run : 0;
+    }
+    if (n <= 0 || n > p.splits) return;
+    const int d = 4 * (lane % LPR);
+    const float2* ml = reinterpret_cast<const float2*>(p.ws_ml) + row * p.splits;
+    const float* o = p.ws_o + row * p.splits * D + d;
+    constexpr int CH = 8;   // splits whose loads are in flight together
+    float M = kNegInf, L = 0.f;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int s0 = 0; s0 < n; s0 += CH) {
+        float2 mlv[CH];
+        float4 ov[CH];
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            const bool in = s0 + j < n;
+            mlv[j] = in ? ml[s0 + j] : make_float2(kNegInf, 0.f);
+            ov[j] = in ? *reinterpret_cast<const float4*>(o + (int64_t)(s0 + j) * D) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        float Mc = M;
+#pragma unroll
+        for (int j = 0; j < CH; ++j) Mc = fmaxf(Mc, mlv[j].x);
+        const float rescale = M == kNegInf ? 0.f : fast_exp2(M - Mc);
+        L *= rescale;
+        acc.x *= rescale;
+        acc.y *= rescale;
+        acc.z *= rescale;
+        acc.w *= rescale;
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            const float sc = mlv[j].x == kNegInf ? 0.f : fast_exp2(mlv[j].x - Mc);
+            L += sc * mlv[j].y;
+            acc.x += sc * ov[j].x;
+            acc.y += sc * ov[j].y;
+            acc.z += sc * ov[j].z;
+            acc.w += sc * ov[j].w;
+        }
+        M = Mc;
+    }
+    T* orow = reinterpret_cast<T*>(p.out) + tok * p.out_st + (row - tok * p.num_heads) * p.out_sh + d;
+    const float inv = 1.f / L;
+    *reinterpret_cast<uint2*>(orow) =
+        make_uint2(Mfma<T>::pack(acc.x * inv, acc.y * inv), Mfma<T>::pack(acc.z * inv, acc.w * inv));
+}
+
+// Workgroups of the flat grid, a multiple of 8: the splits' items, or room for every row
+// tile the batch can hold (a sequence's last tile may be partial), whichever is more.
+int64_t prefill_workgroups(const AttnParams& p) {
+    const int64_t grid = ceil_div((int64_t)p.max_query_len * p.group, kRows) * p.num_seqs;
+    const int64_t fill = p.num_tokens * p.group / kRows + p.num_seqs;
+    int64_t items = (grid < fill || p.num_seqs > kPrefillSortSeqs ? grid : fill) * p.num_kv_heads;
+    if (p.splits > 1 && p.split_items > items) items = p.split_items;
     return ceil_div(items, 8) * 8;
 }
 
-template <typename T, int D, int G>
-int launch_g(const AttnParams& p, hipStream_t stream) {
-    const int64_t wgs = prefill_workgroups(p, G);
+template <typename T, int D, bool BS16>
+int launch_one(const AttnParams& p, hipStream_t stream) {
+    const int64_t wgs = prefill_workgroups(p);
     if (wgs == 0) return PKV_OK;
-    paged_prefill_kernel<T, D, G><<<dim3((unsigned)wgs), 256, 0, stream>>>(p);
-    return check_launch("paged prefill attention");
-}
-
-template <typename T, int D>
-int launch_d(const AttnParams& p, hipStream_t stream) {
-    switch (p.group) {
-        case 1: return launch_g<T, D, 1>(p, stream);
-        case 2: return launch_g<T, D, 2>(p, stream);
-        case 4: return launch_g<T, D, 4>(p, stream);
-        case 8: return launch_g<T, D, 8>(p, stream);
-        default: return PKV_EUNSUPPORTED;
-    }
+    paged_prefill_kernel<T, D, BS16><<<dim3((unsigned)wgs), 256, 0, stream>>>(p);
+    const int rc = check_launch("paged prefill attention");
+    if (rc || p.splits == 1) return rc;
+    const int64_t rows = p.num_tokens * p.num_heads;
+    prefill_merge_kernel<T, D><<<dim3((unsigned)ceil_div(rows, kMergeRows<D>)), 256, 0, stream>>>(p);
+    return check_launch("paged prefill merge");
 }
 
 template <typename T>
 int launch_t(const AttnParams& p, hipStream_t stream) {
-    if (p.head_dim == 64) return launch_d<T, 64>(p, stream);
-    if (p.head_dim == 128) return launch_d<T, 128>(p, stream);
+    const bool bs16 = p.block_size == kBS;
+    switch (p.head_dim) {
+        case 32: return launch_one<T, 32, false>(p, stream);
+        case 48: return launch_one<T, 48, false>(p, stream);
+        case 64: return bs16 ? launch_one<T, 64, true>(p, stream) : launch_one<T, 64, false>(p, stream);
+        case 80: return launch_one<T, 80, false>(p, stream);
+        case 96: return launch_one<T, 96, false>(p, stream);
+        case 112: return launch_one<T, 112, false>(p, stream);
+        case 128: return bs16 ? launch_one<T, 128, true>(p, stream) : launch_one<T, 128, false>(p, stream);
+    }
     return PKV_EUNSUPPORTED;
 }
 
 }  // namespace
 
+// The cheapest of a few run lengths in a model of the launch, in us, from per-workgroup
+// time stamps: a workgroup takes kStart before and after its tiles and then a tile's time,
+// 1.1 us alone and 1.9 us where the GPU is full (two workgroups per CU at head_dim 112 and
+// 128, three at 80 and 96, four below: registers and LDS); once there are more workgroups
+// than slots the last ones start late, half a workgroup's time on average; a split launch
+// adds the merge kernel, and its partials' way to memory at ~4.5 TB/s.
+SplitPlan prefill_split_plan(int64_t num_seqs, int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                             int64_t num_tokens, const int64_t* ctx, const int64_t* qlen, int64_t max_context_len) {
+    constexpr float kStart = 6.f, kTileAlone = 1.1f, kTileFull = 1.9f, kMerge = 4.f, kBytesPerUs = 4.5e6f;
+    constexpr float kWorth = 0.85f;              // the gain that a split has to promise
+    constexpr int64_t kMaxBytes = 128 << 20;
+    static const int kRuns[] = {4, 5, 6, 8, 10, 12, 14, 17, 20, 24, 28, 34, 40, 48, 56, 68, 80, 96, 112, 136, 160, 192};
+    SplitPlan plan{1, 0x7fffffff, 0, 0, 0, 0};
+    if (num_seqs < 1 || num_seqs > kPrefillSortSeqs || num_tokens < 1 || num_kv_heads < 1 || head_dim < 1) return plan;
+    const int64_t group = num_heads / num_kv_heads;
+    const int64_t slots = head_dim >= 112 ? 512 : head_dim >= 80 ? 768 : 1024;
+    // Without the lengths (a decode call): contexts spread evenly up to the bound.
+    auto tiles_of = [&](int64_t i) {
+        return ceil_div(ctx ? ctx[i] : max_context_len * (2 * i + 1) / (2 * num_seqs), kKT);
+    };
+    auto rows_of = [&](int64_t i) { return (qlen ? qlen[i] : 1) * group; };
+    auto launch_us = [&](int64_t wgs, int64_t longest, int64_t work) {
+        const float full = wgs < slots ? (float)wgs / slots : 1.f;
+        const float tile = kTileAlone + (kTileFull - kTileAlone) * full;
+        const float one = longest * tile + kStart;
+        if (wgs <= slots) return one;
+        const float all = (work * tile + wgs * kStart) / slots + 0.5f * one;
+        return all > one ? all : one;
+    };
+    int64_t wgs = 0, work = 0, longest = ctx ? 0 : ceil_div(max_context_len, kKT);
+    for (int64_t i = 0; i < num_seqs; ++i) {
+        const int64_t t = tiles_of(i), w = ceil_div(rows_of(i), kRows) * num_kv_heads;
+        if (t <= 0 || w <= 0) continue;
+        wgs += w;
+        work += w * t;
+        longest = longest > t ? longest : t;
+        if (wgs >= 2 * slots) return plan;       // the GPU is full, and stays so
+    }
+    if (longest * kKT <= kSplitMinContext) return plan;
+    const int64_t rows = num_tokens * num_heads;
+    float best = kWorth * launch_us(wgs, longest, work);
+    for (const int64_t run : kRuns) {
+        if (run >= longest) break;
+        const int64_t splits = ceil_div(longest, run);
+        if (rows * splits * (head_dim + 2) * 4 > kMaxBytes) continue;
+        int64_t n = 0, parts = 0, top = 0;
+        for (int64_t i = 0; i < num_seqs; ++i) {
+            const int64_t t = tiles_of(i), w = ceil_div(rows_of(i), kRows) * num_kv_heads;
+            if (t <= 0 || w <= 0) continue;
+            const int64_t s = ceil_div(t, run);
+            n += w * s;
+            top = top > ceil_div(t, s) ? top : ceil_div(t, s);
+            if (s > 1) parts += rows_of(i) * num_kv_heads * s;
+        }
+        const float us = launch_us(n, top, work) + kMerge + parts * (head_dim + 2) * 4 / kBytesPerUs;
+        if (us >= best) continue;
+        best = us;
+        plan.splits = (int)splits;
+        plan.split_tiles = (int)run;
+        plan.items = ctx ? n : wgs * splits;     // lengths unknown: room for all of them at the bound
+    }
+    if (plan.splits == 1) return plan;
+    auto round256 = [](int64_t b) { return ceil_div(b, 256) * 256; };
+    plan.rows_bytes = round256(rows * 4);
+    plan.ml_bytes = round256(rows * plan.splits * 8);
+    plan.o_bytes = round256(rows * plan.splits * head_dim * 4);
+    return plan;
+}
+
 bool prefill_tuned(const AttnParams& p, int dtype) {
-    if (p.block_size != kBS) return false;
-    if (p.head_dim != 64 && p.head_dim != 128) return false;
+    if (p.block_shift < 3) return false;
+    if (p.head_dim % 16 || p.head_dim < 32 || p.head_dim > 128) return false;
     if (dtype != PKV_FLOAT16 && dtype != PKV_BFLOAT16) return false;
-    // Instances exist for GQA groups 1/2/4/8 only, and the grid is one dimension.
-    const int64_t wgs = prefill_workgroups(p, p.group);
-    if (wgs < 0 || wgs > 0x7fffffff) return false;
+    // The grid is one dimension, and row numbers of a sequence stay below 2^31.
+    if (prefill_workgroups(p) > 0x7fffffff) return false;
+    if (((int64_t)p.max_query_len + kRows) * p.group > 0x7fffffff) return false;
     // Masked-off rows are staged from a valid row of the pool: needs a non-empty pool.
     if (p.num_blocks < 1) return false;
     // 16-byte rows and 8-byte output stores need aligned pointers and strides; so do the

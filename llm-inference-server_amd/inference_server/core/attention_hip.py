@@ -62,21 +62,25 @@ def _host_lengths(context_lens: torch.Tensor, query_lens: torch.Tensor) -> tuple
     if hc is None or hq is None:
         both = torch.stack([context_lens.reshape(-1).long(), query_lens.reshape(-1).long()]).cpu()
         hc, hq = both[0], both[1]
-    return hc.long(), hq.long()
+    return hc.long().contiguous(), hq.long().contiguous()
 
 
 class _Workspaces:
-    """One split-KV decode workspace per (device, stream), grown on demand and reused
-    across calls. It is zero-filled when allocated: the merge counters at its front
-    must read zero when a call starts, and every completed call leaves them zero
-    again (the partials behind them need no initialisation). Calls on one stream are
-    ordered; a different stream gets its own buffer. After a call that did not
-    complete (a launch error, a reset device), `reset()` drops the buffers so the
-    next call gets a zero-filled one."""
+    """One attention workspace per (device, stream), grown on demand and reused across
+    calls (split-KV decode and split prefill; a stream runs one call at a time). It is
+    zero-filled when allocated: the decode merge counters at its front must read zero when
+    a call starts, and every completed call leaves them zero again (the partials behind
+    them need no initialisation). A different stream gets its own buffer. Sizes are powers
+    of two and a buffer that had to grow is kept, not freed: a graph captured on that
+    stream earlier replays into it (the kept ones add up to less than the one in use).
+    Growth inside a capture is a temporary of that graph. After a call that did not
+    complete (a launch error, a reset device), `reset()` drops the buffers so the next call
+    gets a zero-filled one."""
 
     def __init__(self) -> None:
         self._lock = threading.Lock()
         self._bufs: dict[tuple[int, int], torch.Tensor] = {}
+        self._kept: list[torch.Tensor] = []
 
     def partials(self, device: torch.device, stream: int, nbytes: int) -> torch.Tensor:
         idx = device.index if device.index is not None else torch.cuda.current_device()
@@ -84,9 +88,12 @@ class _Workspaces:
         with self._lock:
             buf = self._bufs.get(key)
             if buf is None or buf.numel() < nbytes:
-                # Zero-filled once: the merge counters at its front must start at zero (every
-                # call leaves them zero again); the partials need no initialisation.
-                buf = torch.zeros(max(nbytes, 1 << 16), dtype=torch.uint8, device=device)
+                size = 1 << (max(nbytes, 1 << 16) - 1).bit_length()
+                if torch.cuda.is_current_stream_capturing():
+                    return torch.zeros(size, dtype=torch.uint8, device=device)
+                if buf is not None:
+                    self._kept.append(buf)
+                buf = torch.zeros(size, dtype=torch.uint8, device=device)
                 self._bufs[key] = buf
             return buf
 
@@ -94,6 +101,7 @@ class _Workspaces:
         """Forget every buffer (the next call on each stream allocates a zeroed one)."""
         with self._lock:
             self._bufs.clear()
+            self._kept.clear()
 
 
 _WORKSPACES = _Workspaces()
@@ -256,27 +264,25 @@ def paged_attention_hip_launch(
             qsl_host = torch.zeros(n_seqs + 1, dtype=torch.long)
             torch.cumsum(hql, 0, out=qsl_host[1:])
             qsl = facts["qsl"] = qsl_host.to(dev)
-    if append is not None:
-        rc = L.pkv_paged_attention_prefill_append(
-            out.data_ptr(), out.stride(0), out.stride(1),
-            query.data_ptr(), query.stride(0), query.stride(1),
-            *common_pool[:9],
-            k_new.data_ptr(), v_new.data_ptr(), k_new.stride(0), k_new.stride(1), slots.data_ptr(),
-            *common_pool[9:],
-            ctx_dev.data_ptr(), qsl.data_ptr(),
-            n_seqs, n_heads, n_tok, facts["max_q"],
-            float(scale), dt,
-            stream,
-        )
-        native.check(rc, "pkv_paged_attention_prefill_append")
-        return out
-    rc = L.pkv_paged_attention_prefill(
+    # Workspace for split contexts (0 bytes: a batch that is not split).
+    lens = (facts["hctx"].data_ptr(), hql.data_ptr())
+    ws_bytes = L.pkv_paged_attention_prefill_workspace_bytes(n_seqs, n_heads, n_kv, head_dim, n_tok, *lens)
+    ws_ptr, ws_size = None, 0
+    if ws_bytes:
+        ws = _WORKSPACES.partials(dev, stream, ws_bytes)
+        ws_ptr, ws_size = ws.data_ptr(), ws.numel()
+    new = (None, None, 0, 0, None) if append is None else (
+        k_new.data_ptr(), v_new.data_ptr(), k_new.stride(0), k_new.stride(1), slots.data_ptr())
+    rc = L.pkv_paged_attention_prefill_split(
         out.data_ptr(), out.stride(0), out.stride(1),
         query.data_ptr(), query.stride(0), query.stride(1),
-        *common_pool,
+        *common_pool[:9],
+        *new,
+        *common_pool[9:],
         ctx_dev.data_ptr(), qsl.data_ptr(),
-        n_seqs, n_heads, n_tok, facts["max_q"],
+        n_seqs, n_heads, n_tok, facts["max_q"], *lens,
         float(scale), dt,
+        ws_ptr, ws_size,
         stream,
     )
     native.check(rc, "pkv_paged_attention_prefill")

@@ -1,0 +1,131 @@
+"""The 16-bit prefill kernel on the shapes, groups and block sizes it takes, and its split
+contexts, against oracle.gather (the reference gather path) at the 16-bit bar of 2e-2.
+
+Contexts end on, before and behind the edges of a block, an 8-key half, a 64-key tile, a
+32-row wave and a 128-row workgroup (query rows are tokens x group heads). Decode batches
+of the shapes without a decode kernel run through it too.
+"""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+from inference_server import native
+from inference_server.core.attention_hip import attach_host, paged_attention_hip_launch
+from oracle.gather import paged_attention_gather as oracle_gather
+from oracle.kvops import kv_append
+
+TOL = 2e-2
+EDGES = [(1, 1), (7, 7), (8, 8), (9, 5), (64, 1), (63, 63), (65, 65), (130, 43), (300, 129), (257, 1)]
+DECODE = [(1, 1), (8, 1), (9, 1), (64, 1), (65, 1), (700, 1)]
+#: One prompt of a few tiles among contexts long enough to be split.
+LONG = [(3000, 1), (1500, 33), (70, 70), (5, 5), (2049, 43), (1025, 2)]
+
+
+def _batch(lengths, *, dtype, d, bs, kv, group, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    need = [-(-c // bs) for c, _ in lengths]
+    num_blocks = sum(need) + 3
+    perm = torch.randperm(num_blocks, generator=g).tolist()
+    width = max(need) + 1
+    rows = []
+    for n in need:
+        # Padding past the sequence's blocks is live ids, which a correct kernel never reads.
+        rows.append(perm[:n] + torch.randint(0, num_blocks, (width - n,), generator=g).tolist())
+        perm = perm[n:]
+    t = sum(q for _, q in lengths)
+    rand = lambda *s: torch.randn(*s, generator=g).to(dtype)  # noqa: E731
+    return dict(q=rand(t, kv * group, d), k=rand(num_blocks, bs, kv, d), v=rand(num_blocks, bs, kv, d),
+                tables=torch.tensor(rows), ctx=torch.tensor([c for c, _ in lengths]),
+                ql=torch.tensor([q for _, q in lengths]), k_new=rand(t, kv, d), v_new=rand(t, kv, d))
+
+
+def _check(b, *, fused, told=None):
+    """told: other context lengths for the host copy, which only balances the launch."""
+    d, bs = b["q"].shape[2], b["k"].shape[1]
+    first = b["ctx"] - b["ql"]
+    slots = torch.cat([b["tables"][i, torch.arange(int(f), int(f + n)) // bs] * bs
+                       + torch.arange(int(f), int(f + n)) % bs for i, (f, n) in enumerate(zip(first, b["ql"]))])
+    k, v = b["k"].cuda(), b["v"].cuda()
+    ctx = attach_host(b["ctx"].cuda(), b["ctx"] if told is None else told)
+    ql = attach_host(b["ql"].cuda(), b["ql"])
+    append = (b["k_new"].cuda(), b["v_new"].cuda(), slots.cuda()) if fused else None
+    out = paged_attention_hip_launch(b["q"].cuda(), k, v, b["tables"].cuda(), ctx, ql, d ** -0.5, append=append)
+    torch.cuda.synchronize()
+    kr, vr = b["k"], b["v"]
+    if fused:
+        bits = lambda t: t.view(torch.int16).numpy()  # noqa: E731
+        put = lambda pool, rows: torch.from_numpy(kv_append(bits(pool), bits(rows), slots.numpy()))  # noqa: E731
+        kb, vb = put(kr, b["k_new"]), put(vr, b["v_new"])
+        assert torch.equal(k.cpu().view(torch.int16), kb) and torch.equal(v.cpu().view(torch.int16), vb)
+        kr, vr = kb.view(kr.dtype), vb.view(vr.dtype)
+    ref = oracle_gather(b["q"], kr, vr, b["tables"], b["ctx"], b["ql"], d ** -0.5)
+    torch.testing.assert_close(out.cpu(), ref, atol=TOL, rtol=TOL)
+
+
+def _split_bytes(b):
+    t, heads, d = b["q"].shape
+    kv = b["k"].shape[2]
+    return native.lib().pkv_paged_attention_prefill_workspace_bytes(
+        len(b["ctx"]), heads, kv, d, t, b["ctx"].data_ptr(), b["ql"].data_ptr())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,bs,kv,group,dtype", [
+    (32, 8, 2, 1, torch.float16), (32, 16, 1, 5, torch.bfloat16), (48, 32, 2, 3, torch.float16),
+    (64, 8, 2, 3, torch.bfloat16), (64, 64, 1, 4, torch.float16), (64, 16, 2, 6, torch.float16),
+    (80, 8, 3, 1, torch.bfloat16), (80, 32, 1, 8, torch.float16), (96, 16, 2, 2, torch.bfloat16),
+    (112, 128, 1, 3, torch.float16), (128, 32, 2, 4, torch.bfloat16), (128, 8, 1, 16, torch.float16),
+    (128, 16, 1, 71, torch.bfloat16), (128, 16, 2, 3, torch.float16)])
+@pytest.mark.parametrize("lengths", [EDGES, DECODE], ids=["prompts", "decode"])
+@pytest.mark.parametrize("fused", [False, True], ids=["plain", "append"])
+def test_shapes_groups_and_block_sizes(d, bs, kv, group, dtype, lengths, fused):
+    _check(_batch(lengths, dtype=dtype, d=d, bs=bs, kv=kv, group=group, seed=d + bs + group), fused=fused)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,bs,kv,group,dtype", [
+    (64, 16, 2, 1, torch.float16), (128, 16, 2, 4, torch.bfloat16), (128, 16, 1, 3, torch.float16),
+    (80, 32, 2, 3, torch.bfloat16), (32, 8, 1, 8, torch.float16)])
+@pytest.mark.parametrize("fused", [False, True], ids=["plain", "append"])
+def test_split_contexts(d, bs, kv, group, dtype, fused):
+    b = _batch(LONG, dtype=dtype, d=d, bs=bs, kv=kv, group=group, seed=7 + d)
+    assert _split_bytes(b) > 0
+    _check(b, fused=fused)
+    # A decode batch of long contexts (a decode kernel's where one takes the shape).
+    lone = _batch([(c, 1) for c, _ in LONG], dtype=dtype, d=d, bs=bs, kv=kv, group=group, seed=9 + d)
+    _check(lone, fused=fused)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("told", [[1100] * 6, [3000, 40, 70, 5, 43, 2]], ids=["shorter", "one long"])
+def test_split_contexts_longer_than_told_are_attended_whole(told):
+    b = _batch(LONG, dtype=torch.bfloat16, d=128, bs=16, kv=2, group=4, seed=11)
+    told = torch.tensor(told)
+    heads, kv = 8, 2
+    assert native.lib().pkv_paged_attention_prefill_workspace_bytes(
+        len(told), heads, kv, 128, b["q"].shape[0], told.data_ptr(), b["ql"].data_ptr()) > 0
+    _check(b, fused=False, told=told)
+
+
+def test_split_workspace_is_host_arithmetic():
+    size = native.lib().pkv_paged_attention_prefill_workspace_bytes
+    arr = lambda v: (ctypes.c_int64 * len(v))(*v)  # noqa: E731
+
+    def need(ctx, ql, heads=32, kv=8, d=128):
+        return size(len(ctx), heads, kv, d, sum(ql), arr(ctx), arr(ql))
+
+    assert need([8192], [16]) > 256 * 1024                      # one long context: split
+    assert need([1024], [16]) == 0                              # no context past the shortest split one
+    assert need([4096] * 16, [512] * 16) == 0                   # the GPU is full without
+    assert need([8192] * 257, [1] * 257) == 0                   # more sequences than are ordered
+    assert need([8192], [16], heads=3, kv=2) == 0               # not a group
+    assert size(1, 32, 8, 128, 16, None, None) == 0
+    # Partials stay bounded whatever the batch.
+    for n in (1, 3, 12, 100):
+        for ctx in (2000, 8192, 131072):
+            for q in (1, 40, 300):
+                assert need([ctx] * n, [q] * n) <= (130 << 20) + 8 * n * q * 32 + (1 << 20)
