@@ -136,9 +136,9 @@ def check_contract(q_dim, q_shape, pool_dim, pool_shape, tables_shape, ctx_shape
     """Shape checks first, then `values()` -> (sum of query_lens, any query_len >
     context_len, any sequence needing more blocks than the table width)."""
     if q_dim != 3:
-        raise ValueError(f"query must be [num_tokens, heads, dim], got {q_shape}")
+        raise ValueError(f"query must be [num_tokens, heads, dim], got {tuple(q_shape)}")
     if pool_dim != 4:
-        raise ValueError(f"k_pool must be [blocks, block_size, kv_heads, dim], got {pool_shape}")
+        raise ValueError(f"k_pool must be [blocks, block_size, kv_heads, dim], got {tuple(pool_shape)}")
     batch = tables_shape[0]
     if tuple(ctx_shape) != (batch,) or tuple(qlens_shape) != (batch,):
         raise ValueError("context_lens and query_lens must be [batch] to match block_tables")

@@ -106,6 +106,12 @@ class _Workspaces:
 
 _WORKSPACES = _Workspaces()
 
+
+def _on_device(t: torch.Tensor, dev: torch.device) -> torch.Tensor:
+    """t as int64 on dev: itself when it is (the no-op `.to` costs a microsecond)."""
+    return t if t.dtype is torch.long and t.device == dev else t.to(device=dev, dtype=torch.long)
+
+
 _META_ATTR = "_pkv_step_meta"
 
 
@@ -113,13 +119,15 @@ def _batch_facts(context_lens: torch.Tensor, query_lens: torch.Tensor, block_siz
     """Host-side facts about one batch's lengths: the contract checks' inputs, the
     decode/prefill choice, the maxima that size the grids. The paged executor hands
     the same length tensors, with host copies attached, to every layer of a step, so
-    for attached tensors the facts are computed once and kept on context_lens, keyed
-    by the identity of both host copies (re-attaching new values invalidates them).
-    Tensors without attached copies are read afresh on every call."""
+    for attached tensors the facts are kept on context_lens, keyed by the values of both
+    host copies (new values, attached or written in place, make new facts). Tensors
+    without attached copies are read afresh on every call."""
     hc_att, hq_att = host_copy(context_lens), host_copy(query_lens)
-    cacheable = context_lens.device.type != "cpu" and hc_att is not None and hq_att is not None
-    key = (id(hc_att), id(hq_att), block_size, width)
-    if cacheable:
+    key = None
+    if hc_att is not None and hq_att is not None and context_lens.device.type != "cpu" and not (
+            hc_att.is_cuda or hq_att.is_cuda):
+        hc, hq = hc_att.numpy(), hq_att.numpy()
+        key = (hc.tobytes(), hq.tobytes(), hc.dtype, hq.dtype, block_size, width)
         hit = getattr(context_lens, _META_ATTR, None)
         if hit is not None and hit[0] == key:
             return hit[1]
@@ -134,11 +142,30 @@ def _batch_facts(context_lens: torch.Tensor, query_lens: torch.Tensor, block_siz
         "all_decode": bool((hql == 1).all()),
         "max_ctx": int(hctx.max()) if n else 0,
         "max_q": int(hql.max()) if n else 0,
-        "qsl": None,  # device query_start_loc, built on first prefill use
+        "qsl": {},  # device query_start_loc by (device, stream), built on first prefill use
     }
-    if cacheable:
+    if key is not None:
         setattr(context_lens, _META_ATTR, (key, facts))
     return facts
+
+
+def _query_start(facts: dict, dev: torch.device, stream: int) -> torch.Tensor:
+    """Device query_start_loc of a batch, uploaded once per step and stream. The upload
+    leaves from pinned memory: a pageable one waits for everything queued on the stream,
+    which cost a step one such wait per layer (3 GPT-2 prompts, 31 us a call of which the
+    kernel is 12)."""
+    capturing = torch.cuda.is_current_stream_capturing()
+    # A graph must not hold a buffer that lives as long as this step's length tensors:
+    # inside a capture the pageable upload is refused by the runtime.
+    qsl = None if capturing else facts["qsl"].get((dev, stream))
+    if qsl is None:
+        hql = facts["hql"]
+        host = torch.zeros(hql.numel() + 1, dtype=torch.long, pin_memory=not capturing)
+        torch.cumsum(hql, 0, out=host[1:])
+        qsl = host.to(dev, non_blocking=not capturing)
+        if not capturing:
+            facts["qsl"][(dev, stream)] = qsl
+    return qsl
 
 
 def paged_attention_hip_launch(
@@ -159,61 +186,63 @@ def paged_attention_hip_launch(
     (the MFMA kernel stages new positions from the rows themselves and each workgroup
     writes its own tokens' rows), so the step has no separate append launch."""
     native.require_gpu(query, "paged_attention")
-    bs = k_pool.shape[1] if k_pool.dim() == 4 else 1
-    width = block_tables.shape[1] if block_tables.dim() == 2 else 0
-    facts: dict = {}
+    q_shape, p_shape, t_shape = query.shape, k_pool.shape, block_tables.shape
+    bs = p_shape[1] if len(p_shape) == 4 else 1
+    width = t_shape[1] if len(t_shape) == 2 else 0
+    facts: dict | None = None
 
     def values():
-        facts.update(_batch_facts(context_lens, query_lens, bs, width))
+        nonlocal facts
+        facts = _batch_facts(context_lens, query_lens, bs, width)
         return facts["total"], facts["q_gt_c"], facts["too_few_blocks"]
 
-    check_contract(
-        query.dim(), tuple(query.shape), k_pool.dim(), tuple(k_pool.shape), block_tables.shape,
-        context_lens.shape, query_lens.shape, values,
-    )
-    if not facts:
-        facts.update(_batch_facts(context_lens, query_lens, bs, width))
-    hql = facts["hql"]
-    if k_pool.shape != v_pool.shape:
-        raise ValueError(f"k_pool {tuple(k_pool.shape)} and v_pool {tuple(v_pool.shape)} differ")
-    dev = query.device
+    check_contract(len(q_shape), q_shape, len(p_shape), p_shape, t_shape, context_lens.shape, query_lens.shape, values)
+    if p_shape != v_pool.shape:
+        raise ValueError(f"k_pool {tuple(p_shape)} and v_pool {tuple(v_pool.shape)} differ")
+    dev, dtype = query.device, query.dtype
     for name, t in (("k_pool", k_pool), ("v_pool", v_pool)):
         if t.device != dev:
             raise ValueError(f"{name} is on {t.device}, query is on {dev}")
-        if t.dtype != query.dtype:
-            raise ValueError(f"{name} dtype {t.dtype} differs from query dtype {query.dtype}")
-    n_tok, n_heads, head_dim = query.shape
-    n_blocks, block_size, n_kv, pool_dim = k_pool.shape
+        if t.dtype != dtype:
+            raise ValueError(f"{name} dtype {t.dtype} differs from query dtype {dtype}")
+    n_tok, n_heads, head_dim = q_shape
+    n_blocks, block_size, n_kv, pool_dim = p_shape
     if pool_dim != head_dim:
         raise ValueError(f"query head_dim {head_dim} != pool head_dim {pool_dim}")
     if n_heads % n_kv:
         raise ValueError(f"{n_heads} query heads not divisible by {n_kv} kv heads")
-    dt = native.dtype_code(query.dtype)
+    dt = native.dtype_code(dtype)
 
-    out = torch.empty((n_tok, n_heads, head_dim), dtype=query.dtype, device=dev)
-    n_seqs = block_tables.shape[0]
+    out = torch.empty(q_shape, dtype=dtype, device=dev)
+    n_seqs = t_shape[0]
     if n_tok == 0 or n_seqs == 0:
         return out
 
     if query.stride(2) != 1:
         query = query.contiguous()
-    if k_pool.stride(3) != 1 or v_pool.stride() != k_pool.stride():
+    k_st = k_pool.stride()
+    if k_st[3] != 1 or v_pool.stride() != k_st:
         if append is not None:
             # A fused append writes the new rows into the pool in place; a contiguous
             # copy of the pool would take the rows and be thrown away.
             raise ValueError("a fused append needs k_pool and v_pool with unit head_dim stride and equal strides; "
-                             f"got {tuple(k_pool.stride())} and {tuple(v_pool.stride())}")
+                             f"got {tuple(k_st)} and {tuple(v_pool.stride())}")
         k_pool, v_pool = k_pool.contiguous(), v_pool.contiguous()
-    tables = block_tables.to(device=dev, dtype=torch.long)
-    if tables.stride(1) != 1:
+        k_st = k_pool.stride()
+    tables = _on_device(block_tables, dev)
+    t_st = tables.stride()
+    if t_st[1] != 1:
         tables = tables.contiguous()
-    ctx_dev = context_lens.to(device=dev, dtype=torch.long).contiguous()
+        t_st = tables.stride()
+    ctx_dev = _on_device(context_lens, dev).contiguous()
 
     L = native.lib()
     stream = native.stream_handle(dev)
-    common_pool = (k_pool.data_ptr(), v_pool.data_ptr(), k_pool.stride(0), k_pool.stride(1), k_pool.stride(2),
+    o_st, q_st = out.stride(), query.stride()
+    rows = (out.data_ptr(), o_st[0], o_st[1], query.data_ptr(), q_st[0], q_st[1])
+    common_pool = (k_pool.data_ptr(), v_pool.data_ptr(), k_st[0], k_st[1], k_st[2],
                    n_blocks, block_size, n_kv, head_dim,
-                   tables.data_ptr(), tables.stride(0), tables.shape[1])
+                   tables.data_ptr(), t_st[0], t_shape[1])
     if append is not None:
         k_new, v_new, slots = append
         if k_new.shape != (n_tok, n_kv, head_dim) or v_new.shape != k_new.shape:
@@ -221,14 +250,13 @@ def paged_attention_hip_launch(
                              f"got {tuple(k_new.shape)} and {tuple(v_new.shape)} for {n_tok} tokens")
         if k_new.stride(2) != 1 or v_new.stride() != k_new.stride():
             k_new, v_new = k_new.contiguous(), v_new.contiguous()
-        slots = slots.to(device=dev, dtype=torch.long)
+        slots = _on_device(slots, dev)
     if facts["all_decode"] and append is not None:
         max_ctx = facts["max_ctx"]
         ws_bytes = L.pkv_paged_attention_decode_workspace_bytes(n_seqs, n_heads, n_kv, head_dim, max_ctx)
         ws = _WORKSPACES.partials(dev, stream, ws_bytes)
         rc = L.pkv_paged_attention_decode_append(
-            out.data_ptr(), out.stride(0), out.stride(1),
-            query.data_ptr(), query.stride(0), query.stride(1),
+            *rows,
             *common_pool[:9],
             k_new.data_ptr(), v_new.data_ptr(), k_new.stride(0), k_new.stride(1), slots.data_ptr(),
             *common_pool[9:],
@@ -245,8 +273,7 @@ def paged_attention_hip_launch(
         ws_bytes = L.pkv_paged_attention_decode_workspace_bytes(n_seqs, n_heads, n_kv, head_dim, max_ctx)
         ws = _WORKSPACES.partials(dev, stream, ws_bytes)
         rc = L.pkv_paged_attention_decode(
-            out.data_ptr(), out.stride(0), out.stride(1),
-            query.data_ptr(), query.stride(0), query.stride(1),
+            *rows,
             *common_pool,
             ctx_dev.data_ptr(),
             n_seqs, n_heads, max_ctx,
@@ -259,13 +286,9 @@ def paged_attention_hip_launch(
 
     qsl = getattr(query_lens, _QSL_ATTR, None)
     if qsl is None:
-        qsl = facts["qsl"]
-        if qsl is None or qsl.device != dev:
-            qsl_host = torch.zeros(n_seqs + 1, dtype=torch.long)
-            torch.cumsum(hql, 0, out=qsl_host[1:])
-            qsl = facts["qsl"] = qsl_host.to(dev)
+        qsl = _query_start(facts, dev, stream)
     # Workspace for split contexts (0 bytes: a batch that is not split).
-    lens = (facts["hctx"].data_ptr(), hql.data_ptr())
+    lens = (facts["hctx"].data_ptr(), facts["hql"].data_ptr())
     ws_bytes = L.pkv_paged_attention_prefill_workspace_bytes(n_seqs, n_heads, n_kv, head_dim, n_tok, *lens)
     ws_ptr, ws_size = None, 0
     if ws_bytes:
@@ -274,8 +297,7 @@ def paged_attention_hip_launch(
     new = (None, None, 0, 0, None) if append is None else (
         k_new.data_ptr(), v_new.data_ptr(), k_new.stride(0), k_new.stride(1), slots.data_ptr())
     rc = L.pkv_paged_attention_prefill_split(
-        out.data_ptr(), out.stride(0), out.stride(1),
-        query.data_ptr(), query.stride(0), query.stride(1),
+        *rows,
         *common_pool[:9],
         *new,
         *common_pool[9:],

@@ -213,16 +213,20 @@ class PagedKVPool:
             raise ValueError(f"slots must be [{n_tok}], got {tuple(slots.shape)}")
         self.check_slots(slots, host_slots)
         # One stride pair describes both sources (the executor's K and V views share it).
-        if k.stride(2) != 1 or v.stride() != k.stride():
+        st = k.stride()
+        if st[2] != 1 or v.stride() != st:
             k, v = k.contiguous(), v.contiguous()
+            st = k.stride()
         kp, vp = self.k[layer], self.v[layer]
-        slots = slots.to(device=self.device, dtype=torch.long)
+        if slots.dtype is not torch.long or slots.device != kp.device:
+            slots = slots.to(device=kp.device, dtype=torch.long)
+        pool_st, pool_shape = kp.stride(), kp.shape
         rc = native.lib().pkv_kv_append(
-            kp.data_ptr(), vp.data_ptr(), kp.stride(0), kp.stride(1), kp.stride(2),
-            self.num_blocks, self.block_size, kp.shape[2], kp.shape[3],
-            k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1),
+            kp.data_ptr(), vp.data_ptr(), pool_st[0], pool_st[1], pool_st[2],
+            self.num_blocks, self.block_size, pool_shape[2], pool_shape[3],
+            k.data_ptr(), v.data_ptr(), st[0], st[1],
             slots.data_ptr(), n_tok, native.dtype_code(kp.dtype),
-            self._stream(),
+            native.stream_handle(kp.device),
         )
         native.check(rc, "pkv_kv_append")
 
