@@ -99,17 +99,16 @@ int pkv_graph_node_counts(void* graph, int64_t* counts, int64_t num_types);
 
 /* Workspace bytes pkv_paged_attention_decode needs for this batch shape: 256 KiB of
  * split-KV merge counters (one 32-bit word per (sequence, KV head)) followed by the
- * larger of two partial layouts: the partition kernels' (per sequence, query head and
- * 256-token partition: the running max, the softmax denominator and the unnormalised
- * output row, fp32; 768-token partitions use the first third of each row) and, for
+ * larger of two partial layouts: per sequence, query head and 256 tokens of context the
+ * running max, the softmax denominator and the unnormalised output row, fp32, and, for
  * batches the persistent MFMA kernel may take, its own (a prefix table plus one
  * partial per (workgroup, side, wave, head)). 0 when every context fits one 256-token
  * partition and the MFMA kernel does not apply (the output is then written directly).
  *
  * The counters must read zero when a call starts: zero-fill the workspace once before
  * its first use. Every call that runs to completion leaves them zero again (the
- * partition kernel's last partition of each (sequence, KV head) merges in place and
- * resets its counter; the MFMA kernel never touches them), and the partials need no
+ * last run of a split (sequence, KV head) to finish merges in place and resets its
+ * counter; the persistent kernel never touches them), and the partials need no
  * initialisation, so one workspace serves any later call on the same stream without
  * clearing. After a call that did not complete (a failed launch, an aborted stream, a
  * device reset) the counters may be dirty: zero-fill the workspace again (or use a
@@ -128,8 +127,10 @@ int64_t pkv_paged_attention_decode_workspace_bytes(int64_t num_seqs, int64_t num
  * max_context_len x head_dim x 4 bytes) reaches 512 MiB, with a multiple of 4 KV heads
  * and at most 1024 sequences, run the persistent MFMA kernel (equal runs of 16-key
  * blocks per workgroup, then a small merge kernel for the sequences the runs cut);
- * other 16-bit batches run the partition kernel (768- or 256-token partitions, merged
- * in place or by a small second kernel), fp32 the register kernel plus its merge
+ * other 16-bit batches of head_dims 32..128 (multiples of 16), groups up to 16 and
+ * power-of-two block sizes from 8 run the one-launch MFMA kernel (contexts cut into runs
+ * that fit the GPU, merged in place), groups above 16 the prefill kernel; fp32 runs the
+ * register kernel plus its merge
  * kernel. All launch on the same stream; calls that overlap in time (different
  * streams) need distinct workspaces. */
 int pkv_paged_attention_decode(
@@ -151,9 +152,9 @@ int pkv_paged_attention_decode(
  * pkv_paged_attention_decode computes over the updated pool (context_lens include the
  * new token). Replaces, per layer of a decode step, `_PagedCache.update`
  * (inference_server/core/paged_executor.py:116-125) followed by the decode attention
- * (inference_server/core/attention.py:130-153). With 16-bit pools on the tuned shapes
- * the streaming kernel writes each row itself, from the wave that reads that token
- * (no append launch); otherwise the append kernel runs first. Contract: slots[i] is
+ * (inference_server/core/attention.py:130-153). With 16-bit pools and 16-byte
+ * aligned rows the attention kernel writes each row itself, from the wave that reads that
+ * token (no append launch); otherwise the append kernel runs first. Contract: slots[i] is
  * the slot of position context_lens[i] - 1 of sequence i, and no other sequence's
  * table reaches it (the reference's copy-on-write guarantees both); slots outside the
  * pool are skipped. Same workspace as pkv_paged_attention_decode. */

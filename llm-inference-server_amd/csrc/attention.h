@@ -28,13 +28,13 @@ struct AttnParams {
     float* ws_o;                     // [num_seqs, num_heads, max_parts, head_dim]
     float* ws_ml;                    // [num_seqs, num_heads, max_parts, 2] = (max, denominator)
     int max_parts;
-    // Split-KV merge counters, one per (sequence, KV head), zero between calls (null:
-    // the partials are merged by a second kernel). With them the streaming kernel's
-    // last partition of a (sequence, KV head) to finish does the merge itself.
+    // Split-KV merge counters, one per (sequence, KV head), zero between calls (null: too
+    // many pairs). The one-launch decode kernel's last run of a (sequence, KV head) to
+    // finish merges them all.
     uint32_t* ws_cnt;
-    // Fused KV append (null = none). Decode (streaming kernel): row seq of app_k / app_v
+    // Fused KV append (null = none). Decode: row seq of app_k / app_v
     // ([num_seqs, num_kv_heads, head_dim], element strides app_st, app_sh) goes to flat
-    // pool slot app_slots[seq] before the attention reads it. Prefill (MFMA kernel): row
+    // pool slot app_slots[seq] and the attention sees it there. Prefill (MFMA kernel): row
     // t of [num_tokens, num_kv_heads, head_dim] goes to app_slots[t] and the kernel reads
     // the new positions from these rows.
     const void* app_k;
@@ -55,9 +55,10 @@ struct AttnParams {
     int* ws_pfx;
 };
 
-// True when launch_decode_attention runs the streaming kernel for these parameters
-// (the only decode kernel that performs a fused append).
-bool decode_streams(const AttnParams& p, int dtype);
+// One-launch MFMA decode (attn_decode_split.hip): whether it takes these parameters (with
+// p.app_* set: including the fused append, whose source rows must be 16-byte aligned).
+bool decode_split_applies(const AttnParams& p, int dtype);
+int launch_decode_split(const AttnParams& p, int dtype, hipStream_t stream);
 // True when launch_prefill_attention runs the MFMA kernel for these parameters (with
 // p.app_* set: including the fused append, whose source rows must be 16-byte aligned).
 bool prefill_tuned(const AttnParams& p, int dtype);
@@ -110,7 +111,7 @@ int launch_f32_attention(const AttnParams& p, hipStream_t stream);
 // fp32 MFMA kernel. Returns PKV_EUNSUPPORTED (without setting an error) for anything else.
 int launch_prefill_f32_mfma(const AttnParams& p, hipStream_t stream);
 // Returns PKV_EUNSUPPORTED (without setting an error) when no tuned kernel matches.
-int launch_decode_attention(const AttnParams& p, int dtype, hipStream_t stream);
+int launch_decode_attention(const AttnParams& p, hipStream_t stream);
 int launch_prefill_attention(const AttnParams& p, int dtype, hipStream_t stream);
 
 // ---- prefill dispatch order (the MFMA prefill kernels, 256-thread workgroups).

@@ -1,0 +1,742 @@
+// Paged decode attention on MFMA (gfx950) in one launch, fp16/bf16, head_dim a multiple of
+// 16 from 32 to 128, GQA groups up to 16, block sizes that are powers of two from 8 up.
+// Takes every such decode batch below the size from which the persistent kernel
+// (attn_decode_mfma.hip) is the better one.
+//
+// Bound: HBM for batches of tens of MB, latency below that. Every K/V byte is read once
+// (all heads of a group share the read); what the launch pays on top is its start (lengths,
+// block ids, the first K/V rows: three dependent memory round trips), the tail of unequal
+// contexts, and the merge of split contexts. Hence:
+//
+//  * Work unit: one workgroup = (sequence, KV head, run of 16-key units) x NW waves; wave w
+//    takes units w, w + NW, ... of the run. A batch of few (sequence, KV head) pairs gets
+//    workgroups of more waves (the launch picks NW), so short contexts need no split.
+//  * Runs are cut on the device: every wave sums the batch's units, takes the shortest run
+//    length (no less than 4 units a wave) with which all runs fit the GPU at once, and finds
+//    its own (sequence, split) by a wave scan, no barrier. The grid is bounded by the GPU, not
+//    by the longest context a captured graph must serve, and holds next to no empty
+//    workgroups; a sequence's runs are of even lengths.
+//  * Streaming: per wave a two-slot ring of units in LDS (K and V, 16 rows of one KV head),
+//    filled by nontemporal LDS DMA; a unit's K and V^T fragments are read into registers
+//    first and the slot refilled with the unit after next at once. Waits are explicit vmcnt
+//    counts; DMAs and ring reads are inline asm, unseen by the compiler's wait counting.
+//  * Contraction as in the persistent kernel: S^T = K Q^T on 16x16x32, P^T straight from the
+//    accumulator into O^T += V^T P^T on 16x16x16, V^T by the transposing LDS read. 12 MFMAs
+//    and ~80 VALU instructions per unit at head_dim 128, where v_dot2 arithmetic took ~900.
+//  * Merge: the waves' partials meet in LDS; split contexts leave fp32 partials that the
+//    last workgroup of each (sequence, KV head) to finish merges in run order (agent-scope
+//    stores, one counter, no workgroup ever waits for another).
+//  * Fused append: the new token's row is staged from the caller's rows by the DMA of the
+//    context's last unit, and goes to its pool slot from registers, so nothing waits for the
+//    store.
+//
+// Numerics follow the reference gather path (core/attention.py:130-153) as the persistent
+// kernel does: scores rounded to the pool dtype before and after the scale, softmax in fp32,
+// probabilities exp2(s - m) rounded to the pool dtype before P·V with the running max raised
+// lazily (past 2^8 only), fp32 accumulation, one rounding of the output. Keys at or beyond
+// context_lens are never loaded.
+#include "attention.h"
+
+namespace pkv {
+namespace {
+
+constexpr int kUnit = 16;                     // keys per unit
+constexpr float kLazyMax = 8.f;
+constexpr int kMaxScanSeqs = 1024;            // sequences a wave scans (16 per lane)
+constexpr int kScanPer = kMaxScanSeqs / 64;
+constexpr int kCus = 256;
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+// MFMA lane layouts as pinned for the persistent kernel (attn_decode_mfma.hip).
+template <typename T>
+struct SMfma;
+template <>
+struct SMfma<bf16_t> {
+    __device__ __forceinline__ static f32x4 qk(u32x4 a, u32x4 b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b),
+                                                       c, 0, 0, 0);
+    }
+    __device__ __forceinline__ static f32x4 pv(uint2 a, uint2 b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(bf16x4, a), __builtin_bit_cast(bf16x4, b),
+                                                         c, 0, 0, 0);
+    }
+    __device__ __forceinline__ static uint32_t pack(float lo, float hi) {
+        bf16x2_t v = {(__bf16)lo, (__bf16)hi};
+        return __builtin_bit_cast(uint32_t, v);
+    }
+    __device__ __forceinline__ static float round(float x) { return (float)(__bf16)x; }
+};
+template <>
+struct SMfma<_Float16> {
+    __device__ __forceinline__ static f32x4 qk(u32x4 a, u32x4 b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c,
+                                                      0, 0, 0);
+    }
+    __device__ __forceinline__ static f32x4 pv(uint2 a, uint2 b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, a), __builtin_bit_cast(f16x4, b), c,
+                                                     0, 0, 0);
+    }
+    __device__ __forceinline__ static uint32_t pack(float lo, float hi) {
+        half2_t v = {(_Float16)lo, (_Float16)hi};
+        return __builtin_bit_cast(uint32_t, v);
+    }
+    __device__ __forceinline__ static float round(float x) { return (float)(_Float16)x; }
+};
+
+// Physical 16-byte slot of logical chunk c of ring row r is c ^ unit_swizzle(r): the 16 rows
+// of a K read fall in different banks (at head_dim 48, 80 and 112 in pairs).
+template <int D>
+__device__ __forceinline__ int unit_swizzle(int r) {
+    if constexpr (D == 128) return ((r & 3) << 2) | ((r >> 2) & 3);
+    else if constexpr (D == 64) return (((r >> 1) & 1) << 2) | (((r >> 2) & 1) << 1) | ((r >> 3) & 1);
+    else if constexpr (D % 32 == 0) return (r >> 2) & 3;
+    else return (r >> 3) & 1;
+}
+
+__device__ __forceinline__ uint32_t lds_addr(const void* ptr) {
+    return (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)ptr);
+}
+
+// 16 bytes per lane HBM -> LDS address lds + 16 lane, nontemporal (read once: a stream of
+// this pattern runs 12% faster so). M0 belongs to these helpers alone in this kernel.
+__device__ __forceinline__ void dma16_nt(const char* sbase, uint32_t voff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+                 :
+                 : "s"(lds), "v"(voff), "s"(sbase)
+                 : "memory");
+}
+__device__ __forceinline__ void dma16_nt(const char* addr, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt"
+                 :
+                 : "s"(lds), "v"(addr)
+                 : "memory");
+}
+
+// A unit's MFMA operands from its ring slot: KS b128 reads of K and VT transposing reads of
+// V, all issued, then waited for. Each read and the wait are asm statements of their own,
+// kept in order by "memory"; the results pass through the waiting statement, so no use of
+// them can move above it.
+template <int KS, int VT>
+__device__ __forceinline__ void ring_read(uint32_t kb, const uint32_t (&ka)[KS], uint32_t vb, const uint32_t (&va)[VT],
+                                          u32x4 (&kf)[KS], uint2 (&vf)[VT]);
+
+#define PKV_RD_K(i, a) "ds_read_b128 %" #i ", %" #a "\n\t"
+#define PKV_RD_V(i, a) "ds_read_b64_tr_b16 %" #i ", %" #a "\n\t"
+#define PKV_OUT(x) "=&v"(x)
+#define PKV_IN(x) "v"(x)
+
+template <>
+__device__ __forceinline__ void ring_read<1, 2>(uint32_t kb, const uint32_t (&ka)[1], uint32_t vb,
+                                                const uint32_t (&va)[2], u32x4 (&kf)[1], uint2 (&vf)[2]) {
+    asm volatile(PKV_RD_K(0, 3) PKV_RD_V(1, 4) PKV_RD_V(2, 5) "s_waitcnt lgkmcnt(0)"
+                 : PKV_OUT(kf[0]), PKV_OUT(vf[0]), PKV_OUT(vf[1])
+                 : PKV_IN(kb + ka[0]), PKV_IN(vb + va[0]), PKV_IN(vb + va[1])
+                 : "memory");
+}
+template <>
+__device__ __forceinline__ void ring_read<2, 3>(uint32_t kb, const uint32_t (&ka)[2], uint32_t vb,
+                                                const uint32_t (&va)[3], u32x4 (&kf)[2], uint2 (&vf)[3]) {
+    asm volatile(PKV_RD_K(0, 5) PKV_RD_K(1, 6) PKV_RD_V(2, 7) PKV_RD_V(3, 8) PKV_RD_V(4, 9) "s_waitcnt lgkmcnt(0)"
+                 : PKV_OUT(kf[0]), PKV_OUT(kf[1]), PKV_OUT(vf[0]), PKV_OUT(vf[1]), PKV_OUT(vf[2])
+                 : PKV_IN(kb + ka[0]), PKV_IN(kb + ka[1]), PKV_IN(vb + va[0]), PKV_IN(vb + va[1]), PKV_IN(vb + va[2])
+                 : "memory");
+}
+template <>
+__device__ __forceinline__ void ring_read<2, 4>(uint32_t kb, const uint32_t (&ka)[2], uint32_t vb,
+                                                const uint32_t (&va)[4], u32x4 (&kf)[2], uint2 (&vf)[4]) {
+    asm volatile(PKV_RD_K(0, 6) PKV_RD_K(1, 7) PKV_RD_V(2, 8) PKV_RD_V(3, 9) PKV_RD_V(4, 10) PKV_RD_V(5, 11)
+                     "s_waitcnt lgkmcnt(0)"
+                 : PKV_OUT(kf[0]), PKV_OUT(kf[1]), PKV_OUT(vf[0]), PKV_OUT(vf[1]), PKV_OUT(vf[2]), PKV_OUT(vf[3])
+                 : PKV_IN(kb + ka[0]), PKV_IN(kb + ka[1]), PKV_IN(vb + va[0]), PKV_IN(vb + va[1]), PKV_IN(vb + va[2]),
+                   PKV_IN(vb + va[3])
+                 : "memory");
+}
+template <>
+__device__ __forceinline__ void ring_read<3, 5>(uint32_t kb, const uint32_t (&ka)[3], uint32_t vb,
+                                                const uint32_t (&va)[5], u32x4 (&kf)[3], uint2 (&vf)[5]) {
+    asm volatile(PKV_RD_K(0, 8) PKV_RD_K(1, 9) PKV_RD_K(2, 10) PKV_RD_V(3, 11) PKV_RD_V(4, 12) PKV_RD_V(5, 13)
+                     PKV_RD_V(6, 14) PKV_RD_V(7, 15) "s_waitcnt lgkmcnt(0)"
+                 : PKV_OUT(kf[0]), PKV_OUT(kf[1]), PKV_OUT(kf[2]), PKV_OUT(vf[0]), PKV_OUT(vf[1]), PKV_OUT(vf[2]),
+                   PKV_OUT(vf[3]), PKV_OUT(vf[4])
+                 : PKV_IN(kb + ka[0]), PKV_IN(kb + ka[1]), PKV_IN(kb + ka[2]), PKV_IN(vb + va[0]), PKV_IN(vb + va[1]),
+                   PKV_IN(vb + va[2]), PKV_IN(vb + va[3]), PKV_IN(vb + va[4])
+                 : "memory");
+}
+template <>
+__device__ __forceinline__ void ring_read<3, 6>(uint32_t kb, const uint32_t (&ka)[3], uint32_t vb,
+                                                const uint32_t (&va)[6], u32x4 (&kf)[3], uint2 (&vf)[6]) {
+    asm volatile(PKV_RD_K(0, 9) PKV_RD_K(1, 10) PKV_RD_K(2, 11) PKV_RD_V(3, 12) PKV_RD_V(4, 13) PKV_RD_V(5, 14)
+                     PKV_RD_V(6, 15) PKV_RD_V(7, 16) PKV_RD_V(8, 17) "s_waitcnt lgkmcnt(0)"
+                 : PKV_OUT(kf[0]), PKV_OUT(kf[1]), PKV_OUT(kf[2]), PKV_OUT(vf[0]), PKV_OUT(vf[1]), PKV_OUT(vf[2]),
+                   PKV_OUT(vf[3]), PKV_OUT(vf[4]), PKV_OUT(vf[5])
+                 : PKV_IN(kb + ka[0]), PKV_IN(kb + ka[1]), PKV_IN(kb + ka[2]), PKV_IN(vb + va[0]), PKV_IN(vb + va[1]),
+                   PKV_IN(vb + va[2]), PKV_IN(vb + va[3]), PKV_IN(vb + va[4]), PKV_IN(vb + va[5])
+                 : "memory");
+}
+template <>
+__device__ __forceinline__ void ring_read<4, 7>(uint32_t kb, const uint32_t (&ka)[4], uint32_t vb,
+                                                const uint32_t (&va)[7], u32x4 (&kf)[4], uint2 (&vf)[7]) {
+    asm volatile(PKV_RD_K(0, 11) PKV_RD_K(1, 12) PKV_RD_K(2, 13) PKV_RD_K(3, 14) PKV_RD_V(4, 15) PKV_RD_V(5, 16)
+                     PKV_RD_V(6, 17) PKV_RD_V(7, 18) PKV_RD_V(8, 19) PKV_RD_V(9, 20) PKV_RD_V(10, 21)
+                         "s_waitcnt lgkmcnt(0)"
+                 : PKV_OUT(kf[0]), PKV_OUT(kf[1]), PKV_OUT(kf[2]), PKV_OUT(kf[3]), PKV_OUT(vf[0]), PKV_OUT(vf[1]),
+                   PKV_OUT(vf[2]), PKV_OUT(vf[3]), PKV_OUT(vf[4]), PKV_OUT(vf[5]), PKV_OUT(vf[6])
+                 : PKV_IN(kb + ka[0]), PKV_IN(kb + ka[1]), PKV_IN(kb + ka[2]), PKV_IN(kb + ka[3]), PKV_IN(vb + va[0]),
+                   PKV_IN(vb + va[1]), PKV_IN(vb + va[2]), PKV_IN(vb + va[3]), PKV_IN(vb + va[4]), PKV_IN(vb + va[5]),
+                   PKV_IN(vb + va[6])
+                 : "memory");
+}
+template <>
+__device__ __forceinline__ void ring_read<4, 8>(uint32_t kb, const uint32_t (&ka)[4], uint32_t vb,
+                                                const uint32_t (&va)[8], u32x4 (&kf)[4], uint2 (&vf)[8]) {
+    asm volatile(PKV_RD_K(0, 12) PKV_RD_K(1, 13) PKV_RD_K(2, 14) PKV_RD_K(3, 15) PKV_RD_V(4, 16) PKV_RD_V(5, 17)
+                     PKV_RD_V(6, 18) PKV_RD_V(7, 19) PKV_RD_V(8, 20) PKV_RD_V(9, 21) PKV_RD_V(10, 22)
+                         PKV_RD_V(11, 23) "s_waitcnt lgkmcnt(0)"
+                 : PKV_OUT(kf[0]), PKV_OUT(kf[1]), PKV_OUT(kf[2]), PKV_OUT(kf[3]), PKV_OUT(vf[0]), PKV_OUT(vf[1]),
+                   PKV_OUT(vf[2]), PKV_OUT(vf[3]), PKV_OUT(vf[4]), PKV_OUT(vf[5]), PKV_OUT(vf[6]), PKV_OUT(vf[7])
+                 : PKV_IN(kb + ka[0]), PKV_IN(kb + ka[1]), PKV_IN(kb + ka[2]), PKV_IN(kb + ka[3]), PKV_IN(vb + va[0]),
+                   PKV_IN(vb + va[1]), PKV_IN(vb + va[2]), PKV_IN(vb + va[3]), PKV_IN(vb + va[4]), PKV_IN(vb + va[5]),
+                   PKV_IN(vb + va[6]), PKV_IN(vb + va[7])
+                 : "memory");
+}
+#undef PKV_RD_K
+#undef PKV_RD_V
+#undef PKV_OUT
+#undef PKV_IN
+
+// ------------------------------------------------------------------ wave scans (int)
+template <int CTRL>
+__device__ __forceinline__ int dpp_shr(int x) {   // 0 where the source is outside the row
+    return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true);
+}
+// Inclusive sum over lanes 0 .. l, in every lane l.
+__device__ __forceinline__ int wave_scan(int x, int lane) {
+    x += dpp_shr<0x111>(x);   // row_shr:1, 2, 4, 8 within rows of 16
+    x += dpp_shr<0x112>(x);
+    x += dpp_shr<0x114>(x);
+    x += dpp_shr<0x118>(x);
+    const int r0 = __builtin_amdgcn_readlane(x, 15), r1 = __builtin_amdgcn_readlane(x, 31),
+              r2 = __builtin_amdgcn_readlane(x, 47);
+    return x + (lane >= 16 ? r0 : 0) + (lane >= 32 ? r1 : 0) + (lane >= 48 ? r2 : 0);
+}
+__device__ __forceinline__ int wave_total(int x, int lane) {
+    return __builtin_amdgcn_readlane(wave_scan(x, lane), 63);
+}
+
+// Context length as every decode kernel clamps it: never past the table row or the
+// partials the workspace was sized for (neither binds for valid input).
+__device__ __forceinline__ int decode_ctx(const AttnParams& p, int seq) {
+    const int64_t cap = p.table_width * (int64_t)p.block_size;
+    const int64_t parts = (int64_t)p.max_parts * kDecodePart;
+    int64_t c = p.ctx_lens[seq];
+    c = c < cap ? c : cap;
+    c = c < parts ? c : parts;
+    return c > 0 ? (int)c : 0;
+}
+
+// The `at`-th run of one KV head's batch, numbered sequence by sequence; seq < 0: none.
+struct Pick {
+    int seq, ctx, split, n_splits;
+};
+
+// Every wave by itself, lane l holding the contexts of sequences PER l .. PER l + PER - 1.
+template <int PER>
+__device__ __forceinline__ Pick pick_run(const AttnParams& p, int lane, int at, int min_run, int slots) {
+    int units_of[PER], cl[PER], units = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int s = lane * PER + i;
+        cl[i] = s < p.num_seqs ? decode_ctx(p, s) : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        units_of[i] = (cl[i] + kUnit - 1) / kUnit;
+        units += units_of[i];
+    }
+    // The shortest run with which one KV head's runs fit its share of the GPU's slots: from
+    // the even share of those left when every sequence's last run is half empty, up in
+    // growing steps (mostly none or one).
+    const int total = wave_total(units, lane);
+    const int even = slots - p.num_seqs / 2;  // slots >= num_seqs
+    int run = (total + even - 1) / even;
+    run = run > min_run ? run : min_run;
+    int n_of[PER], mine = 0;
+    for (int step = (run + 15) >> 4;; run += step, step += (step + 1) >> 1) {
+        mine = 0;
+        const float inv = 1.f / (float)run;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            // ceil(units / run): exact after one correction either way.
+            const int u = units_of[i];
+            int q = (int)((float)u * inv);
+            q -= q * run > u ? 1 : 0;
+            q += (q + 1) * run <= u ? 1 : 0;
+            n_of[i] = q + (q * run < u ? 1 : 0);
+            mine += n_of[i];
+        }
+        if (run >= total || wave_total(mine, lane) <= slots) break;
+    }
+    const int incl = wave_scan(mine, lane);
+    const uint64_t found = __builtin_amdgcn_ballot_w64(at < incl);
+    if (!found) return Pick{-1, 0, 0, 0};
+    const int src = __builtin_ctzll(found);   // the first lane whose runs reach past `at`
+    int left = at - (__builtin_amdgcn_readlane(incl, src) - __builtin_amdgcn_readlane(mine, src));
+    if constexpr (PER == 1) {
+        return Pick{src, __builtin_amdgcn_readlane(cl[0], src), left, __builtin_amdgcn_readlane(n_of[0], src)};
+    } else {
+        Pick r{-1, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if (r.seq < 0) {
+                const int n = __builtin_amdgcn_readlane(n_of[i], src);
+                if (left < n) r = Pick{src * PER + i, __builtin_amdgcn_readlane(cl[i], src), left, n};
+                else left -= n;
+            }
+        return r;
+    }
+}
+
+// LDS bytes of a workgroup (the ring; the merge's partials reuse it) and how many a CU holds.
+constexpr int ring_bytes(int D, int NW) { return NW * 2 * 2 * kUnit * D * 2; }
+constexpr int wgs_per_cu(int D, int NW) {
+    const int lds = (160 * 1024) / (ring_bytes(D, NW) + NW * 128 + 16), waves = 16 / NW;
+    const int n = lds < waves ? lds : waves;
+    return n < 1 ? 0 : n;
+}
+
+template <typename T, int D, int NW>
+__global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnParams p, int min_run, int slots) {
+    constexpr int ROWB = D * 2;               // bytes per (token, head) row
+    constexpr int CPR = ROWB / 16;            // 16-byte chunks per row
+    constexpr int IPB = (kUnit * CPR + 63) / 64;   // DMA instructions per unit, K or V
+    constexpr bool kWhole = kUnit * CPR % 64 == 0;
+    constexpr bool kHalf = 64 % CPR == 0 && 64 / CPR <= 8;   // one 8-row half per instruction
+    constexpr int KS = (D + 31) / 32;         // S^T MFMAs per unit
+    constexpr int VT = D / 16;                // P·V MFMAs per unit
+    constexpr int NT = NW * 64;
+    constexpr int UB = kUnit * ROWB;          // bytes of a unit, K or V
+
+    __shared__ __attribute__((aligned(1024))) char s_ring[NW][2][2][UB];   // [wave][slot][K, V]
+    __shared__ float s_ml[NW][16][2];
+    __shared__ uint32_t s_arrived;
+
+    const int tid = (int)threadIdx.x;
+    const int lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int KV = p.num_kv_heads, G = p.group;
+    const int kvh = (int)(blockIdx.x % (uint32_t)KV);
+    const int at = (int)(blockIdx.x / (uint32_t)KV);
+
+    // ---- this workgroup's (sequence, run)
+    int seq, ctx, split = 0, n_splits = 1;
+    if (slots == 0) {                         // one workgroup per (sequence, KV head)
+        seq = at;
+        ctx = __builtin_amdgcn_readfirstlane(decode_ctx(p, seq));
+        if (ctx == 0) return;
+    } else {
+        const Pick pick = p.num_seqs <= 64 ? pick_run<1>(p, lane, at, min_run, slots)
+                                           : pick_run<kScanPer>(p, lane, at, min_run, slots);
+        if (pick.seq < 0) return;
+        seq = pick.seq;
+        ctx = pick.ctx;
+        split = pick.split;
+        n_splits = pick.n_splits;
+    }
+    const int n_units = (ctx + kUnit - 1) / kUnit;
+    const int run = (n_units + n_splits - 1) / n_splits;   // even runs
+    n_splits = (n_units + run - 1) / run;
+    if (split >= n_splits) return;            // an even cut took one run fewer
+    const int u_end = split * run + run < n_units ? split * run + run : n_units;
+    const int u_first = split * run + wave;   // this wave's units: u_first, + NW, ...
+    const int nu = u_first < u_end ? (u_end - u_first + NW - 1) / NW : 0;
+
+    const int lg = lane >> 4;                 // MFMA lane group
+    const int ln = lane & 15;                 // MFMA row / column index
+
+    // ---- Q^T B operand: lane (lg, ln) takes head ln, dims 32 j + 8 lg .. +8 (zero for the
+    // padding heads and dims). Issued before the block ids, whose wait covers it.
+    u32x4 qf[KS];
+#pragma unroll
+    for (int j = 0; j < KS; ++j) {
+        qf[j] = u32x4{0u, 0u, 0u, 0u};
+        if (ln < G && 4 * j + lg < CPR) {
+            const Vec16 v = load16(reinterpret_cast<const char*>(p.q) +
+                                   ((int64_t)seq * p.q_st + (int64_t)(kvh * G + ln) * p.q_sh) * 2 + (4 * j + lg) * 16);
+            qf[j] = u32x4{v.w[0], v.w[1], v.w[2], v.w[3]};
+        }
+    }
+
+    // ---- fused append: the new token is the context's last key. The wave whose units end
+    // with it holds the row (lanes 0 .. CPR-1 K, CPR .. 2 CPR-1 V) and stores it at the end.
+    const int new_row = p.app_slots && nu > 0 && u_first + (nu - 1) * NW == n_units - 1 ? (ctx - 1) % kUnit : -1;
+    const char* knew = reinterpret_cast<const char*>(p.app_k) + ((int64_t)seq * p.app_st + (int64_t)kvh * p.app_sh) * 2;
+    const char* vnew = reinterpret_cast<const char*>(p.app_v) + ((int64_t)seq * p.app_st + (int64_t)kvh * p.app_sh) * 2;
+    Vec16 new_piece = Vec16{{0u, 0u, 0u, 0u}};
+    int64_t new_slot = -1;
+    if (new_row >= 0 && lane < 2 * CPR) {
+        new_slot = p.app_slots[seq];
+        new_piece = load16((lane < CPR ? knew : vnew) + (lane % CPR) * 16);
+    }
+
+    const int64_t slot_bytes = p.ss * 2;
+    const int64_t block_bytes = p.sb * 2;
+    const char* kbase = reinterpret_cast<const char*>(p.k) + (int64_t)kvh * p.sh * 2;
+    const char* vbase = reinterpret_cast<const char*>(p.v) + (int64_t)kvh * p.sh * 2;
+    const int64_t* table = p.tables + (int64_t)seq * p.table_stride;
+
+    // ---- DMA of a unit: row and swizzled source chunk of this lane's instruction j.
+    auto dma_row = [&](int j) { return (64 * j + lane) / CPR; };
+    auto dma_chunk = [&](int j) { return (64 * j + lane) % CPR ^ unit_swizzle<D>((64 * j + lane) / CPR); };
+    uint32_t lane_off[IPB];                   // inside an 8-row half
+#pragma unroll
+    for (int j = 0; j < IPB; ++j)
+        lane_off[j] = (uint32_t)((dma_row(j) & 7) * slot_bytes) + (uint32_t)(dma_chunk(j) * 16);
+    // offs: this lane's 8-key half's byte offset in the pool (half lane & 1 of the chunk's
+    // unit lane / 2).
+    auto dma_unit = [&](int k, int64_t offs, int slot) {
+        const int64_t half0 = readlane64(offs, 2 * (k & 31)), half1 = readlane64(offs, 2 * (k & 31) + 1);
+        const int unit = u_first + k * NW;
+        const int rows = ctx - unit * kUnit < kUnit ? ctx - unit * kUnit : kUnit;   // keys of the unit
+        const uint32_t lk = lds_addr(s_ring[wave][slot][0]), lv = lds_addr(s_ring[wave][slot][1]);
+        const int app_row = unit == n_units - 1 ? new_row : -1;
+        if (rows == kUnit && app_row < 0) {
+#pragma unroll
+            for (int j = 0; j < IPB; ++j) {
+                if constexpr (kHalf) {
+                    const int64_t half = 64 * j / CPR < 8 ? half0 : half1;
+                    dma16_nt(kbase + half, lane_off[j], lk + j * 1024);
+                    dma16_nt(vbase + half, lane_off[j], lv + j * 1024);
+                } else if (kWhole || 64 * j + lane < kUnit * CPR) {
+                    const int64_t off = (dma_row(j) < 8 ? half0 : half1) + lane_off[j];
+                    dma16_nt(kbase + off, lk + j * 1024);
+                    dma16_nt(vbase + off, lv + j * 1024);
+                }
+            }
+            return;
+        }
+        // The context's last unit: rows past the context re-read its last key, the new
+        // token's row comes from the caller (its pool slot is not read in this launch).
+#pragma unroll
+        for (int j = 0; j < IPB; ++j) {
+            const int r = dma_row(j) < rows ? dma_row(j) : rows - 1;
+            const int64_t off = (r < 8 ? half0 : half1) + (r & 7) * slot_bytes + dma_chunk(j) * 16;
+            const char* ks = r == app_row ? knew + dma_chunk(j) * 16 : kbase + off;
+            const char* vs = r == app_row ? vnew + dma_chunk(j) * 16 : vbase + off;
+            if (kWhole || 64 * j + lane < kUnit * CPR) {
+                dma16_nt(ks, lk + j * 1024);
+                dma16_nt(vs, lv + j * 1024);
+            }
+        }
+    };
+
+    // ---- per-lane operand addresses inside a unit: K row ln, logical chunk 4 j + lg (a
+    // chunk past head_dim re-reads another, zeroed below); V^T rows 4 lg + ln / 4, columns
+    // 16 t + 4 (ln % 4).
+    uint32_t k_addr[KS], v_addr[VT];
+#pragma unroll
+    for (int j = 0; j < KS; ++j) {
+        const int c = 4 * j + lg < CPR ? 4 * j + lg : 4 * j + (lg & 1);
+        k_addr[j] = (uint32_t)(ln * ROWB + ((c ^ unit_swizzle<D>(ln)) << 4));
+    }
+    const int v_row = 4 * lg + (ln >> 2);
+#pragma unroll
+    for (int t = 0; t < VT; ++t)
+        v_addr[t] = (uint32_t)(v_row * ROWB + (((2 * t + ((ln & 3) >> 1)) ^ unit_swizzle<D>(v_row)) << 4) + 8 * (ln & 1));
+
+    f32x4 o[VT];
+#pragma unroll
+    for (int t = 0; t < VT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run = kNegInf, l_part = 0.f;
+    const float scale = p.scale;
+
+    constexpr int kUnitDmas = 2 * IPB;
+    for (int k0 = 0; k0 < nu; k0 += 32) {     // 32 units' block ids at a time
+        int64_t offs;
+        {
+            int key = (u_first + (k0 + (lane >> 1)) * NW) * kUnit + 8 * (lane & 1);
+            const int last = (ctx - 1) & ~7;
+            key = key < last ? key : last;    // halves past the context: the last one's block
+            const int64_t id = table[key >> p.block_shift];
+            offs = ((uint64_t)id < (uint64_t)p.num_blocks ? id : 0) * block_bytes +
+                   (key & (p.block_size - 1)) * slot_bytes;
+        }
+        const int k1 = k0 + 32 < nu ? k0 + 32 : nu;
+        dma_unit(k0, offs, 0);
+        if (k0 + 1 < k1) dma_unit(k0 + 1, offs, 1);
+        for (int k = k0; k < k1; ++k) {
+            const int slot = k & 1;
+            if (k + 1 < k1) __builtin_amdgcn_s_waitcnt(kWaitVm<kUnitDmas>);
+            else __builtin_amdgcn_s_waitcnt(kWaitVm<0>);
+            u32x4 kf[KS];
+            uint2 vf[VT];
+            ring_read<KS, VT>(lds_addr(s_ring[wave][slot][0]), k_addr, lds_addr(s_ring[wave][slot][1]), v_addr, kf, vf);
+            if (k + 2 < k1) dma_unit(k + 2, offs, slot);
+            if constexpr (D % 32 != 0)
+                if (lg >= 2) kf[KS - 1] = u32x4{0u, 0u, 0u, 0u};
+
+            // S^T for the 16 keys: lane (lg, ln) holds keys 4 lg + r of head ln.
+            f32x4 st = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < KS; ++j) st = SMfma<T>::qk(kf[j], qf[j], st);
+            const int valid = ctx - (u_first + k * NW) * kUnit;
+            float bmax = kNegInf;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float x = SMfma<T>::round(SMfma<T>::round(st[r]) * scale) * kLog2e;
+                st[r] = 4 * lg + r < valid ? x : kNegInf;
+                bmax = fmaxf(bmax, st[r]);
+            }
+            {
+                SwapPair sp = swap16(bmax);
+                bmax = fmaxf(sp.a, sp.b);
+                sp = swap32(bmax);
+                bmax = fmaxf(sp.a, sp.b);
+            }
+            const bool raise = bmax > m_run + kLazyMax;
+            if (__builtin_amdgcn_ballot_w64(raise)) {
+                const float m_new = raise ? bmax : m_run;
+                const float alpha = !raise ? 1.f : (m_run == kNegInf ? 0.f : fast_exp2(m_run - m_new));
+#pragma unroll
+                for (int t = 0; t < VT; ++t) o[t] *= alpha;
+                l_part *= alpha;
+                m_run = m_new;
+            }
+            const float m_off = m_run == kNegInf ? 0.f : m_run;
+            float pr[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                pr[r] = fast_exp2(st[r] - m_off);
+                l_part += pr[r];
+            }
+            const uint2 pb = make_uint2(SMfma<T>::pack(pr[0], pr[1]), SMfma<T>::pack(pr[2], pr[3]));
+#pragma unroll
+            for (int t = 0; t < VT; ++t) o[t] = SMfma<T>::pv(vf[t], pb, o[t]);
+        }
+    }
+    if (new_row >= 0 && (uint64_t)new_slot < (uint64_t)(p.num_blocks << p.block_shift)) {
+        const int64_t dst = (new_slot >> p.block_shift) * block_bytes +
+                            (new_slot & (p.block_size - 1)) * slot_bytes + (lane % CPR) * 16;
+        store16(const_cast<char*>(lane < CPR ? kbase : vbase) + dst, new_piece);
+    }
+
+    // ---- the waves' partials over their own ring slices (no longer in use), then the merge.
+    {
+        SwapPair sp = swap16(l_part);
+        l_part = sp.a + sp.b;
+        sp = swap32(l_part);
+        l_part = sp.a + sp.b;
+    }
+    float* w_acc = reinterpret_cast<float*>(s_ring[wave]);   // [G][D]
+    if (ln < G) {
+#pragma unroll
+        for (int t = 0; t < VT; ++t)
+            *reinterpret_cast<float4*>(w_acc + ln * D + 16 * t + 4 * lg) = make_float4(o[t][0], o[t][1], o[t][2], o[t][3]);
+        if (lg == 0) {
+            s_ml[wave][ln][0] = m_run;
+            s_ml[wave][ln][1] = l_part;
+        }
+    }
+    lds_barrier();
+
+    const int head0 = kvh * G;
+    // Four consecutive elements per thread.
+    auto store_out = [&](int g, int d, float4 v) {
+        T* orow = reinterpret_cast<T*>(p.out) + (int64_t)seq * p.out_st + (int64_t)(head0 + g) * p.out_sh + d;
+        const uint32_t w0 = SMfma<T>::pack(v.x, v.y), w1 = SMfma<T>::pack(v.z, v.w);
+        if ((((uint64_t)(uintptr_t)p.out | (uint64_t)(p.out_st * 2) | (uint64_t)(p.out_sh * 2)) & 7) == 0) {
+            *reinterpret_cast<uint2*>(orow) = make_uint2(w0, w1);
+        } else {
+            uint16_t* o16 = reinterpret_cast<uint16_t*>(orow);
+            o16[0] = (uint16_t)w0;
+            o16[1] = (uint16_t)(w0 >> 16);
+            o16[2] = (uint16_t)w1;
+            o16[3] = (uint16_t)(w1 >> 16);
+        }
+    };
+    for (int e = tid * 4; e < G * D; e += NT * 4) {
+        const int g = e / D, d = e - g * D;
+        float M = kNegInf;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) M = fmaxf(M, s_ml[w][g][0]);
+        float L = 0.f;
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const float mw = s_ml[w][g][0];
+            const float sc = mw == kNegInf ? 0.f : fast_exp2(mw - M);
+            L += sc * s_ml[w][g][1];
+            const float4 v = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(s_ring[w]) + e);
+            acc.x += sc * v.x;
+            acc.y += sc * v.y;
+            acc.z += sc * v.z;
+            acc.w += sc * v.w;
+        }
+        if (n_splits == 1) {
+            const float inv = 1.f / L;
+            store_out(g, d, make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv));
+        } else {
+            // Agent-scope stores: written through to where every XCD's agent-scope loads
+            // read (the merging workgroup may run behind another L2).
+            const int64_t slot = ((int64_t)seq * p.num_heads + head0 + g) * p.max_parts + split;
+            const uint64_t lo = (uint64_t)__builtin_bit_cast(uint32_t, acc.y) << 32 | __builtin_bit_cast(uint32_t, acc.x);
+            const uint64_t hi = (uint64_t)__builtin_bit_cast(uint32_t, acc.w) << 32 | __builtin_bit_cast(uint32_t, acc.z);
+            uint64_t* po = reinterpret_cast<uint64_t*>(p.ws_o + slot * D + d);
+            __hip_atomic_store(po, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(po + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (d == 0) {
+                const uint64_t ml = (uint64_t)__builtin_bit_cast(uint32_t, L) << 32 | __builtin_bit_cast(uint32_t, M);
+                __hip_atomic_store(reinterpret_cast<uint64_t*>(p.ws_ml + slot * 2), ml, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+    }
+    if (n_splits == 1) return;
+
+    // ---- the last workgroup of the (sequence, KV head) to get here merges its runs, in run
+    // order, and returns the counter to zero for the next call. The partial stores above are
+    // performed before the counter moves: s_waitcnt vmcnt(0) holds the wave until each store
+    // is acknowledged from the agent's coherence point, and the "memory" clobber keeps the
+    // compiler from moving them past it. (No agent-scope release fence: it also writes back
+    // the XCD's L2 and was measured to serialise the launch.)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    uint32_t* cnt = p.ws_cnt + ((int64_t)seq * KV + kvh);
+    if (tid == 0) s_arrived = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (s_arrived != (uint32_t)(n_splits - 1)) return;
+    if (tid == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    constexpr int CH = 8;                     // runs whose loads are in flight together
+    for (int e = tid * 4; e < G * D; e += NT * 4) {
+        const int g = e / D, d = e - g * D;
+        const int64_t base = ((int64_t)seq * p.num_heads + head0 + g) * p.max_parts;
+        uint64_t* ml = reinterpret_cast<uint64_t*>(p.ws_ml + base * 2);
+        uint64_t* po = reinterpret_cast<uint64_t*>(p.ws_o + base * D + d);
+        float M = kNegInf, L = 0.f;
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int s0 = 0; s0 < n_splits; s0 += CH) {
+            uint64_t mlv[CH], a[CH], b[CH];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                const int s = s0 + j < n_splits ? s0 + j : n_splits - 1;
+                mlv[j] = __hip_atomic_load(ml + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                a[j] = __hip_atomic_load(po + (int64_t)s * (D / 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                b[j] = __hip_atomic_load(po + (int64_t)s * (D / 2) + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            auto lo = [](uint64_t x) { return __builtin_bit_cast(float, (uint32_t)x); };
+            auto hi = [](uint64_t x) { return __builtin_bit_cast(float, (uint32_t)(x >> 32)); };
+            float Mc = M;
+#pragma unroll
+            for (int j = 0; j < CH; ++j) Mc = fmaxf(Mc, lo(mlv[j]));
+            const float rs = M == kNegInf ? 0.f : fast_exp2(M - Mc);
+            L *= rs;
+            acc.x *= rs;
+            acc.y *= rs;
+            acc.z *= rs;
+            acc.w *= rs;
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                const float mj = lo(mlv[j]);
+                const float sc = s0 + j >= n_splits || mj == kNegInf ? 0.f : fast_exp2(mj - Mc);
+                if (s0 + j < n_splits) {
+                    L += sc * hi(mlv[j]);
+                    acc.x += sc * lo(a[j]);
+                    acc.y += sc * hi(a[j]);
+                    acc.z += sc * lo(b[j]);
+                    acc.w += sc * hi(b[j]);
+                }
+            }
+            M = Mc;
+        }
+        const float inv = 1.f / L;
+        store_out(g, d, make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv));
+    }
+}
+
+// Workgroups of NW waves for one (sequence, KV head) run each.
+template <typename T, int D, int NW>
+int launch_nw(const AttnParams& p, hipStream_t stream) {
+    const int64_t pairs = (int64_t)p.num_seqs * p.num_kv_heads;
+    int64_t fits = (int64_t)kCus * wgs_per_cu(D, NW);
+    // Many pairs of long contexts: runs for two rounds, or the longest context would be
+    // walked whole (250 sequences of 512-8192 tokens, 8/2 heads, bf16: 219 -> 189 us); with
+    // less to read the second round's start and merges cost more than it evens out (64
+    // sequences of 16-2048, 12 heads of 64, fp16: 24 -> 25.5).
+    if (2 * pairs > fits && pairs * p.max_parts * kDecodePart * D * 4 > ((int64_t)1 << 30)) fits *= 2;
+    // At least 4 units a wave and run (and a workspace slot's tokens); contexts of up to 8
+    // units a wave are not worth the merge (12 layers of a GPT-2 decode step captured for
+    // 1024 tokens, 8 sequences, fp16: 161.5 -> 158.2 us with the projections).
+    const int min_run = NW * 4 > kDecodePart / kUnit ? NW * 4 : kDecodePart / kUnit;
+    // No split either where the pairs fill the GPU by themselves, or where the counters or
+    // the scan do not reach.
+    int slots = 0;
+    if (p.max_parts * (kDecodePart / kUnit) > NW * 8 && p.ws_cnt && p.num_seqs <= kMaxScanSeqs && pairs < fits &&
+        (int64_t)p.num_seqs * p.max_parts * (kDecodePart / kUnit) < ((int64_t)1 << 31))
+        slots = (int)(fits / p.num_kv_heads);
+    const int64_t grid = slots > 0 ? (int64_t)(slots > p.num_seqs ? slots : p.num_seqs) * p.num_kv_heads : pairs;
+    if (grid > 0x7fffffff) return PKV_EUNSUPPORTED;
+    paged_decode_split_kernel<T, D, NW><<<dim3((unsigned)grid), NW * 64, 0, stream>>>(p, min_run, slots);
+    return check_launch("paged decode attention (split)");
+}
+
+// Waves per workgroup: 8 while the pairs fit the GPU so (each context is walked by more
+// waves: fewer splits, shorter chains), else 4. Measured, us a call, 8 vs 4 waves: 8
+// sequences of 1-8k, 32/8 heads of 128, bf16 35.3 vs 37.5; 30 x 4096 82 vs 88; 64 sequences
+// of 16-2048, 12 heads of 64, fp16 (768 pairs, more than fit) 25.2 vs 21.9; 1000 of 1-60
+// (8000 pairs) 120 vs 70. 16 waves were never better than 8 by more than the noise, but
+// for 500 single-head sequences of 16-4000 (51 vs 58).
+template <typename T, int D>
+int launch_d(const AttnParams& p, hipStream_t stream) {
+    const int64_t pairs = (int64_t)p.num_seqs * p.num_kv_heads;
+    if (pairs <= (int64_t)kCus * wgs_per_cu(D, 8)) return launch_nw<T, D, 8>(p, stream);
+    return launch_nw<T, D, 4>(p, stream);
+}
+
+template <typename T>
+int launch_t(const AttnParams& p, hipStream_t stream) {
+    switch (p.head_dim) {
+        case 32: return launch_d<T, 32>(p, stream);
+        case 48: return launch_d<T, 48>(p, stream);
+        case 64: return launch_d<T, 64>(p, stream);
+        case 80: return launch_d<T, 80>(p, stream);
+        case 96: return launch_d<T, 96>(p, stream);
+        case 112: return launch_d<T, 112>(p, stream);
+        case 128: return launch_d<T, 128>(p, stream);
+    }
+    return PKV_EUNSUPPORTED;
+}
+
+}  // namespace
+
+bool decode_split_applies(const AttnParams& p, int dtype) {
+    if (dtype != PKV_FLOAT16 && dtype != PKV_BFLOAT16) return false;
+    if (p.num_blocks < 1 || p.block_shift < 3 || p.group > 16) return false;
+    if (p.head_dim % 16 || p.head_dim < 32 || p.head_dim > 128) return false;
+    if ((int64_t)p.num_seqs * p.num_kv_heads > 0x7fffffff) return false;
+    if (p.max_parts > 1 && (!p.ws_o || !p.ws_ml)) return false;
+    // Units of a sequence are exact in fp32 (the run search divides in it).
+    if ((int64_t)p.max_parts * kDecodePart >= ((int64_t)1 << 28)) return false;
+    // Offsets inside an 8-row half in 32 bits.
+    if (8 * p.ss * 2 + p.head_dim * 2 > 0xffffffffll || p.ss < 0) return false;
+    // 16-byte rows, those of a fused append among them.
+    uint64_t probe = (uint64_t)(uintptr_t)p.q | (uint64_t)(uintptr_t)p.k | (uint64_t)(uintptr_t)p.v |
+                     (uint64_t)(p.q_st * 2) | (uint64_t)(p.q_sh * 2) | (uint64_t)(p.sb * 2) |
+                     (uint64_t)(p.ss * 2) | (uint64_t)(p.sh * 2);
+    if (p.app_slots)
+        probe |= (uint64_t)(uintptr_t)p.app_k | (uint64_t)(uintptr_t)p.app_v | (uint64_t)(p.app_st * 2) |
+                 (uint64_t)(p.app_sh * 2);
+    return probe % 16 == 0;
+}
+
+int launch_decode_split(const AttnParams& p, int dtype, hipStream_t stream) {
+    if (!decode_split_applies(p, dtype)) return PKV_EUNSUPPORTED;
+    if (p.num_seqs == 0) return PKV_OK;
+    return dtype == PKV_FLOAT16 ? launch_t<_Float16>(p, stream) : launch_t<bf16_t>(p, stream);
+}
+
+}  // namespace pkv

@@ -62,7 +62,7 @@ int fill_common(AttnParams& p, const char* what, void* out, int64_t out_st, int6
 
 // Layout: [merge counters, kMergeCounterBytes][ml][o] when any context spans more than
 // one partition; empty otherwise.
-// Behind the counters two layouts share the space: the partition kernels' partials
+// Behind the counters two layouts share the space: the split contexts' partials
 // ([ml][o] per (sequence, head, 256-token partition)) and the persistent MFMA kernel's
 // ([prefix table][ml][o], partials per (workgroup, side, wave, head)); the workspace
 // holds the larger. The MFMA kernel never touches the counters, so they stay zero.
@@ -167,44 +167,44 @@ int decode_impl(void* out, int64_t out_stride_t, int64_t out_stride_h, const voi
         p.ws_o = (float*)((char*)workspace + w.cnt_bytes + w.mfma_pfx_bytes + w.mfma_ml_bytes);
     }
 
-    // 16-bit shapes without a decode kernel (block sizes other than 16, other head_dims and
-    // groups) run as one-token prompts on the prefill MFMA kernel, their contexts split into
-    // the workspace's partials (never more than one per 256 tokens).
-    const bool streams = decode_streams(p, dtype);
+    auto append_first = [&]() -> int {
+        p.app_k = p.app_v = nullptr;
+        p.app_slots = nullptr;
+        return pkv_kv_append(const_cast<void*>(k_pool), const_cast<void*>(v_pool), pool_stride_block,
+                             pool_stride_slot, pool_stride_head, num_blocks, block_size, num_kv_heads, head_dim,
+                             app->k_new, app->v_new, app->st, app->sh, app->slots, num_seqs, dtype, stream);
+    };
     if (app) {
         p.app_k = app->k_new;
         p.app_v = app->v_new;
         p.app_st = app->st;
         p.app_sh = app->sh;
         p.app_slots = app->slots;
-        // The streaming kernels write the rows themselves (4-byte copies: even strides and
-        // 4-byte aligned sources), and so does the prefill kernel (16-byte rows); any other
+        // The MFMA kernels write the rows themselves: the persistent one by 4-byte copies
+        // (even strides, 4-byte aligned sources), the others from 16-byte rows. Any other
         // kernel gets the append launch first.
-        const bool fuse = streams ? app->st % 2 == 0 && app->sh % 2 == 0 &&
-                                        ((uintptr_t)app->k_new | (uintptr_t)app->v_new) % 4 == 0
-                                  : prefill_tuned(p, dtype);
-        if (!fuse) {
-            p.app_k = p.app_v = nullptr;
-            p.app_slots = nullptr;
-            rc = pkv_kv_append(const_cast<void*>(k_pool), const_cast<void*>(v_pool), pool_stride_block,
-                               pool_stride_slot, pool_stride_head, num_blocks, block_size, num_kv_heads, head_dim,
-                               app->k_new, app->v_new, app->st, app->sh, app->slots, num_seqs, dtype, stream);
-            if (rc) return rc;
-        }
+        const bool fuse = mfma ? app->st % 2 == 0 && app->sh % 2 == 0 &&
+                                     ((uintptr_t)app->k_new | (uintptr_t)app->v_new) % 4 == 0
+                               : decode_split_applies(p, dtype) || prefill_tuned(p, dtype);
+        if (!fuse && (rc = append_first())) return rc;
     }
     if (mfma) {
         rc = launch_decode_mfma(p, dtype, stream);
         if (rc != PKV_EUNSUPPORTED) return rc;
         clear_error();
-        // Not launched after all (no occupancy on this device): the partition kernels,
-        // with their own partial layout.
+        // Not launched after all (no occupancy on this device): the one-launch kernel, with
+        // its own partial layout.
         p.ws_pfx = nullptr;
         p.ws_ml = (float*)((char*)workspace + w.cnt_bytes);
         p.ws_o = (float*)((char*)workspace + w.cnt_bytes + w.ml_bytes);
+        if (p.app_slots && !decode_split_applies(p, dtype) && !prefill_tuned(p, dtype) && (rc = append_first()))
+            return rc;
     }
-    rc = streams || dtype == PKV_FLOAT32 ? launch_decode_attention(p, dtype, stream) : PKV_EUNSUPPORTED;
+    rc = dtype == PKV_FLOAT32 ? launch_decode_attention(p, stream) : launch_decode_split(p, dtype, stream);
     if (rc != PKV_EUNSUPPORTED) return rc;
     clear_error();
+    // Groups of more than 16 heads run as one-token prompts on the prefill MFMA kernel, their
+    // contexts split into the workspace's partials (never more than one per 256 tokens).
     if (prefill_tuned(p, dtype)) {
         if (w.max_parts > 1) {
             const SplitPlan plan = prefill_split_plan(num_seqs, num_heads, num_kv_heads, head_dim, num_seqs, nullptr,

@@ -1,0 +1,147 @@
+"""The one-launch MFMA decode kernel (csrc/attn_decode_split.hip) against oracle.gather at the
+16-bit bar of 2e-2: head_dims, groups, block sizes, contexts around the edges of a unit (16
+keys), a wave's round (4 or 8 units) and a run, sequence counts around the 64 lanes and 16
+sequences per lane of its run search, runs longer than the 32 units whose block ids a wave
+holds, and the fused append. Pool rows no key may come from are NaN.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from inference_server import native
+from inference_server.core.attention_hip import paged_attention_hip_launch
+from oracle.gather import paged_attention_gather as oracle_gather
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-2
+
+
+def _batch(ctx, *, dtype, d, bs, kv, group, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    need = [-(-c // bs) for c in ctx]
+    num_blocks = sum(need) + 2
+    perm = torch.randperm(num_blocks, generator=g).tolist()
+    tables = torch.zeros(len(ctx), max(need) + 1, dtype=torch.long)
+    live = torch.zeros(num_blocks, bs, dtype=torch.bool)
+    at = 0
+    for i, (c, n) in enumerate(zip(ctx, need)):
+        tables[i, :n] = torch.tensor(perm[at:at + n])
+        at += n
+        pos = torch.arange(c)
+        live[tables[i, pos // bs], pos % bs] = True
+    rand = lambda *s: torch.randn(*s, generator=g).to(dtype)  # noqa: E731
+    k, v = rand(num_blocks, bs, kv, d), rand(num_blocks, bs, kv, d)
+    k[~live], v[~live] = float("nan"), float("nan")
+    n = len(ctx)
+    return dict(q=2 * rand(n, kv * group, d), k=k, v=v, tables=tables, ctx=torch.tensor(ctx),
+                k_new=rand(n, kv, d), v_new=rand(n, kv, d))
+
+
+def _run(b, *, fused):
+    n, bs, d = len(b["ctx"]), b["k"].shape[1], b["q"].shape[2]
+    last = b["ctx"] - 1
+    slots = b["tables"][torch.arange(n), last // bs] * bs + last % bs
+    k, v = b["k"].clone(), b["v"].clone()
+    if fused:                                   # what the call must not read: the new slots
+        k.view(-1, *k.shape[2:])[slots] = float("nan")
+        v.view(-1, *v.shape[2:])[slots] = float("nan")
+    kd, vd = k.cuda(), v.cuda()
+    append = (b["k_new"].cuda(), b["v_new"].cuda(), slots.cuda()) if fused else None
+    args = (b["q"].cuda(), kd, vd, b["tables"].cuda(), b["ctx"].cuda(), torch.ones(n, dtype=torch.long).cuda(), d ** -0.5)
+    outs = [paged_attention_hip_launch(*args, append=append) for _ in range(2)]
+    torch.cuda.synchronize()
+    if fused:
+        k.view(-1, *k.shape[2:])[slots] = b["k_new"]
+        v.view(-1, *v.shape[2:])[slots] = b["v_new"]
+    bits = lambda t: t.cpu().view(torch.int16)  # noqa: E731
+    assert torch.equal(bits(kd), bits(k)) and torch.equal(bits(vd), bits(v))
+    assert torch.equal(bits(outs[0]), bits(outs[1]))        # and the merge counters were left zero
+    return outs[0].cpu(), k, v, slots
+
+
+def _check(b, *, fused, rows=None):
+    out, k, v, _ = _run(b, fused=fused)
+    rows = torch.arange(len(b["ctx"])) if rows is None else torch.tensor(rows)
+    clean = lambda t: torch.nan_to_num(t)  # noqa: E731  (never read: the oracle masks, 0 x NaN is NaN)
+    ref = oracle_gather(b["q"][rows], clean(k), clean(v), b["tables"][rows], b["ctx"][rows],
+                        torch.ones(len(rows), dtype=torch.long), b["q"].shape[2] ** -0.5)
+    torch.testing.assert_close(out[rows], ref, atol=TOL, rtol=TOL)
+
+
+EDGES = [1, 7, 8, 9, 15, 16, 17, 63, 64, 65, 127, 129, 512, 513]
+
+
+@pytest.mark.parametrize("d,bs,kv,group,dtype", [
+    (32, 8, 2, 16, torch.float16), (32, 16, 3, 1, torch.bfloat16), (48, 16, 1, 5, torch.bfloat16),
+    (64, 16, 12, 1, torch.float16), (64, 32, 3, 7, torch.bfloat16), (80, 8, 2, 2, torch.float16),
+    (80, 16, 1, 12, torch.bfloat16), (96, 64, 2, 3, torch.float16), (112, 16, 1, 4, torch.bfloat16),
+    (128, 16, 8, 4, torch.bfloat16), (128, 8, 1, 8, torch.float16), (128, 128, 2, 9, torch.float16)])
+@pytest.mark.parametrize("fused", [False, True], ids=["plain", "append"])
+def test_shapes_and_context_edges(d, bs, kv, group, dtype, fused):
+    _check(_batch(EDGES, dtype=dtype, d=d, bs=bs, kv=kv, group=group, seed=d + bs), fused=fused)
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 130, 300])
+@pytest.mark.parametrize("fused", [False, True], ids=["plain", "append"])
+def test_run_search_over_sequence_counts(n, fused):
+    """Long contexts among short ones, so that runs are cut and found across lanes."""
+    ctx = [5 + (37 * i) % 150 for i in range(n)]
+    for i, c in ((0, 3000), (n // 2, 1900), (n - 1, 4099)):
+        ctx[i] = c
+    rows = sorted({0, n // 2, n - 1, n // 3, max(0, n - 2)})
+    _check(_batch(ctx, dtype=torch.bfloat16, d=64, bs=16, kv=1, group=4, seed=n), fused=fused, rows=rows)
+
+
+@pytest.mark.parametrize("n,kv,d,long", [
+    (350, 3, 32, 2200),      # as many pairs as the GPU holds: unsplit, 34 units a wave
+    (1030, 1, 64, 300),      # more sequences than the search takes
+    (40, 3, 128, 9000)],     # runs of several chunks of block ids
+    ids=["unsplit", "many", "long"])
+def test_unsplit_and_long_runs(n, kv, d, long):
+    ctx = [1 + (29 * i) % 70 for i in range(n)]
+    ctx[1], ctx[n // 2], ctx[n - 1] = long, long - 7, long + 13
+    _check(_batch(ctx, dtype=torch.float16, d=d, bs=16, kv=kv, group=2, seed=n + d), fused=True,
+           rows=[0, 1, 2, n // 2, n - 2, n - 1])
+
+
+def test_contexts_of_zero_write_nothing_and_split_nothing():
+    b = _batch([2500, 40, 17], dtype=torch.float16, d=128, bs=16, kv=2, group=4, seed=5)
+    ref, _, _, _ = _run(b, fused=False)
+    L, dev, s = native.lib(), "cuda", torch.cuda.current_stream().cuda_stream
+    tables = torch.cat([b["tables"][:1], torch.zeros_like(b["tables"][:1]), b["tables"][1:]]).to(dev)
+    ctx = torch.tensor([2500, 0, 40, 17], device=dev)
+    q = torch.cat([b["q"][:1], b["q"][:1], b["q"][1:]]).to(dev)
+    k, v = b["k"].to(dev), b["v"].to(dev)
+    out = torch.full((4, 8, 129), 7.0, dtype=torch.float16, device=dev)[:, :, :128]    # rows of 129: 2-byte stores
+    need = L.pkv_paged_attention_decode_workspace_bytes(4, 8, 2, 128, 2500)
+    ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+    rc = L.pkv_paged_attention_decode(out.data_ptr(), out.stride(0), out.stride(1), q.data_ptr(), q.stride(0),
+                                      q.stride(1), k.data_ptr(), v.data_ptr(), *k.stride()[:3], *k.shape,
+                                      tables.data_ptr(), tables.stride(0), tables.shape[1], ctx.data_ptr(), 4, 8, 2500,
+                                      128 ** -0.5, native.PKV_FLOAT16, ws.data_ptr(), need, s)
+    native.check(rc, "decode")
+    torch.cuda.synchronize()
+    assert torch.equal(out[1], torch.full_like(out[1], 7.0))
+    torch.testing.assert_close(out[[0, 2, 3]].cpu(), ref, atol=2e-3, rtol=2e-3)
+    assert int(ws[:256 * 1024].count_nonzero()) == 0
+
+
+def test_rows_off_16_bytes_are_appended_by_the_append_kernel():
+    b = _batch([33, 900, 64], dtype=torch.float16, d=64, bs=16, kv=2, group=2, seed=8)
+    plain = _run(b, fused=True)[0]
+    wide = torch.zeros(3, 2, 66, dtype=torch.float16)
+    odd = dict(b)
+    for name in ("k_new", "v_new"):
+        w = wide.clone().cuda()
+        w[:, :, 2:] = b[name].cuda()
+        odd[name] = w[:, :, 2:]
+    n, bs = 3, 16
+    last = b["ctx"] - 1
+    slots = b["tables"][torch.arange(n), last // bs] * bs + last % bs
+    kd, vd = b["k"].cuda(), b["v"].cuda()
+    out = paged_attention_hip_launch(b["q"].cuda(), kd, vd, b["tables"].cuda(), b["ctx"].cuda(),
+                                     torch.ones(n, dtype=torch.long).cuda(), 64 ** -0.5,
+                                     append=(odd["k_new"], odd["v_new"], slots.cuda()))
+    assert torch.equal(out.cpu(), plain)
