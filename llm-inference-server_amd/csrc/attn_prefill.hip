@@ -408,10 +408,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
         asm volatile("" : "+v"(voff_lo[t]), "+v"(voff_hi[t]));
     }
 
-    // The first tile's block ids, then everything that needs no id, so that one memory
-    // round trip covers them all; the fused append's stores go out behind the first DMAs
-    // (in front of them, with its row loads behind the slot's, it held every workgroup up
-    // for 5.8 us on config 4 chunks).
+    // The first tile's block ids, then the queries, so that one memory round trip covers
+    // both.
     int64_t ids = tile_ids(t_begin);
     // Q^T B operand: lane supplies Q[query my_q][d = 16*step + 8*h .. +8].
     u32x4 qfrag[DSTEPS];
@@ -428,7 +426,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
     // Fused KV append (p.app_k set): the new K/V rows of the tokens whose first query row
     // is this workgroup's go to their pool slots (the first split writes them). Nothing in
     // this launch reads those slots: every workgroup stages positions >= pos0 from the
-    // source rows instead (dma_tile), so no workgroup waits for another.
+    // source rows instead (dma_tile), so no workgroup waits for another. It happens behind
+    // the last tile: in front of the first one it held every workgroup up for 5.8 us (config 4
+    // chunks), behind the first DMAs for 2.5-6 us (mixed chunks, 32 heads of 80: 47.2 -> 45.8
+    // us a call for the move to the end; short tails 55.4 -> 54.2).
     constexpr int kAppend = 4;                // 16-byte pieces of K and V in flight per thread
     const int tok_begin = (int)(((uint32_t)row0 + G - 1) / G);
     const int n_pieces =
@@ -462,13 +463,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
             store16(const_cast<char*>(vbase) + dst, app_v[j]);
         }
     };
-    if (n_pieces) append_load(0);
     dma_tile(t_begin, ids, s_k0, s_v0);
     ids = tile_ids(t_begin + 1);
-    for (int i0 = 0; i0 < n_pieces; i0 += kAppend * 256) {
-        if (i0) append_load(i0);
-        append_store(i0);
-    }
     // One tile: wait for this wave's DMA of tile kt, meet the other waves (their DMAs
     // have landed and they are done with tile kt-1, so its buffer is free), compute S^T,
     // start the DMA of tile kt+1 into the free buffer, then the softmax and P·V.
@@ -580,6 +576,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
         if (kt + 1 < t_end) tile(kt + 1, s_k1, s_v1, s_k0, s_v0);
     }
 
+    for (int i0 = 0; i0 < n_pieces; i0 += kAppend * 256) {
+        append_load(i0);
+        append_store(i0);
+    }
     // ---- store: the lane holds d = 32 t + 8 (r/4) + 4 h + r%4 of its query row.
     if (!my_live) return;
     const int64_t tok = q_first + my_q;
