@@ -127,11 +127,11 @@ int64_t pkv_paged_attention_decode_workspace_bytes(int64_t num_seqs, int64_t num
  * max_context_len x head_dim x 4 bytes) reaches 512 MiB, with a multiple of 4 KV heads
  * and at most 1024 sequences, run the persistent MFMA kernel (equal runs of 16-key
  * blocks per workgroup, then a small merge kernel for the sequences the runs cut);
- * other 16-bit batches of head_dims 32..128 (multiples of 16), groups up to 16 and
- * power-of-two block sizes from 8 run the one-launch MFMA kernel (contexts cut into runs
- * that fit the GPU, merged in place), groups above 16 the prefill kernel; fp32 runs the
- * register kernel plus its merge
- * kernel. All launch on the same stream; calls that overlap in time (different
+ * fp32 batches of much K/V with ungrouped heads of 64 run the register kernel and its
+ * merge kernel; any other batch of head_dims 32..128 (multiples of 16), groups up to 16 and
+ * power-of-two block sizes from 8 runs the one-launch MFMA kernel (contexts cut into runs
+ * that fit the GPU, merged in place), 16-bit groups above 16 the prefill kernel, the rest
+ * the generic kernel. All launch on the same stream; calls that overlap in time (different
  * streams) need distinct workspaces. */
 int pkv_paged_attention_decode(
     void* out, int64_t out_stride_t, int64_t out_stride_h,
@@ -152,8 +152,8 @@ int pkv_paged_attention_decode(
  * pkv_paged_attention_decode computes over the updated pool (context_lens include the
  * new token). Replaces, per layer of a decode step, `_PagedCache.update`
  * (inference_server/core/paged_executor.py:116-125) followed by the decode attention
- * (inference_server/core/attention.py:130-153). With 16-bit pools and 16-byte
- * aligned rows the attention kernel writes each row itself, from the wave that reads that
+ * (inference_server/core/attention.py:130-153). On most shapes,
+ * given 16-byte aligned rows, the attention kernel writes each row itself, from the wave that reads that
  * token (no append launch); otherwise the append kernel runs first. Contract: slots[i] is
  * the slot of position context_lens[i] - 1 of sequence i, and no other sequence's
  * table reaches it (the reference's copy-on-write guarantees both); slots outside the

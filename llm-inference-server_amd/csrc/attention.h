@@ -59,6 +59,10 @@ struct AttnParams {
 // p.app_* set: including the fused append, whose source rows must be 16-byte aligned).
 bool decode_split_applies(const AttnParams& p, int dtype);
 int launch_decode_split(const AttnParams& p, int dtype, hipStream_t stream);
+// fp32 register kernel (attn_decode.hip): the shapes and sizes where it beats the kernel
+// above; it appends nothing itself.
+bool decode_f32_applies(const AttnParams& p);
+int launch_decode_f32(const AttnParams& p, hipStream_t stream);
 // True when launch_prefill_attention runs the MFMA kernel for these parameters (with
 // p.app_* set: including the fused append, whose source rows must be 16-byte aligned).
 bool prefill_tuned(const AttnParams& p, int dtype);
@@ -83,9 +87,8 @@ constexpr int64_t kSplitMinContext = 1024;
 // size, so counters never overlap another call's partials in a reused workspace).
 constexpr int64_t kMergeCounterBytes = 256 * 1024;
 
-// Tokens per split-KV partition of the decode kernel (one workgroup's share).
-// Measured on config 4 (ragged contexts 512-8192): 256 -> 5.03 TB/s, 512 -> 4.81,
-// 128 -> 4.80 (512 wins only for uniform long contexts, 5.44 vs 5.31).
+// Tokens per split-KV partial that the decode workspace holds: a run of a split context is
+// never shorter.
 constexpr int kDecodePart = 256;
 
 // Persistent MFMA decode (attn_decode_mfma.hip): whether it takes a batch of these
@@ -103,7 +106,7 @@ int launch_decode_mfma(const AttnParams& p, int dtype, hipStream_t stream);
 
 int launch_generic_attention(const AttnParams& p, int dtype, hipStream_t stream);
 // fp32 pools, block size 16, head_dim 64/128, GQA 1/2/4/8, 16-byte aligned rows: the
-// tiled fp32 kernel (any query lengths; p.qsl null for a decode batch). Returns
+// tiled fp32 kernel (any query lengths). Returns
 // PKV_EUNSUPPORTED (without setting an error) for anything else.
 int launch_f32_attention(const AttnParams& p, hipStream_t stream);
 // fp32 pools, prefill / chunked-prefill batches (p.qsl set, no fused append, a row of at
@@ -111,7 +114,6 @@ int launch_f32_attention(const AttnParams& p, hipStream_t stream);
 // fp32 MFMA kernel. Returns PKV_EUNSUPPORTED (without setting an error) for anything else.
 int launch_prefill_f32_mfma(const AttnParams& p, hipStream_t stream);
 // Returns PKV_EUNSUPPORTED (without setting an error) when no tuned kernel matches.
-int launch_decode_attention(const AttnParams& p, hipStream_t stream);
 int launch_prefill_attention(const AttnParams& p, int dtype, hipStream_t stream);
 
 // ---- prefill dispatch order (the MFMA prefill kernels, 256-thread workgroups).

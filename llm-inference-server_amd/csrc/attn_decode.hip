@@ -1,9 +1,17 @@
-// Paged decode attention for fp32 pools, block_size 16, head_dim 64, GQA group 1/2/4/8: a
-// partition kernel with K/V staged in registers, and a split-KV merge kernel.
+// Paged decode attention for fp32 pools, block_size 16, head_dim 64, ungrouped heads, for
+// batches of much K/V: a partition kernel with K/V staged in registers, and a split-KV merge
+// kernel.
+//
+// Bound: HBM and the arithmetic beside it. With one head a group the one-launch MFMA kernel
+// (attn_decode_split.hip) spends its fp32 matrix steps on 16 columns of which one counts;
+// here each product is computed once. Measured, us a call with the append launch, this kernel
+// first, 12 heads: 32 sequences of 16-1024 tokens 27.3 vs 29.0, 60 of 16-2000 73 vs 77; with
+// less K/V its second launch decides: 22 of 16-1000 24.7 vs 22.8, 32 of 16-300 24.5 vs 22.1.
+// Groups of 2 are even (64 of 16-1000 38.0 vs 38.5), larger ones lose (16 of 100-3000, groups
+// of 8, 26.8 vs 20.5).
 //
 //  * Work unit = (KV head, 256-token partition, sequence): one 256-thread workgroup of 4
-//    wave64s, 64 tokens (4 blocks) per wave. All G query heads of the GQA group are served
-//    by the same K/V read.
+//    wave64s, 64 tokens (4 blocks) per wave.
 //  * Latency chain per wave: ONE vector load of the wave's 4 block-table entries (broadcast
 //    with readlane), then all K loads of the 4 blocks at once, the scores, then all V loads
 //    at once, issued before the softmax so they are in flight while it runs.
@@ -24,47 +32,20 @@ constexpr int kTPW = 64;
 constexpr int kBPW = kTPW / kBS;          // blocks per wave
 
 // Partial dot product of one 16-byte chunk of K with the matching chunk of q.
-template <typename T>
-struct ChunkDot {
-    __device__ __forceinline__ static float run(const Vec16& k, const Vec16& q, float acc) {
+__device__ __forceinline__ float chunk_dot(const Vec16& k, const Vec16& q, float acc) {
 #pragma unroll
-        for (int w = 0; w < 4; ++w) acc = Pair<T>::dot2(k.w[w], q.w[w], acc);
-        return acc;
-    }
-};
-template <>
-struct ChunkDot<float> {
-    __device__ __forceinline__ static float run(const Vec16& k, const Vec16& q, float acc) {
-#pragma unroll
-        for (int w = 0; w < 4; ++w)
-            acc = fmaf(__builtin_bit_cast(float, k.w[w]), __builtin_bit_cast(float, q.w[w]), acc);
-        return acc;
-    }
-};
-
-// Two probabilities packed (round to nearest even) into the 16-bit pool dtype.
-template <typename T>
-__device__ __forceinline__ uint32_t pack_probs(float lo, float hi);
-template <>
-__device__ __forceinline__ uint32_t pack_probs<bf16_t>(float lo, float hi) {
-    bf16x2_t v = {(__bf16)lo, (__bf16)hi};
-    return __builtin_bit_cast(uint32_t, v);
-}
-template <>
-__device__ __forceinline__ uint32_t pack_probs<_Float16>(float lo, float hi) {
-    half2_t v = {(_Float16)lo, (_Float16)hi};
-    return __builtin_bit_cast(uint32_t, v);
+    for (int w = 0; w < 4; ++w)
+        acc = fmaf(__builtin_bit_cast(float, k.w[w]), __builtin_bit_cast(float, q.w[w]), acc);
+    return acc;
 }
 
-// K/V rows are read exactly once per launch: streaming loads (config 4: 5.02 TB/s
-// with them, 4.80 TB/s with cached loads).
+// K/V rows are read exactly once per launch: streaming loads.
 __device__ __forceinline__ Vec16 kv_load16(const void* ptr) { return load16_stream(ptr); }
 __device__ __forceinline__ uint2 kv_load8(const void* ptr) { return load8_stream(ptr); }
-// Cache-policy operand of global_load_lds for the same streaming data: nontemporal.
-constexpr int kDmaNontemporal = 2;
 
-template <typename T, int D, int G>
+template <int D, int G>
 __global__ __launch_bounds__(kWaves * 64) void paged_decode_kernel(const AttnParams p) {
+    using T = float;
     constexpr int ISZ = (int)sizeof(T);
     constexpr int CHUNKS = D * ISZ / 16;      // K: 16-byte chunks per (token, head) row
     constexpr int KLPT = 8;                   // K: lanes per token (8 x 16 B = one 128-byte line)
@@ -74,7 +55,6 @@ __global__ __launch_bounds__(kWaves * 64) void paged_decode_kernel(const AttnPar
     constexpr int VLPT = D * ISZ / 8;         // V: lanes per token
     constexpr int TSV = 64 / VLPT;            // V: tokens per load step
     constexpr int VSTEPS = kTPW / TSV;        // V: load steps per wave
-    constexpr bool kPacked = ISZ == 2;        // fp16/bf16: P·V through v_dot2
     static_assert(CHUNKS % KLPT == 0 && G <= KLPT && 64 % VLPT == 0 && kBS % TSV == 0 && VSTEPS % 2 == 0,
                   "unsupported head_dim / group");
 
@@ -172,7 +152,7 @@ __global__ __launch_bounds__(kWaves * 64) void paged_decode_kernel(const AttnPar
                 for (int g = 0; g < G; ++g) {
                     float s = 0.f;
 #pragma unroll
-                    for (int i = 0; i < CPL; ++i) s = ChunkDot<T>::run(kv[b][gr][i], q[g][i], s);
+                    for (int i = 0; i < CPL; ++i) s = chunk_dot(kv[b][gr][i], q[g][i], s);
                     s = ref_score_log2<T>(octet_sum(s), p.scale);
                     if (g == kj) s_p[wave][t_rel][g] = valid ? s : kNegInf;
                 }
@@ -216,38 +196,14 @@ __global__ __launch_bounds__(kWaves * 64) void paged_decode_kernel(const AttnPar
     for (int g = 0; g < G; ++g)
 #pragma unroll
         for (int e = 0; e < EPV; ++e) acc[g][e] = 0.f;
-    if constexpr (kPacked) {
 #pragma unroll
-        for (int st = 0; st < VSTEPS; st += 2) {
-            const int t0 = st * TSV + vslot;
-            const int t1 = t0 + TSV;
-            // (token t0, token t1) values of each element, packed for v_dot2.
-            uint32_t vp[EPV];
+    for (int st = 0; st < VSTEPS; ++st) {
+        const int t_rel = st * TSV + vslot;
 #pragma unroll
-            for (int w = 0; w < 2; ++w) {
-                const uint32_t a = w ? vv[st].y : vv[st].x;
-                const uint32_t c = w ? vv[st + 1].y : vv[st + 1].x;
-                // One v_perm_b32 each: bytes {a.0, a.1, c.0, c.1} and {a.2, a.3, c.2, c.3}.
-                vp[2 * w] = __builtin_amdgcn_perm(c, a, 0x05040100u);
-                vp[2 * w + 1] = __builtin_amdgcn_perm(c, a, 0x07060302u);
-            }
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const uint32_t pp = pack_probs<T>(s_p[wave][t0][g], s_p[wave][t1][g]);
-#pragma unroll
-                for (int e = 0; e < EPV; ++e) acc[g][e] = Pair<T>::dot2(vp[e], pp, acc[g][e]);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int st = 0; st < VSTEPS; ++st) {
-            const int t_rel = st * TSV + vslot;
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const float pg = s_p[wave][t_rel][g];
-                acc[g][0] = fmaf(pg, __builtin_bit_cast(float, vv[st].x), acc[g][0]);
-                acc[g][1] = fmaf(pg, __builtin_bit_cast(float, vv[st].y), acc[g][1]);
-            }
+        for (int g = 0; g < G; ++g) {
+            const float pg = s_p[wave][t_rel][g];
+            acc[g][0] = fmaf(pg, __builtin_bit_cast(float, vv[st].x), acc[g][0]);
+            acc[g][1] = fmaf(pg, __builtin_bit_cast(float, vv[st].y), acc[g][1]);
         }
     }
 #pragma unroll
@@ -308,8 +264,10 @@ __global__ __launch_bounds__(kWaves * 64) void paged_decode_kernel(const AttnPar
 template <int G, int D>
 constexpr int kCombineThreads = (G * D / 2 + 63) / 64 * 64 < 256 ? (G * D / 2 + 63) / 64 * 64 : 256;
 
-template <typename T, int D, int G, int PART>
+template <int D, int G>
 __global__ __launch_bounds__((kCombineThreads<G, D>)) void paged_decode_combine_kernel(const AttnParams p) {
+    using T = float;
+    constexpr int PART = kDecodePart;
     const int kvh = (int)blockIdx.x;
     const int seq = (int)blockIdx.y;
     int64_t ctx64 = p.ctx_lens[seq];
@@ -359,46 +317,35 @@ __global__ __launch_bounds__((kCombineThreads<G, D>)) void paged_decode_combine_
     }
 }
 
-// Instantiated only where the query registers (G * D / 8 VGPRs per lane) leave room for the
-// in-flight K and V loads without spilling: at most 64 VGPRs of query per lane, and no
-// head_dim 128 (its V step alone would take 128 VGPRs). Other shapes take the tiled fp32
-// kernel (attn_f32.hip).
-template <int D, int G>
-constexpr bool kDecodeFits = G * D * 4 <= 2048 && D <= 64;
-
 template <int D, int G>
 int launch_g(const AttnParams& p, dim3 grid, hipStream_t stream) {
-    if constexpr (kDecodeFits<D, G>) {
-        paged_decode_kernel<float, D, G><<<grid, kWaves * 64, 0, stream>>>(p);
-        int rc = check_launch("paged decode attention");
-        if (rc || p.max_parts == 1) return rc;
-        paged_decode_combine_kernel<float, D, G, kDecodePart>
-            <<<dim3(grid.x, grid.z), kCombineThreads<G, D>, 0, stream>>>(p);
-        return check_launch("paged decode combine");
-    }
-    return PKV_EUNSUPPORTED;
+    paged_decode_kernel<D, G><<<grid, kWaves * 64, 0, stream>>>(p);
+    int rc = check_launch("paged decode attention");
+    if (rc || p.max_parts == 1) return rc;
+    paged_decode_combine_kernel<D, G><<<dim3(grid.x, grid.z), kCombineThreads<G, D>, 0, stream>>>(p);
+    return check_launch("paged decode combine");
 }
+
+// K/V (at the batch's longest context) from which this kernel is the faster one (see above).
+constexpr int64_t kMinBytes = (int64_t)160 << 20;
 
 }  // namespace
 
-int launch_decode_attention(const AttnParams& p, hipStream_t stream) {
-    if (p.block_size != kBS || p.head_dim != 64) return PKV_EUNSUPPORTED;
-    if (p.num_kv_heads > 65535 || p.max_parts > 65535 || p.num_seqs > 65535) return PKV_EUNSUPPORTED;
-    if (p.max_parts > 1 && (!p.ws_o || !p.ws_ml)) return PKV_EUNSUPPORTED;
+bool decode_f32_applies(const AttnParams& p) {
+    if (p.block_size != kBS || p.head_dim != 64 || p.group != 1) return false;
+    if ((int64_t)p.num_seqs * p.num_kv_heads * p.max_parts * kDecodePart * 64 * 8 < kMinBytes) return false;
+    if (p.num_kv_heads > 65535 || p.max_parts > 65535 || p.num_seqs > 65535) return false;
+    if (p.max_parts > 1 && (!p.ws_o || !p.ws_ml)) return false;
     // 16-byte chunk loads need 16-byte aligned rows.
     const uint64_t probe = (uint64_t)(uintptr_t)p.q | (uint64_t)(uintptr_t)p.k | (uint64_t)(uintptr_t)p.v |
                            (uint64_t)(p.q_st * 4) | (uint64_t)(p.q_sh * 4) | (uint64_t)(p.sb * 4) |
                            (uint64_t)(p.ss * 4) | (uint64_t)(p.sh * 4);
-    if (probe % 16) return PKV_EUNSUPPORTED;
-    if (p.num_seqs == 0) return PKV_OK;
-    dim3 grid((unsigned)p.num_kv_heads, (unsigned)p.max_parts, (unsigned)p.num_seqs);
-    switch (p.group) {
-        case 1: return launch_g<64, 1>(p, grid, stream);
-        case 2: return launch_g<64, 2>(p, grid, stream);
-        case 4: return launch_g<64, 4>(p, grid, stream);
-        case 8: return launch_g<64, 8>(p, grid, stream);
-    }
-    return PKV_EUNSUPPORTED;
+    return probe % 16 == 0;
+}
+
+int launch_decode_f32(const AttnParams& p, hipStream_t stream) {
+    if (!decode_f32_applies(p)) return PKV_EUNSUPPORTED;
+    return launch_g<64, 1>(p, dim3((unsigned)p.num_kv_heads, (unsigned)p.max_parts, (unsigned)p.num_seqs), stream);
 }
 
 }  // namespace pkv

@@ -1,6 +1,6 @@
-// Paged decode attention on MFMA (gfx950) in one launch, fp16/bf16, head_dim a multiple of
-// 16 from 32 to 128, GQA groups up to 16, block sizes that are powers of two from 8 up.
-// Takes every such decode batch below the size from which the persistent kernel
+// Paged decode attention on MFMA (gfx950) in one launch, fp32/fp16/bf16, head_dim a multiple
+// of 16 from 32 to 128, GQA groups up to 16, block sizes that are powers of two from 8 up.
+// Takes every such decode batch, in 16 bits below the size from which the persistent kernel
 // (attn_decode_mfma.hip) is the better one.
 //
 // Bound: HBM for batches of tens of MB, latency below that. Every K/V byte is read once
@@ -20,9 +20,10 @@
 //    filled by nontemporal LDS DMA; a unit's K and V^T fragments are read into registers
 //    first and the slot refilled with the unit after next at once. Waits are explicit vmcnt
 //    counts; DMAs and ring reads are inline asm, unseen by the compiler's wait counting.
-//  * Contraction as in the persistent kernel: S^T = K Q^T on 16x16x32, P^T straight from the
+//  * Contraction (Contract), in 16 bits as in the persistent kernel: S^T = K Q^T on 16x16x32, P^T straight from the
 //    accumulator into O^T += V^T P^T on 16x16x16, V^T by the transposing LDS read. 12 MFMAs
 //    and ~80 VALU instructions per unit at head_dim 128, where v_dot2 arithmetic took ~900.
+//    fp32 on 16x16x4.
 //  * Merge: the waves' partials meet in LDS; split contexts leave fp32 partials that the
 //    last workgroup of each (sequence, KV head) to finish merges in run order (agent-scope
 //    stores, one counter, no workgroup ever waits for another).
@@ -53,11 +54,37 @@ typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
-// MFMA lane layouts as pinned for the persistent kernel (attn_decode_mfma.hip).
+// 16-byte LDS read / transposing LDS read (ds_read_b64_tr_b16: within 16 lanes, source lane c
+// pointing at V[key0 + c / 4][d0 + 4 (c % 4)], lane i receives V[key0 .. key0 + 3][d0 + i]).
+__device__ __forceinline__ u32x4 lds_read16(const char* ptr) {
+    const uint4 v = *reinterpret_cast<const uint4*>(ptr);
+    return u32x4{v.x, v.y, v.z, v.w};
+}
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint2 lds_read_tr16(const char* ptr) {
+    const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(ptr));
+    return __builtin_bit_cast(uint2, v);
+}
+// Waits that also keep the compiler's memory operations on their side: the ring's DMAs are
+// unseen by it, so nothing else orders LDS reads against them.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// The contraction of one unit, from its ring slot. MFMA lane layouts as pinned for the
+// persistent kernel (attn_decode_mfma.hip): 16x16xK puts A[i][k] in lane i + 16 (k / (K/4)),
+// B[k][j] in lane j + 16 (k / (K/4)), D[i][j] in lane j + 16 (i / 4), register i % 4.
 template <typename T>
-struct SMfma;
+struct Half {
+    __device__ __forceinline__ static uint32_t pack(float lo, float hi);
+    __device__ __forceinline__ static f32x4 qk(u32x4 a, u32x4 b, f32x4 c);
+    __device__ __forceinline__ static f32x4 pv(uint2 a, uint2 b, f32x4 c);
+    __device__ __forceinline__ static float round(float x);
+};
 template <>
-struct SMfma<bf16_t> {
+struct Half<bf16_t> {
     __device__ __forceinline__ static f32x4 qk(u32x4 a, u32x4 b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b),
                                                        c, 0, 0, 0);
@@ -73,7 +100,7 @@ struct SMfma<bf16_t> {
     __device__ __forceinline__ static float round(float x) { return (float)(__bf16)x; }
 };
 template <>
-struct SMfma<_Float16> {
+struct Half<_Float16> {
     __device__ __forceinline__ static f32x4 qk(u32x4 a, u32x4 b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c,
                                                       0, 0, 0);
@@ -89,15 +116,151 @@ struct SMfma<_Float16> {
     __device__ __forceinline__ static float round(float x) { return (float)(_Float16)x; }
 };
 
-// Physical 16-byte slot of logical chunk c of ring row r is c ^ unit_swizzle(r): the 16 rows
-// of a K read fall in different banks (at head_dim 48, 80 and 112 in pairs).
+// 16-bit pools: S^T on 16x16x32 (the K read of step j gives a lane 8 dims), O^T on 16x16x16
+// from the transposing V read, probabilities in the pool dtype.
+template <typename T, int D>
+struct Contract {
+    static constexpr int KS = (D + 31) / 32;  // 16-byte K (and Q) pieces per lane
+    static constexpr int VT = D / 16;
+    static constexpr int CPR = D * 2 / 16;
+    // Physical 16-byte slot of logical chunk c of ring row r is c ^ swizzle(r): the 16 rows
+    // of a K read fall in different banks (at head_dim 48, 80 and 112 in pairs).
+    __device__ __forceinline__ static int swizzle(int r) {
+        if constexpr (D == 128) return ((r & 3) << 2) | ((r >> 2) & 3);
+        else if constexpr (D == 64) return (((r >> 1) & 1) << 2) | (((r >> 2) & 1) << 1) | ((r >> 3) & 1);
+        else if constexpr (D % 32 == 0) return (r >> 2) & 3;
+        else return (r >> 3) & 1;
+    }
+    __device__ __forceinline__ static int k_chunk(int j, int lg) { return 4 * j + lg; }
+    u32x4 kf[KS];
+    uint2 vf[VT];
+    uint32_t k_addr[KS], v_addr[VT];
+    // Per-lane addresses inside a unit: K row ln, chunk 4 j + lg (one past head_dim re-reads
+    // another and is zeroed); V^T rows 4 lg + ln / 4, columns 16 t + 4 (ln % 4).
+    __device__ __forceinline__ void address(int lg, int ln) {
+#pragma unroll
+        for (int j = 0; j < KS; ++j) {
+            const int c = 4 * j + lg < CPR ? 4 * j + lg : 4 * j + (lg & 1);
+            k_addr[j] = (uint32_t)(ln * D * 2 + ((c ^ swizzle(ln)) << 4));
+        }
+        const int row = 4 * lg + (ln >> 2);
+#pragma unroll
+        for (int t = 0; t < VT; ++t)
+            v_addr[t] = (uint32_t)(row * D * 2 + (((2 * t + ((ln & 3) >> 1)) ^ swizzle(row)) << 4) + 8 * (ln & 1));
+    }
+    __device__ __forceinline__ void read(const char* k, const char* v, int lg) {
+#pragma unroll
+        for (int j = 0; j < KS; ++j) kf[j] = lds_read16(k + k_addr[j]);
+#pragma unroll
+        for (int t = 0; t < VT; ++t) vf[t] = lds_read_tr16(v + v_addr[t]);
+        wait_lds();
+        if constexpr (D % 32 != 0)
+            if (lg >= 2) kf[KS - 1] = u32x4{0u, 0u, 0u, 0u};
+    }
+    __device__ __forceinline__ f32x4 scores(const u32x4 (&qf)[KS]) const {
+        f32x4 st = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < KS; ++j) st = Half<T>::qk(kf[j], qf[j], st);
+        return st;
+    }
+    __device__ __forceinline__ static float scaled(float dot, float scale) {
+        return Half<T>::round(Half<T>::round(dot) * scale) * kLog2e;
+    }
+    __device__ __forceinline__ void accumulate(const float (&pr)[4], f32x4 (&o)[VT]) const {
+        const uint2 pb = make_uint2(Half<T>::pack(pr[0], pr[1]), Half<T>::pack(pr[2], pr[3]));
+#pragma unroll
+        for (int t = 0; t < VT; ++t) o[t] = Half<T>::pv(vf[t], pb, o[t]);
+    }
+    __device__ __forceinline__ static void store4(T* to, float4 v, bool wide) {
+        const uint32_t w0 = Half<T>::pack(v.x, v.y), w1 = Half<T>::pack(v.z, v.w);
+        if (wide) {
+            *reinterpret_cast<uint2*>(to) = make_uint2(w0, w1);
+        } else {
+            uint16_t* o16 = reinterpret_cast<uint16_t*>(to);
+            o16[0] = (uint16_t)w0;
+            o16[1] = (uint16_t)(w0 >> 16);
+            o16[2] = (uint16_t)w1;
+            o16[3] = (uint16_t)(w1 >> 16);
+        }
+    }
+};
+
+// fp32 pools: 16x16x4, one element per lane and step. S^T: a 16-byte K read gives a lane four
+// dims, one for each of four steps (Q^T is held in the same order). O^T: step r takes keys
+// 4 lg + r, whose probabilities are accumulator register r as it stands; V^T by 4-byte reads.
+// Nothing is rounded below fp32.
 template <int D>
-__device__ __forceinline__ int unit_swizzle(int r) {
-    if constexpr (D == 128) return ((r & 3) << 2) | ((r >> 2) & 3);
-    else if constexpr (D == 64) return (((r >> 1) & 1) << 2) | (((r >> 2) & 1) << 1) | ((r >> 3) & 1);
-    else if constexpr (D % 32 == 0) return (r >> 2) & 3;
-    else return (r >> 3) & 1;
-}
+struct Contract<float, D> {
+    static constexpr int KS = D / 16;
+    static constexpr int VT = D / 16;
+    static constexpr int CPR = D * 4 / 16;
+    // Conflict-free at D = 64 and 128: the 16 rows of a K read go to 16 slots, the rows 4 lg + r
+    // of a V read to four different 64-byte groups.
+    __device__ __forceinline__ static int swizzle(int r) {
+        if constexpr (D % 64 == 0) return r & 15;
+        else if constexpr (D == 32) return r & 7;
+        else return r & 3;
+    }
+    __device__ __forceinline__ static int k_chunk(int j, int lg) { return 4 * j + lg; }
+    u32x4 kf[KS];
+    float vf[4][VT];
+    uint32_t k_addr[KS];
+    int lg_, ln_;
+    __device__ __forceinline__ void address(int lg, int ln) {
+#pragma unroll
+        for (int j = 0; j < KS; ++j) k_addr[j] = (uint32_t)(ln * D * 4 + (((4 * j + lg) ^ swizzle(ln)) << 4));
+        lg_ = lg;
+        ln_ = ln;
+    }
+    __device__ __forceinline__ void read(const char* k, const char* v, int) {
+#pragma unroll
+        for (int j = 0; j < KS; ++j) kf[j] = lds_read16(k + k_addr[j]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = 4 * lg_ + r;
+#pragma unroll
+            for (int t = 0; t < VT; ++t)
+                vf[r][t] = *reinterpret_cast<const float*>(v + row * D * 4 + (((4 * t + (ln_ >> 2)) ^ swizzle(row)) << 4) +
+                                                           4 * (ln_ & 3));
+        }
+        wait_lds();
+    }
+    __device__ __forceinline__ f32x4 scores(const u32x4 (&qf)[KS]) const {
+        // Eight chains, summed as a tree: shorter ones are faster (each step waits for the one
+        // before it) and lose less (a score's rounding errors are the output's).
+        f32x4 st[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) st[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < KS; ++j) {
+            const f32x4 a = __builtin_bit_cast(f32x4, kf[j]), b = __builtin_bit_cast(f32x4, qf[j]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                st[4 * (j & 1) + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], st[4 * (j & 1) + e], 0, 0, 0);
+        }
+        return ((st[0] + st[1]) + (st[2] + st[3])) + ((st[4] + st[5]) + (st[6] + st[7]));
+    }
+    __device__ __forceinline__ static float scaled(float dot, float scale) { return ref_score_log2<float>(dot, scale); }
+    __device__ __forceinline__ void accumulate(const float (&pr)[4], f32x4 (&o)[VT]) const {
+#pragma unroll
+        for (int t = 0; t < VT; ++t) {
+            f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) a = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[r][t], pr[r], a, 0, 0, 0);
+            o[t] += a;
+        }
+    }
+    __device__ __forceinline__ static void store4(float* to, float4 v, bool wide) {
+        if (wide) {
+            *reinterpret_cast<float4*>(to) = v;
+        } else {
+            to[0] = v.x;
+            to[1] = v.y;
+            to[2] = v.z;
+            to[3] = v.w;
+        }
+    }
+};
 
 __device__ __forceinline__ uint32_t lds_addr(const void* ptr) {
     return (uint32_t)(uintptr_t)((const __attribute__((address_space(3))) char*)ptr);
@@ -117,98 +280,6 @@ __device__ __forceinline__ void dma16_nt(const char* addr, uint32_t lds) {
                  : "s"(lds), "v"(addr)
                  : "memory");
 }
-
-// A unit's MFMA operands from its ring slot: KS b128 reads of K and VT transposing reads of
-// V, all issued, then waited for. Each read and the wait are asm statements of their own,
-// kept in order by "memory"; the results pass through the waiting statement, so no use of
-// them can move above it.
-template <int KS, int VT>
-__device__ __forceinline__ void ring_read(uint32_t kb, const uint32_t (&ka)[KS], uint32_t vb, const uint32_t (&va)[VT],
-                                          u32x4 (&kf)[KS], uint2 (&vf)[VT]);
-
-#define PKV_RD_K(i, a) "ds_read_b128 %" #i ", %" #a "\n\t"
-#define PKV_RD_V(i, a) "ds_read_b64_tr_b16 %" #i ", %" #a "\n\t"
-#define PKV_OUT(x) "=&v"(x)
-#define PKV_IN(x) "v"(x)
-
-template <>
-__device__ __forceinline__ void ring_read<1, 2>(uint32_t kb, const uint32_t (&ka)[1], uint32_t vb,
-                                                const uint32_t (&va)[2], u32x4 (&kf)[1], uint2 (&vf)[2]) {
-    asm volatile(PKV_RD_K(0, 3) PKV_RD_V(1, 4) PKV_RD_V(2, 5) "s_waitcnt lgkmcnt(0)"
-                 : PKV_OUT(kf[0]), PKV_OUT(vf[0]), PKV_OUT(vf[1])
-                 : PKV_IN(kb + ka[0]), PKV_IN(vb + va[0]), PKV_IN(vb + va[1])
-                 : "memory");
-}
-template <>
-__device__ __forceinline__ void ring_read<2, 3>(uint32_t kb, const uint32_t (&ka)[2], uint32_t vb,
-                                                const uint32_t (&va)[3], u32x4 (&kf)[2], uint2 (&vf)[3]) {
-    asm volatile(PKV_RD_K(0, 5) PKV_RD_K(1, 6) PKV_RD_V(2, 7) PKV_RD_V(3, 8) PKV_RD_V(4, 9) "s_waitcnt lgkmcnt(0)"
-                 : PKV_OUT(kf[0]), PKV_OUT(kf[1]), PKV_OUT(vf[0]), PKV_OUT(vf[1]), PKV_OUT(vf[2])
-                 : PKV_IN(kb + ka[0]), PKV_IN(kb + ka[1]), PKV_IN(vb + va[0]), PKV_IN(vb + va[1]), PKV_IN(vb + va[2])
-                 : "memory");
-}
-template <>
-__device__ __forceinline__ void ring_read<2, 4>(uint32_t kb, const uint32_t (&ka)[2], uint32_t vb,
-                                                const uint32_t (&va)[4], u32x4 (&kf)[2], uint2 (&vf)[4]) {
-    asm volatile(PKV_RD_K(0, 6) PKV_RD_K(1, 7) PKV_RD_V(2, 8) PKV_RD_V(3, 9) PKV_RD_V(4, 10) PKV_RD_V(5, 11)
-                     "s_waitcnt lgkmcnt(0)"
-                 : PKV_OUT(kf[0]), PKV_OUT(kf[1]), PKV_OUT(vf[0]), PKV_OUT(vf[1]), PKV_OUT(vf[2]), PKV_OUT(vf[3])
-                 : PKV_IN(kb + ka[0]), PKV_IN(kb + ka[1]), PKV_IN(vb + va[0]), PKV_IN(vb + va[1]), PKV_IN(vb + va[2]),
-                   PKV_IN(vb + va[3])
-                 : "memory");
-}
-template <>
-__device__ __forceinline__ void ring_read<3, 5>(uint32_t kb, const uint32_t (&ka)[3], uint32_t vb,
-                                                const uint32_t (&va)[5], u32x4 (&kf)[3], uint2 (&vf)[5]) {
-    asm volatile(PKV_RD_K(0, 8) PKV_RD_K(1, 9) PKV_RD_K(2, 10) PKV_RD_V(3, 11) PKV_RD_V(4, 12) PKV_RD_V(5, 13)
-                     PKV_RD_V(6, 14) PKV_RD_V(7, 15) "s_waitcnt lgkmcnt(0)"
-                 : PKV_OUT(kf[0]), PKV_OUT(kf[1]), PKV_OUT(kf[2]), PKV_OUT(vf[0]), PKV_OUT(vf[1]), PKV_OUT(vf[2]),
-                   PKV_OUT(vf[3]), PKV_OUT(vf[4])
-                 : PKV_IN(kb + ka[0]), PKV_IN(kb + ka[1]), PKV_IN(kb + ka[2]), PKV_IN(vb + va[0]), PKV_IN(vb + va[1]),
-                   PKV_IN(vb + va[2]), PKV_IN(vb + va[3]), PKV_IN(vb + va[4])
-                 : "memory");
-}
-template <>
-__device__ __forceinline__ void ring_read<3, 6>(uint32_t kb, const uint32_t (&ka)[3], uint32_t vb,
-                                                const uint32_t (&va)[6], u32x4 (&kf)[3], uint2 (&vf)[6]) {
-    asm volatile(PKV_RD_K(0, 9) PKV_RD_K(1, 10) PKV_RD_K(2, 11) PKV_RD_V(3, 12) PKV_RD_V(4, 13) PKV_RD_V(5, 14)
-                     PKV_RD_V(6, 15) PKV_RD_V(7, 16) PKV_RD_V(8, 17) "s_waitcnt lgkmcnt(0)"
-                 : PKV_OUT(kf[0]), PKV_OUT(kf[1]), PKV_OUT(kf[2]), PKV_OUT(vf[0]), PKV_OUT(vf[1]), PKV_OUT(vf[2]),
-                   PKV_OUT(vf[3]), PKV_OUT(vf[4]), PKV_OUT(vf[5])
-                 : PKV_IN(kb + ka[0]), PKV_IN(kb + ka[1]), PKV_IN(kb + ka[2]), PKV_IN(vb + va[0]), PKV_IN(vb + va[1]),
-                   PKV_IN(vb + va[2]), PKV_IN(vb + va[3]), PKV_IN(vb + va[4]), PKV_IN(vb + va[5])
-                 : "memory");
-}
-template <>
-__device__ __forceinline__ void ring_read<4, 7>(uint32_t kb, const uint32_t (&ka)[4], uint32_t vb,
-                                                const uint32_t (&va)[7], u32x4 (&kf)[4], uint2 (&vf)[7]) {
-    asm volatile(PKV_RD_K(0, 11) PKV_RD_K(1, 12) PKV_RD_K(2, 13) PKV_RD_K(3, 14) PKV_RD_V(4, 15) PKV_RD_V(5, 16)
-                     PKV_RD_V(6, 17) PKV_RD_V(7, 18) PKV_RD_V(8, 19) PKV_RD_V(9, 20) PKV_RD_V(10, 21)
-                         "s_waitcnt lgkmcnt(0)"
-                 : PKV_OUT(kf[0]), PKV_OUT(kf[1]), PKV_OUT(kf[2]), PKV_OUT(kf[3]), PKV_OUT(vf[0]), PKV_OUT(vf[1]),
-                   PKV_OUT(vf[2]), PKV_OUT(vf[3]), PKV_OUT(vf[4]), PKV_OUT(vf[5]), PKV_OUT(vf[6])
-                 : PKV_IN(kb + ka[0]), PKV_IN(kb + ka[1]), PKV_IN(kb + ka[2]), PKV_IN(kb + ka[3]), PKV_IN(vb + va[0]),
-                   PKV_IN(vb + va[1]), PKV_IN(vb + va[2]), PKV_IN(vb + va[3]), PKV_IN(vb + va[4]), PKV_IN(vb + va[5]),
-                   PKV_IN(vb + va[6])
-                 : "memory");
-}
-template <>
-__device__ __forceinline__ void ring_read<4, 8>(uint32_t kb, const uint32_t (&ka)[4], uint32_t vb,
-                                                const uint32_t (&va)[8], u32x4 (&kf)[4], uint2 (&vf)[8]) {
-    asm volatile(PKV_RD_K(0, 12) PKV_RD_K(1, 13) PKV_RD_K(2, 14) PKV_RD_K(3, 15) PKV_RD_V(4, 16) PKV_RD_V(5, 17)
-                     PKV_RD_V(6, 18) PKV_RD_V(7, 19) PKV_RD_V(8, 20) PKV_RD_V(9, 21) PKV_RD_V(10, 22)
-                         PKV_RD_V(11, 23) "s_waitcnt lgkmcnt(0)"
-                 : PKV_OUT(kf[0]), PKV_OUT(kf[1]), PKV_OUT(kf[2]), PKV_OUT(kf[3]), PKV_OUT(vf[0]), PKV_OUT(vf[1]),
-                   PKV_OUT(vf[2]), PKV_OUT(vf[3]), PKV_OUT(vf[4]), PKV_OUT(vf[5]), PKV_OUT(vf[6]), PKV_OUT(vf[7])
-                 : PKV_IN(kb + ka[0]), PKV_IN(kb + ka[1]), PKV_IN(kb + ka[2]), PKV_IN(kb + ka[3]), PKV_IN(vb + va[0]),
-                   PKV_IN(vb + va[1]), PKV_IN(vb + va[2]), PKV_IN(vb + va[3]), PKV_IN(vb + va[4]), PKV_IN(vb + va[5]),
-                   PKV_IN(vb + va[6]), PKV_IN(vb + va[7])
-                 : "memory");
-}
-#undef PKV_RD_K
-#undef PKV_RD_V
-#undef PKV_OUT
-#undef PKV_IN
 
 // ------------------------------------------------------------------ wave scans (int)
 template <int CTRL>
@@ -303,22 +374,23 @@ __device__ __forceinline__ Pick pick_run(const AttnParams& p, int lane, int at, 
 }
 
 // LDS bytes of a workgroup (the ring; the merge's partials reuse it) and how many a CU holds.
-constexpr int ring_bytes(int D, int NW) { return NW * 2 * 2 * kUnit * D * 2; }
-constexpr int wgs_per_cu(int D, int NW) {
-    const int lds = (160 * 1024) / (ring_bytes(D, NW) + NW * 128 + 16), waves = 16 / NW;
+constexpr int wgs_per_cu(int row_bytes, int NW) {
+    const int ring = NW * 2 * 2 * kUnit * row_bytes;
+    const int lds = (160 * 1024) / (ring + NW * 128 + 16), waves = 16 / NW;
     const int n = lds < waves ? lds : waves;
     return n < 1 ? 0 : n;
 }
 
 template <typename T, int D, int NW>
 __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnParams p, int min_run, int slots) {
-    constexpr int ROWB = D * 2;               // bytes per (token, head) row
+    using C = Contract<T, D>;
+    constexpr int ISZ = (int)sizeof(T);
+    constexpr int ROWB = D * ISZ;             // bytes per (token, head) row
     constexpr int CPR = ROWB / 16;            // 16-byte chunks per row
     constexpr int IPB = (kUnit * CPR + 63) / 64;   // DMA instructions per unit, K or V
     constexpr bool kWhole = kUnit * CPR % 64 == 0;
     constexpr bool kHalf = 64 % CPR == 0 && 64 / CPR <= 8;   // one 8-row half per instruction
-    constexpr int KS = (D + 31) / 32;         // S^T MFMAs per unit
-    constexpr int VT = D / 16;                // P·V MFMAs per unit
+    constexpr int KS = C::KS, VT = C::VT;
     constexpr int NT = NW * 64;
     constexpr int UB = kUnit * ROWB;          // bytes of a unit, K or V
 
@@ -359,7 +431,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
     const int lg = lane >> 4;                 // MFMA lane group
     const int ln = lane & 15;                 // MFMA row / column index
 
-    // ---- Q^T B operand: lane (lg, ln) takes head ln, dims 32 j + 8 lg .. +8 (zero for the
+    // ---- Q^T B operand: lane (lg, ln) takes head ln, 16-byte pieces 4 j + lg (zero for the
     // padding heads and dims). Issued before the block ids, whose wait covers it.
     u32x4 qf[KS];
 #pragma unroll
@@ -367,7 +439,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
         qf[j] = u32x4{0u, 0u, 0u, 0u};
         if (ln < G && 4 * j + lg < CPR) {
             const Vec16 v = load16(reinterpret_cast<const char*>(p.q) +
-                                   ((int64_t)seq * p.q_st + (int64_t)(kvh * G + ln) * p.q_sh) * 2 + (4 * j + lg) * 16);
+                                   ((int64_t)seq * p.q_st + (int64_t)(kvh * G + ln) * p.q_sh) * ISZ + (4 * j + lg) * 16);
             qf[j] = u32x4{v.w[0], v.w[1], v.w[2], v.w[3]};
         }
     }
@@ -375,24 +447,25 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
     // ---- fused append: the new token is the context's last key. The wave whose units end
     // with it holds the row (lanes 0 .. CPR-1 K, CPR .. 2 CPR-1 V) and stores it at the end.
     const int new_row = p.app_slots && nu > 0 && u_first + (nu - 1) * NW == n_units - 1 ? (ctx - 1) % kUnit : -1;
-    const char* knew = reinterpret_cast<const char*>(p.app_k) + ((int64_t)seq * p.app_st + (int64_t)kvh * p.app_sh) * 2;
-    const char* vnew = reinterpret_cast<const char*>(p.app_v) + ((int64_t)seq * p.app_st + (int64_t)kvh * p.app_sh) * 2;
+    const char* knew = reinterpret_cast<const char*>(p.app_k) + ((int64_t)seq * p.app_st + (int64_t)kvh * p.app_sh) * ISZ;
+    const char* vnew = reinterpret_cast<const char*>(p.app_v) + ((int64_t)seq * p.app_st + (int64_t)kvh * p.app_sh) * ISZ;
     Vec16 new_piece = Vec16{{0u, 0u, 0u, 0u}};
     int64_t new_slot = -1;
+    static_assert(2 * CPR <= 64, "one piece per lane");
     if (new_row >= 0 && lane < 2 * CPR) {
         new_slot = p.app_slots[seq];
         new_piece = load16((lane < CPR ? knew : vnew) + (lane % CPR) * 16);
     }
 
-    const int64_t slot_bytes = p.ss * 2;
-    const int64_t block_bytes = p.sb * 2;
-    const char* kbase = reinterpret_cast<const char*>(p.k) + (int64_t)kvh * p.sh * 2;
-    const char* vbase = reinterpret_cast<const char*>(p.v) + (int64_t)kvh * p.sh * 2;
+    const int64_t slot_bytes = p.ss * ISZ;
+    const int64_t block_bytes = p.sb * ISZ;
+    const char* kbase = reinterpret_cast<const char*>(p.k) + (int64_t)kvh * p.sh * ISZ;
+    const char* vbase = reinterpret_cast<const char*>(p.v) + (int64_t)kvh * p.sh * ISZ;
     const int64_t* table = p.tables + (int64_t)seq * p.table_stride;
 
     // ---- DMA of a unit: row and swizzled source chunk of this lane's instruction j.
     auto dma_row = [&](int j) { return (64 * j + lane) / CPR; };
-    auto dma_chunk = [&](int j) { return (64 * j + lane) % CPR ^ unit_swizzle<D>((64 * j + lane) / CPR); };
+    auto dma_chunk = [&](int j) { return (64 * j + lane) % CPR ^ C::swizzle((64 * j + lane) / CPR); };
     uint32_t lane_off[IPB];                   // inside an 8-row half
 #pragma unroll
     for (int j = 0; j < IPB; ++j)
@@ -435,20 +508,8 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
         }
     };
 
-    // ---- per-lane operand addresses inside a unit: K row ln, logical chunk 4 j + lg (a
-    // chunk past head_dim re-reads another, zeroed below); V^T rows 4 lg + ln / 4, columns
-    // 16 t + 4 (ln % 4).
-    uint32_t k_addr[KS], v_addr[VT];
-#pragma unroll
-    for (int j = 0; j < KS; ++j) {
-        const int c = 4 * j + lg < CPR ? 4 * j + lg : 4 * j + (lg & 1);
-        k_addr[j] = (uint32_t)(ln * ROWB + ((c ^ unit_swizzle<D>(ln)) << 4));
-    }
-    const int v_row = 4 * lg + (ln >> 2);
-#pragma unroll
-    for (int t = 0; t < VT; ++t)
-        v_addr[t] = (uint32_t)(v_row * ROWB + (((2 * t + ((ln & 3) >> 1)) ^ unit_swizzle<D>(v_row)) << 4) + 8 * (ln & 1));
-
+    C unit;
+    unit.address(lg, ln);
     f32x4 o[VT];
 #pragma unroll
     for (int t = 0; t < VT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -471,24 +532,18 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
         if (k0 + 1 < k1) dma_unit(k0 + 1, offs, 1);
         for (int k = k0; k < k1; ++k) {
             const int slot = k & 1;
-            if (k + 1 < k1) __builtin_amdgcn_s_waitcnt(kWaitVm<kUnitDmas>);
-            else __builtin_amdgcn_s_waitcnt(kWaitVm<0>);
-            u32x4 kf[KS];
-            uint2 vf[VT];
-            ring_read<KS, VT>(lds_addr(s_ring[wave][slot][0]), k_addr, lds_addr(s_ring[wave][slot][1]), v_addr, kf, vf);
+            if (k + 1 < k1) wait_vm<kUnitDmas>();
+            else wait_vm<0>();
+            unit.read(s_ring[wave][slot][0], s_ring[wave][slot][1], lg);
             if (k + 2 < k1) dma_unit(k + 2, offs, slot);
-            if constexpr (D % 32 != 0)
-                if (lg >= 2) kf[KS - 1] = u32x4{0u, 0u, 0u, 0u};
 
             // S^T for the 16 keys: lane (lg, ln) holds keys 4 lg + r of head ln.
-            f32x4 st = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int j = 0; j < KS; ++j) st = SMfma<T>::qk(kf[j], qf[j], st);
+            f32x4 st = unit.scores(qf);
             const int valid = ctx - (u_first + k * NW) * kUnit;
             float bmax = kNegInf;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float x = SMfma<T>::round(SMfma<T>::round(st[r]) * scale) * kLog2e;
+                const float x = C::scaled(st[r], scale);
                 st[r] = 4 * lg + r < valid ? x : kNegInf;
                 bmax = fmaxf(bmax, st[r]);
             }
@@ -514,9 +569,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
                 pr[r] = fast_exp2(st[r] - m_off);
                 l_part += pr[r];
             }
-            const uint2 pb = make_uint2(SMfma<T>::pack(pr[0], pr[1]), SMfma<T>::pack(pr[2], pr[3]));
-#pragma unroll
-            for (int t = 0; t < VT; ++t) o[t] = SMfma<T>::pv(vf[t], pb, o[t]);
+            unit.accumulate(pr, o);
         }
     }
     if (new_row >= 0 && (uint64_t)new_slot < (uint64_t)(p.num_blocks << p.block_shift)) {
@@ -546,18 +599,11 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
 
     const int head0 = kvh * G;
     // Four consecutive elements per thread.
+    const bool wide =
+        (((uint64_t)(uintptr_t)p.out | (uint64_t)(p.out_st * ISZ) | (uint64_t)(p.out_sh * ISZ)) & (4 * ISZ - 1)) == 0;
     auto store_out = [&](int g, int d, float4 v) {
         T* orow = reinterpret_cast<T*>(p.out) + (int64_t)seq * p.out_st + (int64_t)(head0 + g) * p.out_sh + d;
-        const uint32_t w0 = SMfma<T>::pack(v.x, v.y), w1 = SMfma<T>::pack(v.z, v.w);
-        if ((((uint64_t)(uintptr_t)p.out | (uint64_t)(p.out_st * 2) | (uint64_t)(p.out_sh * 2)) & 7) == 0) {
-            *reinterpret_cast<uint2*>(orow) = make_uint2(w0, w1);
-        } else {
-            uint16_t* o16 = reinterpret_cast<uint16_t*>(orow);
-            o16[0] = (uint16_t)w0;
-            o16[1] = (uint16_t)(w0 >> 16);
-            o16[2] = (uint16_t)w1;
-            o16[3] = (uint16_t)(w1 >> 16);
-        }
+        C::store4(orow, v, wide);
     };
     for (int e = tid * 4; e < G * D; e += NT * 4) {
         const int g = e / D, d = e - g * D;
@@ -662,12 +708,16 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
 template <typename T, int D, int NW>
 int launch_nw(const AttnParams& p, hipStream_t stream) {
     const int64_t pairs = (int64_t)p.num_seqs * p.num_kv_heads;
-    int64_t fits = (int64_t)kCus * wgs_per_cu(D, NW);
+    int64_t fits = (int64_t)kCus * wgs_per_cu(D * (int)sizeof(T), NW);
     // Many pairs of long contexts: runs for two rounds, or the longest context would be
-    // walked whole (250 sequences of 512-8192 tokens, 8/2 heads, bf16: 219 -> 189 us); with
-    // less to read the second round's start and merges cost more than it evens out (64
-    // sequences of 16-2048, 12 heads of 64, fp16: 24 -> 25.5).
-    if (2 * pairs > fits && pairs * p.max_parts * kDecodePart * D * 4 > ((int64_t)1 << 30)) fits *= 2;
+    // walked whole (250 sequences of 512-8192 tokens, 8/2 heads, bf16: 219 -> 189 us; 60 of
+    // 16-2000, 12 heads of 64, fp32: 84 -> 72); with less to read the second round's start and
+    // merges cost more than it evens out (64 of 16-2048, 12 heads of 64, fp16: 24 -> 25.5;
+    // 120 of 1-1000, 32/8 heads, fp16: 49 -> 55).
+    const int64_t units = (int64_t)p.max_parts * (kDecodePart / kUnit);
+    if ((2 * pairs > fits && pairs * units * kUnit * D * 2 * (int64_t)sizeof(T) > ((int64_t)1 << 30)) ||
+        (pairs >= fits && units >= 24 * NW))
+        fits *= 2;
     // At least 4 units a wave and run (and a workspace slot's tokens); contexts of up to 8
     // units a wave are not worth the merge (12 layers of a GPT-2 decode step captured for
     // 1024 tokens, 8 sequences, fp16: 161.5 -> 158.2 us with the projections).
@@ -675,8 +725,8 @@ int launch_nw(const AttnParams& p, hipStream_t stream) {
     // No split either where the pairs fill the GPU by themselves, or where the counters or
     // the scan do not reach.
     int slots = 0;
-    if (p.max_parts * (kDecodePart / kUnit) > NW * 8 && p.ws_cnt && p.num_seqs <= kMaxScanSeqs && pairs < fits &&
-        (int64_t)p.num_seqs * p.max_parts * (kDecodePart / kUnit) < ((int64_t)1 << 31))
+    if (units > NW * 8 && p.ws_cnt && p.num_seqs <= kMaxScanSeqs && pairs < fits &&
+        p.num_seqs * units < ((int64_t)1 << 31))
         slots = (int)(fits / p.num_kv_heads);
     const int64_t grid = slots > 0 ? (int64_t)(slots > p.num_seqs ? slots : p.num_seqs) * p.num_kv_heads : pairs;
     if (grid > 0x7fffffff) return PKV_EUNSUPPORTED;
@@ -687,13 +737,19 @@ int launch_nw(const AttnParams& p, hipStream_t stream) {
 // Waves per workgroup: 8 while the pairs fit the GPU so (each context is walked by more
 // waves: fewer splits, shorter chains), else 4. Measured, us a call, 8 vs 4 waves: 8
 // sequences of 1-8k, 32/8 heads of 128, bf16 35.3 vs 37.5; 30 x 4096 82 vs 88; 64 sequences
-// of 16-2048, 12 heads of 64, fp16 (768 pairs, more than fit) 25.2 vs 21.9; 1000 of 1-60
-// (8000 pairs) 120 vs 70. 16 waves were never better than 8 by more than the noise, but
+// of 16-2048, 12 heads of 64, fp16 (768 pairs, more than fit) 25.2 vs 21.9. 2 where there
+// are many rounds of pairs, whose starts and merges then overlap (4 vs 2 waves): 1000 of 1-60,
+// 32/8 heads, bf16 69.8 vs 42.6; 300 of 1-120 26.9 vs 20.4; 400 of 1-60, 12 heads of 64 22.0
+// vs 16.9; 200 of 1-100 (2.3 rounds) 16.2 vs 16.4;
+// 128 of 512-4096, 32/8 heads of 128, fp32 418 vs 483: short contexts only. 16 waves were never better than 8 by more than the noise, but
 // for 500 single-head sequences of 16-4000 (51 vs 58).
 template <typename T, int D>
 int launch_d(const AttnParams& p, hipStream_t stream) {
     const int64_t pairs = (int64_t)p.num_seqs * p.num_kv_heads;
-    if (pairs <= (int64_t)kCus * wgs_per_cu(D, 8)) return launch_nw<T, D, 8>(p, stream);
+    if constexpr (wgs_per_cu(D * (int)sizeof(T), 8) > 0)
+        if (pairs <= (int64_t)kCus * wgs_per_cu(D * (int)sizeof(T), 8)) return launch_nw<T, D, 8>(p, stream);
+    if (pairs >= 4ll * kCus * wgs_per_cu(D * (int)sizeof(T), 4) && p.max_parts * (kDecodePart / kUnit) <= 32)
+        return launch_nw<T, D, 2>(p, stream);
     return launch_nw<T, D, 4>(p, stream);
 }
 
@@ -714,7 +770,7 @@ int launch_t(const AttnParams& p, hipStream_t stream) {
 }  // namespace
 
 bool decode_split_applies(const AttnParams& p, int dtype) {
-    if (dtype != PKV_FLOAT16 && dtype != PKV_BFLOAT16) return false;
+    const int isz = dtype == PKV_FLOAT32 ? 4 : 2;
     if (p.num_blocks < 1 || p.block_shift < 3 || p.group > 16) return false;
     if (p.head_dim % 16 || p.head_dim < 32 || p.head_dim > 128) return false;
     if ((int64_t)p.num_seqs * p.num_kv_heads > 0x7fffffff) return false;
@@ -722,20 +778,21 @@ bool decode_split_applies(const AttnParams& p, int dtype) {
     // Units of a sequence are exact in fp32 (the run search divides in it).
     if ((int64_t)p.max_parts * kDecodePart >= ((int64_t)1 << 28)) return false;
     // Offsets inside an 8-row half in 32 bits.
-    if (8 * p.ss * 2 + p.head_dim * 2 > 0xffffffffll || p.ss < 0) return false;
+    if (8 * p.ss * isz + p.head_dim * isz > 0xffffffffll || p.ss < 0) return false;
     // 16-byte rows, those of a fused append among them.
     uint64_t probe = (uint64_t)(uintptr_t)p.q | (uint64_t)(uintptr_t)p.k | (uint64_t)(uintptr_t)p.v |
-                     (uint64_t)(p.q_st * 2) | (uint64_t)(p.q_sh * 2) | (uint64_t)(p.sb * 2) |
-                     (uint64_t)(p.ss * 2) | (uint64_t)(p.sh * 2);
+                     (uint64_t)(p.q_st * isz) | (uint64_t)(p.q_sh * isz) | (uint64_t)(p.sb * isz) |
+                     (uint64_t)(p.ss * isz) | (uint64_t)(p.sh * isz);
     if (p.app_slots)
-        probe |= (uint64_t)(uintptr_t)p.app_k | (uint64_t)(uintptr_t)p.app_v | (uint64_t)(p.app_st * 2) |
-                 (uint64_t)(p.app_sh * 2);
+        probe |= (uint64_t)(uintptr_t)p.app_k | (uint64_t)(uintptr_t)p.app_v | (uint64_t)(p.app_st * isz) |
+                 (uint64_t)(p.app_sh * isz);
     return probe % 16 == 0;
 }
 
 int launch_decode_split(const AttnParams& p, int dtype, hipStream_t stream) {
     if (!decode_split_applies(p, dtype)) return PKV_EUNSUPPORTED;
     if (p.num_seqs == 0) return PKV_OK;
+    if (dtype == PKV_FLOAT32) return launch_t<float>(p, stream);
     return dtype == PKV_FLOAT16 ? launch_t<_Float16>(p, stream) : launch_t<bf16_t>(p, stream);
 }
 

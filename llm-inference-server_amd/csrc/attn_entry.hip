@@ -167,6 +167,7 @@ int decode_impl(void* out, int64_t out_stride_t, int64_t out_stride_h, const voi
         p.ws_o = (float*)((char*)workspace + w.cnt_bytes + w.mfma_pfx_bytes + w.mfma_ml_bytes);
     }
 
+    const bool f32_regs = dtype == PKV_FLOAT32 && decode_f32_applies(p);
     auto append_first = [&]() -> int {
         p.app_k = p.app_v = nullptr;
         p.app_slots = nullptr;
@@ -180,12 +181,12 @@ int decode_impl(void* out, int64_t out_stride_t, int64_t out_stride_h, const voi
         p.app_st = app->st;
         p.app_sh = app->sh;
         p.app_slots = app->slots;
-        // The MFMA kernels write the rows themselves: the persistent one by 4-byte copies
+        // The fp32 register kernel reads the pool only. The MFMA kernels write the rows themselves: the persistent one by 4-byte copies
         // (even strides, 4-byte aligned sources), the others from 16-byte rows. Any other
         // kernel gets the append launch first.
         const bool fuse = mfma ? app->st % 2 == 0 && app->sh % 2 == 0 &&
                                      ((uintptr_t)app->k_new | (uintptr_t)app->v_new) % 4 == 0
-                               : decode_split_applies(p, dtype) || prefill_tuned(p, dtype);
+                               : !f32_regs && (decode_split_applies(p, dtype) || prefill_tuned(p, dtype));
         if (!fuse && (rc = append_first())) return rc;
     }
     if (mfma) {
@@ -200,7 +201,8 @@ int decode_impl(void* out, int64_t out_stride_t, int64_t out_stride_h, const voi
         if (p.app_slots && !decode_split_applies(p, dtype) && !prefill_tuned(p, dtype) && (rc = append_first()))
             return rc;
     }
-    rc = dtype == PKV_FLOAT32 ? launch_decode_attention(p, stream) : launch_decode_split(p, dtype, stream);
+    if (f32_regs) return launch_decode_f32(p, stream);
+    rc = launch_decode_split(p, dtype, stream);
     if (rc != PKV_EUNSUPPORTED) return rc;
     clear_error();
     // Groups of more than 16 heads run as one-token prompts on the prefill MFMA kernel, their
@@ -219,10 +221,6 @@ int decode_impl(void* out, int64_t out_stride_t, int64_t out_stride_h, const voi
         p.splits = 1;                              // the split grid is too large: unsplit
         p.split_tiles = 0x7fffffff;
         return launch_prefill_attention(p, dtype, stream);
-    }
-    if (dtype == PKV_FLOAT32) {
-        rc = launch_f32_attention(p, stream);
-        if (rc != PKV_EUNSUPPORTED) return rc;
     }
     return launch_generic_attention(p, dtype, stream);
 }

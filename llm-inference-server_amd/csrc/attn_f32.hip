@@ -1,7 +1,6 @@
 // fp32 paged attention on 16-key tiles (one block each) over a float32 pool with block
-// size 16 and head_dim 64 or 128: decode batches at head_dim 128, prefill-entry batches
-// of 1-token rows, and prefill batches the fp32 MFMA kernel (attn_prefill_f32.hip)
-// declines. Replaces, for float32 pools, the reference's ragged loop and batched decode
+// size 16 and head_dim 64 or 128: prefill-entry batches of 1-token rows, and prefill
+// batches the fp32 MFMA kernel (attn_prefill_f32.hip) declines. Replaces, for float32 pools, the reference's ragged loop and batched decode
 // (inference_server/core/attention.py:130-187) where the only other kernel walks the
 // keys one at a time.
 //
@@ -69,8 +68,8 @@ __global__ __launch_bounds__(64) void paged_f32_kernel(const AttnParams p) {
     const int lane = lane_id();
     const int kvh = (int)blockIdx.y;
     const int seq = (int)blockIdx.z;
-    const int64_t q_first = p.qsl ? p.qsl[seq] : (int64_t)seq;
-    const int q_len = p.qsl ? (int)(p.qsl[seq + 1] - q_first) : 1;
+    const int64_t q_first = p.qsl[seq];
+    const int q_len = (int)(p.qsl[seq + 1] - q_first);
     const int t0 = (int)blockIdx.x * TPW;   // the wave's first query token (index within the sequence)
     if (t0 >= q_len) return;
     int64_t ctx = p.ctx_lens[seq];
@@ -234,9 +233,8 @@ int launch_dg(const AttnParams& p, hipStream_t stream) {
     constexpr int L1 = D / 16, L2 = D / 4;
     constexpr int T1 = 64 / L1 / G;
     constexpr int T2 = (64 / L2) / G;  // 0 when the group exceeds the narrow shape's slots
-    const int64_t mq = p.qsl ? p.max_query_len : 1;
-    const int64_t tokens = p.qsl ? p.num_tokens : p.num_seqs;
-    const int64_t waves = (tokens / T1 + p.num_seqs) * (int64_t)p.num_kv_heads;
+    const int64_t mq = p.max_query_len;
+    const int64_t waves = (p.num_tokens / T1 + p.num_seqs) * (int64_t)p.num_kv_heads;
     const int max_q = (int)(mq > 0 ? mq : 1);
     if constexpr (T2 >= 1) {
         if (T1 > mq || waves < 1024) return launch_one<D, L2, G>(p, max_q, stream);
@@ -269,7 +267,8 @@ int launch_f32_attention(const AttnParams& p, hipStream_t stream) {
     if (probe % 16) return PKV_EUNSUPPORTED;
     // Byte offsets inside a block fit the 32-bit-friendly range the DMA offsets assume.
     if ((int64_t)kTile * p.ss * 4 > 0x7fffffff) return PKV_EUNSUPPORTED;
-    if (p.num_seqs == 0 || (p.qsl && p.num_tokens == 0)) return PKV_OK;
+    if (!p.qsl) return PKV_EUNSUPPORTED;
+    if (p.num_seqs == 0 || p.num_tokens == 0) return PKV_OK;
     return p.head_dim == 64 ? launch_d<64>(p, stream) : launch_d<128>(p, stream);
 }
 

@@ -1,5 +1,5 @@
 """The one-launch MFMA decode kernel (csrc/attn_decode_split.hip) against oracle.gather at the
-16-bit bar of 2e-2: head_dims, groups, block sizes, contexts around the edges of a unit (16
+bars of 2e-2 in 16 bits and 1e-5 in fp32: head_dims, groups, block sizes, contexts around the edges of a unit (16
 keys), a wave's round (4 or 8 units) and a run, sequence counts around the 64 lanes and 16
 sequences per lane of its run search, runs longer than the 32 units whose block ids a wave
 holds, and the fused append. Pool rows no key may come from are NaN.
@@ -15,7 +15,7 @@ from inference_server.core.attention_hip import paged_attention_hip_launch
 from oracle.gather import paged_attention_gather as oracle_gather
 
 pytestmark = pytest.mark.gpu
-TOL = 2e-2
+TOL = {torch.float16: 2e-2, torch.bfloat16: 2e-2, torch.float32: 1e-5}
 
 
 def _batch(ctx, *, dtype, d, bs, kv, group, seed=0):
@@ -55,7 +55,7 @@ def _run(b, *, fused):
     if fused:
         k.view(-1, *k.shape[2:])[slots] = b["k_new"]
         v.view(-1, *v.shape[2:])[slots] = b["v_new"]
-    bits = lambda t: t.cpu().view(torch.int16)  # noqa: E731
+    bits = lambda t: t.cpu().view(torch.int32 if t.dtype == torch.float32 else torch.int16)  # noqa: E731
     assert torch.equal(bits(kd), bits(k)) and torch.equal(bits(vd), bits(v))
     assert torch.equal(bits(outs[0]), bits(outs[1]))        # and the merge counters were left zero
     return outs[0].cpu(), k, v, slots
@@ -67,7 +67,7 @@ def _check(b, *, fused, rows=None):
     clean = lambda t: torch.nan_to_num(t)  # noqa: E731  (never read: the oracle masks, 0 x NaN is NaN)
     ref = oracle_gather(b["q"][rows], clean(k), clean(v), b["tables"][rows], b["ctx"][rows],
                         torch.ones(len(rows), dtype=torch.long), b["q"].shape[2] ** -0.5)
-    torch.testing.assert_close(out[rows], ref, atol=TOL, rtol=TOL)
+    torch.testing.assert_close(out[rows], ref, atol=TOL[out.dtype], rtol=TOL[out.dtype])
 
 
 EDGES = [1, 7, 8, 9, 15, 16, 17, 63, 64, 65, 127, 129, 512, 513]
@@ -77,28 +77,32 @@ EDGES = [1, 7, 8, 9, 15, 16, 17, 63, 64, 65, 127, 129, 512, 513]
     (32, 8, 2, 16, torch.float16), (32, 16, 3, 1, torch.bfloat16), (48, 16, 1, 5, torch.bfloat16),
     (64, 16, 12, 1, torch.float16), (64, 32, 3, 7, torch.bfloat16), (80, 8, 2, 2, torch.float16),
     (80, 16, 1, 12, torch.bfloat16), (96, 64, 2, 3, torch.float16), (112, 16, 1, 4, torch.bfloat16),
-    (128, 16, 8, 4, torch.bfloat16), (128, 8, 1, 8, torch.float16), (128, 128, 2, 9, torch.float16)])
+    (128, 16, 8, 4, torch.bfloat16), (128, 8, 1, 8, torch.float16), (128, 128, 2, 9, torch.float16),
+    (32, 8, 2, 3, torch.float32), (48, 32, 1, 16, torch.float32), (64, 16, 12, 1, torch.float32),
+    (80, 8, 2, 2, torch.float32), (112, 16, 1, 5, torch.float32), (128, 16, 2, 4, torch.float32)])
 @pytest.mark.parametrize("fused", [False, True], ids=["plain", "append"])
 def test_shapes_and_context_edges(d, bs, kv, group, dtype, fused):
     _check(_batch(EDGES, dtype=dtype, d=d, bs=bs, kv=kv, group=group, seed=d + bs), fused=fused)
 
 
-@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 130, 300])
+@pytest.mark.parametrize("n,dtype", [(n, torch.bfloat16) for n in (1, 2, 63, 64, 65, 130, 300)]
+                         + [(n, torch.float32) for n in (2, 66)])
 @pytest.mark.parametrize("fused", [False, True], ids=["plain", "append"])
-def test_run_search_over_sequence_counts(n, fused):
+def test_run_search_over_sequence_counts(n, dtype, fused):
     """Long contexts among short ones, so that runs are cut and found across lanes."""
     ctx = [5 + (37 * i) % 150 for i in range(n)]
     for i, c in ((0, 3000), (n // 2, 1900), (n - 1, 4099)):
         ctx[i] = c
     rows = sorted({0, n // 2, n - 1, n // 3, max(0, n - 2)})
-    _check(_batch(ctx, dtype=torch.bfloat16, d=64, bs=16, kv=1, group=4, seed=n), fused=fused, rows=rows)
+    _check(_batch(ctx, dtype=dtype, d=64, bs=16, kv=1, group=4, seed=n), fused=fused, rows=rows)
 
 
 @pytest.mark.parametrize("n,kv,d,long", [
     (350, 3, 32, 2200),      # as many pairs as the GPU holds: unsplit, 34 units a wave
     (1030, 1, 64, 300),      # more sequences than the search takes
+    (700, 6, 64, 90),        # many rounds of pairs: two waves a workgroup
     (40, 3, 128, 9000)],     # runs of several chunks of block ids
-    ids=["unsplit", "many", "long"])
+    ids=["unsplit", "many", "rounds", "long"])
 def test_unsplit_and_long_runs(n, kv, d, long):
     ctx = [1 + (29 * i) % 70 for i in range(n)]
     ctx[1], ctx[n // 2], ctx[n - 1] = long, long - 7, long + 13
