@@ -59,6 +59,12 @@ struct AttnParams {
 // p.app_* set: including the fused append, whose source rows must be 16-byte aligned).
 bool decode_split_applies(const AttnParams& p, int dtype);
 int launch_decode_split(const AttnParams& p, int dtype, hipStream_t stream);
+// The same kernel on fp32 prompts (p.qsl set, no fused append, p.max_parts sized for the
+// table): 16 query rows a workgroup.
+bool prompt_split_f32_applies(const AttnParams& p);
+int launch_prompt_split_f32(const AttnParams& p, hipStream_t stream);
+// Whether the batch's row tiles make at most two and a quarter rounds of the GPU there.
+bool prompt_split_f32_few(const AttnParams& p);
 // fp32 register kernel (attn_decode.hip): the shapes and sizes where it beats the kernel
 // above; it appends nothing itself.
 bool decode_f32_applies(const AttnParams& p);

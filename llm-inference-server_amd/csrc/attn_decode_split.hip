@@ -24,6 +24,10 @@
 //    accumulator into O^T += V^T P^T on 16x16x16, V^T by the transposing LDS read. 12 MFMAs
 //    and ~80 VALU instructions per unit at head_dim 128, where v_dot2 arithmetic took ~900.
 //    fp32 on 16x16x4.
+//  * fp32 prompts of few query rows, or of shapes without another kernel, take the same
+//    kernel with 16 (token, head) rows in place of one token's heads. us a call with the
+//    append: 8 prompts of 1-150 tokens behind up to 1,000, 12/4 heads of 80, block size 32,
+//    1,000 -> 44; 16 of 1-200 behind up to 1,500, 24/8 heads of 32, block size 8, 3,295 -> 73.
 //  * Merge: the waves' partials meet in LDS; split contexts leave fp32 partials that the
 //    last workgroup of each (sequence, KV head) to finish merges in run order (agent-scope
 //    stores, one counter, no workgroup ever waits for another).
@@ -373,6 +377,39 @@ __device__ __forceinline__ Pick pick_run(const AttnParams& p, int lane, int at, 
     }
 }
 
+// Prompts: the `at`-th tile of 16 query rows of one KV head's batch, numbered sequence by
+// sequence; seq < 0: none. Same lanes as above.
+struct PickTile {
+    int seq, q_len, tile;
+    int64_t q_first;
+};
+template <int PER>
+__device__ __forceinline__ PickTile pick_tile(const AttnParams& p, int lane, int at) {
+    int n_of[PER], ql[PER], mine = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int s = lane * PER + i;
+        ql[i] = s < p.num_seqs ? (int)(p.qsl[s + 1] - p.qsl[s]) : 0;
+        n_of[i] = ql[i] > 0 ? (int)(((uint32_t)ql[i] * (uint32_t)p.group + kUnit - 1) / kUnit) : 0;
+        mine += n_of[i];
+    }
+    const int incl = wave_scan(mine, lane);
+    const uint64_t found = __builtin_amdgcn_ballot_w64(at < incl);
+    PickTile r{-1, 0, 0, 0};
+    if (!found) return r;
+    const int src = __builtin_ctzll(found);
+    int left = at - (__builtin_amdgcn_readlane(incl, src) - __builtin_amdgcn_readlane(mine, src));
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        if (r.seq < 0) {
+            const int n = __builtin_amdgcn_readlane(n_of[i], src);
+            if (left < n) r = PickTile{src * PER + i, __builtin_amdgcn_readlane(ql[i], src), left, 0};
+            else left -= n;
+        }
+    if (r.seq >= 0) r.q_first = p.qsl[r.seq];
+    return r;
+}
+
 // LDS bytes of a workgroup (the ring; the merge's partials reuse it) and how many a CU holds.
 constexpr int wgs_per_cu(int row_bytes, int NW) {
     const int ring = NW * 2 * 2 * kUnit * row_bytes;
@@ -381,7 +418,10 @@ constexpr int wgs_per_cu(int row_bytes, int NW) {
     return n < 1 ? 0 : n;
 }
 
-template <typename T, int D, int NW>
+// PROMPT: the 16 rows are (token, head) pairs of a prompt, row f of a sequence being token
+// f / G, head f % G, each with its own causal bound; no split and no append. Else they are
+// the G heads of a sequence's one token.
+template <typename T, int D, int NW, bool PROMPT>
 __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnParams p, int min_run, int slots) {
     using C = Contract<T, D>;
     constexpr int ISZ = (int)sizeof(T);
@@ -407,7 +447,20 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
 
     // ---- this workgroup's (sequence, run)
     int seq, ctx, split = 0, n_splits = 1;
-    if (slots == 0) {                         // one workgroup per (sequence, KV head)
+    int rows = G, row0 = 0, pos0 = 0;         // query rows, the first one's number, token 0's position
+    int64_t q_first = 0;
+    if constexpr (PROMPT) {
+        const PickTile pick = p.num_seqs <= 64 ? pick_tile<1>(p, lane, at) : pick_tile<kScanPer>(p, lane, at);
+        if (pick.seq < 0) return;
+        seq = pick.seq;
+        q_first = pick.q_first;
+        row0 = pick.tile * kUnit;
+        rows = pick.q_len * G - row0 < kUnit ? pick.q_len * G - row0 : kUnit;
+        pos0 = __builtin_amdgcn_readfirstlane(decode_ctx(p, seq)) - pick.q_len;
+        // Keys visible to the tile's last token.
+        ctx = pos0 + (int)((uint32_t)(row0 + rows - 1) / (uint32_t)G) + 1;
+        if (ctx <= 0) return;
+    } else if (slots == 0) {                         // one workgroup per (sequence, KV head)
         seq = at;
         ctx = __builtin_amdgcn_readfirstlane(decode_ctx(p, seq));
         if (ctx == 0) return;
@@ -430,6 +483,11 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
 
     const int lg = lane >> 4;                 // MFMA lane group
     const int ln = lane & 15;                 // MFMA row / column index
+    // Token and head (of the KV head's group) of query row r, and this lane's last key + 1.
+    auto row_token = [&](int r) { return PROMPT ? (int)((uint32_t)(row0 + r) / (uint32_t)G) : 0; };
+    auto row_head = [&](int r) { return PROMPT ? row0 + r - row_token(r) * G : r; };
+    auto q_row = [&](int r) { return PROMPT ? q_first + row_token(r) : (int64_t)seq; };
+    const int my_keys = PROMPT ? pos0 + row_token(ln) + 1 : ctx;
 
     // ---- Q^T B operand: lane (lg, ln) takes head ln, 16-byte pieces 4 j + lg (zero for the
     // padding heads and dims). Issued before the block ids, whose wait covers it.
@@ -437,16 +495,17 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
 #pragma unroll
     for (int j = 0; j < KS; ++j) {
         qf[j] = u32x4{0u, 0u, 0u, 0u};
-        if (ln < G && 4 * j + lg < CPR) {
+        if (ln < rows && 4 * j + lg < CPR) {
             const Vec16 v = load16(reinterpret_cast<const char*>(p.q) +
-                                   ((int64_t)seq * p.q_st + (int64_t)(kvh * G + ln) * p.q_sh) * ISZ + (4 * j + lg) * 16);
+                                   (q_row(ln) * p.q_st + (int64_t)(kvh * G + row_head(ln)) * p.q_sh) * ISZ +
+                                   (4 * j + lg) * 16);
             qf[j] = u32x4{v.w[0], v.w[1], v.w[2], v.w[3]};
         }
     }
 
     // ---- fused append: the new token is the context's last key. The wave whose units end
     // with it holds the row (lanes 0 .. CPR-1 K, CPR .. 2 CPR-1 V) and stores it at the end.
-    const int new_row = p.app_slots && nu > 0 && u_first + (nu - 1) * NW == n_units - 1 ? (ctx - 1) % kUnit : -1;
+    const int new_row = !PROMPT && p.app_slots && nu > 0 && u_first + (nu - 1) * NW == n_units - 1 ? (ctx - 1) % kUnit : -1;
     const char* knew = reinterpret_cast<const char*>(p.app_k) + ((int64_t)seq * p.app_st + (int64_t)kvh * p.app_sh) * ISZ;
     const char* vnew = reinterpret_cast<const char*>(p.app_v) + ((int64_t)seq * p.app_st + (int64_t)kvh * p.app_sh) * ISZ;
     Vec16 new_piece = Vec16{{0u, 0u, 0u, 0u}};
@@ -539,7 +598,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
 
             // S^T for the 16 keys: lane (lg, ln) holds keys 4 lg + r of head ln.
             f32x4 st = unit.scores(qf);
-            const int valid = ctx - (u_first + k * NW) * kUnit;
+            const int valid = my_keys - (u_first + k * NW) * kUnit;
             float bmax = kNegInf;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -586,7 +645,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
         l_part = sp.a + sp.b;
     }
     float* w_acc = reinterpret_cast<float*>(s_ring[wave]);   // [G][D]
-    if (ln < G) {
+    if (ln < rows) {
 #pragma unroll
         for (int t = 0; t < VT; ++t)
             *reinterpret_cast<float4*>(w_acc + ln * D + 16 * t + 4 * lg) = make_float4(o[t][0], o[t][1], o[t][2], o[t][3]);
@@ -602,10 +661,10 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
     const bool wide =
         (((uint64_t)(uintptr_t)p.out | (uint64_t)(p.out_st * ISZ) | (uint64_t)(p.out_sh * ISZ)) & (4 * ISZ - 1)) == 0;
     auto store_out = [&](int g, int d, float4 v) {
-        T* orow = reinterpret_cast<T*>(p.out) + (int64_t)seq * p.out_st + (int64_t)(head0 + g) * p.out_sh + d;
+        T* orow = reinterpret_cast<T*>(p.out) + q_row(g) * p.out_st + (int64_t)(head0 + row_head(g)) * p.out_sh + d;
         C::store4(orow, v, wide);
     };
-    for (int e = tid * 4; e < G * D; e += NT * 4) {
+    for (int e = tid * 4; e < rows * D; e += NT * 4) {
         const int g = e / D, d = e - g * D;
         float M = kNegInf;
 #pragma unroll
@@ -623,7 +682,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
             acc.z += sc * v.z;
             acc.w += sc * v.w;
         }
-        if (n_splits == 1) {
+        if (PROMPT || n_splits == 1) {
             const float inv = 1.f / L;
             store_out(g, d, make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv));
         } else {
@@ -642,7 +701,7 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
             }
         }
     }
-    if (n_splits == 1) return;
+    if (PROMPT || n_splits == 1) return;
 
     // ---- the last workgroup of the (sequence, KV head) to get here merges its runs, in run
     // order, and returns the counter to zero for the next call. The partial stores above are
@@ -730,7 +789,7 @@ int launch_nw(const AttnParams& p, hipStream_t stream) {
         slots = (int)(fits / p.num_kv_heads);
     const int64_t grid = slots > 0 ? (int64_t)(slots > p.num_seqs ? slots : p.num_seqs) * p.num_kv_heads : pairs;
     if (grid > 0x7fffffff) return PKV_EUNSUPPORTED;
-    paged_decode_split_kernel<T, D, NW><<<dim3((unsigned)grid), NW * 64, 0, stream>>>(p, min_run, slots);
+    paged_decode_split_kernel<T, D, NW, false><<<dim3((unsigned)grid), NW * 64, 0, stream>>>(p, min_run, slots);
     return check_launch("paged decode attention (split)");
 }
 
@@ -767,14 +826,23 @@ int launch_t(const AttnParams& p, hipStream_t stream) {
     return PKV_EUNSUPPORTED;
 }
 
+// Row tiles of one KV head's batch at most (a sequence's last tile may be partial).
+int64_t prompt_tiles(const AttnParams& p) { return p.num_tokens * p.group / kUnit + p.num_seqs; }
+
+template <int D>
+int launch_prompt(const AttnParams& p, hipStream_t stream) {
+    const unsigned grid = (unsigned)(prompt_tiles(p) * p.num_kv_heads);
+    paged_decode_split_kernel<float, D, 4, true><<<dim3(grid), 256, 0, stream>>>(p, 0, 0);
+    return check_launch("paged prompt attention (split)");
+}
+
 }  // namespace
 
-bool decode_split_applies(const AttnParams& p, int dtype) {
+// What both forms of the kernel ask of a batch.
+static bool split_shape(const AttnParams& p, int dtype) {
     const int isz = dtype == PKV_FLOAT32 ? 4 : 2;
-    if (p.num_blocks < 1 || p.block_shift < 3 || p.group > 16) return false;
+    if (p.num_blocks < 1 || p.block_shift < 3) return false;
     if (p.head_dim % 16 || p.head_dim < 32 || p.head_dim > 128) return false;
-    if ((int64_t)p.num_seqs * p.num_kv_heads > 0x7fffffff) return false;
-    if (p.max_parts > 1 && (!p.ws_o || !p.ws_ml)) return false;
     // Units of a sequence are exact in fp32 (the run search divides in it).
     if ((int64_t)p.max_parts * kDecodePart >= ((int64_t)1 << 28)) return false;
     // Offsets inside an 8-row half in 32 bits.
@@ -787,6 +855,38 @@ bool decode_split_applies(const AttnParams& p, int dtype) {
         probe |= (uint64_t)(uintptr_t)p.app_k | (uint64_t)(uintptr_t)p.app_v | (uint64_t)(p.app_st * isz) |
                  (uint64_t)(p.app_sh * isz);
     return probe % 16 == 0;
+}
+
+bool decode_split_applies(const AttnParams& p, int dtype) {
+    if (p.group > 16 || (int64_t)p.num_seqs * p.num_kv_heads > 0x7fffffff) return false;
+    if (p.max_parts > 1 && (!p.ws_o || !p.ws_ml)) return false;
+    return split_shape(p, dtype);
+}
+
+bool prompt_split_f32_applies(const AttnParams& p) {
+    if (!p.qsl || p.app_slots || p.num_seqs > kMaxScanSeqs) return false;
+    if (((int64_t)p.num_tokens + kUnit) * p.group > 0x7fffffff || prompt_tiles(p) * p.num_kv_heads > 0x7fffffff)
+        return false;
+    return split_shape(p, PKV_FLOAT32);
+}
+
+bool prompt_split_f32_few(const AttnParams& p) {
+    const int per_cu = (160 * 1024) / (4 * 2 * 2 * kUnit * p.head_dim * 4 + 4 * 128 + 16);
+    return p.num_tokens * p.num_heads / kUnit * 4 <= 9ll * kCus * (per_cu < 4 ? per_cu : 4);
+}
+
+int launch_prompt_split_f32(const AttnParams& p, hipStream_t stream) {
+    if (!prompt_split_f32_applies(p)) return PKV_EUNSUPPORTED;
+    switch (p.head_dim) {
+        case 32: return launch_prompt<32>(p, stream);
+        case 48: return launch_prompt<48>(p, stream);
+        case 64: return launch_prompt<64>(p, stream);
+        case 80: return launch_prompt<80>(p, stream);
+        case 96: return launch_prompt<96>(p, stream);
+        case 112: return launch_prompt<112>(p, stream);
+        case 128: return launch_prompt<128>(p, stream);
+    }
+    return PKV_EUNSUPPORTED;
 }
 
 int launch_decode_split(const AttnParams& p, int dtype, hipStream_t stream) {

@@ -395,8 +395,27 @@ int prefill_impl(void* out, int64_t out_stride_t, int64_t out_stride_h, const vo
         if (rc) return rc;
     }
     if (dtype == PKV_FLOAT32) {
-        rc = launch_prefill_f32_mfma(p, stream);
+        // Context clamp of the kernel below: the table row.
+        p.max_parts = (int)(ceil_div(table_width * block_size, kDecodePart) < 0x7fffffff
+                                ? ceil_div(table_width * block_size, kDecodePart)
+                                : 0x7fffffff);
+        // Few row tiles (each walked by four waves) go to the 16-row kernel, many to the
+        // 128-row one, and shapes that one does not take back to the first. Measured, us a
+        // call with the append, 16-row first: GPT-2 shape, 2 x 250 tokens 20.7 vs 28.9, 8 of
+        // 60-244 (1,022 tiles, two rounds of the GPU) 28.6 vs 30.6, 4 x 500 (1,500) 52.0 vs 50.7;
+        // 32/8 heads of 128, 8 of 1-30 behind 500-2000 69 vs 256, 2 x 200 (800 tiles, three
+        // rounds) 40.6 vs 39.5, 4 x 300 behind 2000 662 vs 570.
+        const bool few = prompt_split_f32_few(p);
+        if (!few) {
+            rc = launch_prefill_f32_mfma(p, stream);
+            if (rc != PKV_EUNSUPPORTED) return rc;
+        }
+        rc = launch_prompt_split_f32(p, stream);
         if (rc != PKV_EUNSUPPORTED) return rc;
+        if (few) {
+            rc = launch_prefill_f32_mfma(p, stream);
+            if (rc != PKV_EUNSUPPORTED) return rc;
+        }
         rc = launch_f32_attention(p, stream);
         if (rc != PKV_EUNSUPPORTED) return rc;
     }

@@ -1,5 +1,6 @@
 """The 16-bit prefill kernel on the shapes, groups and block sizes it takes, and its split
-contexts, against oracle.gather (the reference gather path) at the 16-bit bar of 2e-2.
+contexts, and fp32 prompts of the same shapes (16 rows a workgroup), against oracle.gather
+(the reference gather path) at the bars of 2e-2 in 16 bits and 1e-5 in fp32.
 
 Contexts end on, before and behind the edges of a block, an 8-key half, a 64-key tile, a
 32-row wave and a 128-row workgroup (query rows are tokens x group heads). Decode batches
@@ -18,7 +19,7 @@ from inference_server.core.attention_hip import attach_host, paged_attention_hip
 from oracle.gather import paged_attention_gather as oracle_gather
 from oracle.kvops import kv_append
 
-TOL = 2e-2
+TOL = {torch.float16: 2e-2, torch.bfloat16: 2e-2, torch.float32: 1e-5}
 EDGES = [(1, 1), (7, 7), (8, 8), (9, 5), (64, 1), (63, 63), (65, 65), (130, 43), (300, 129), (257, 1)]
 DECODE = [(1, 1), (8, 1), (9, 1), (64, 1), (65, 1), (700, 1)]
 #: One prompt of a few tiles among contexts long enough to be split.
@@ -57,13 +58,14 @@ def _check(b, *, fused, told=None):
     torch.cuda.synchronize()
     kr, vr = b["k"], b["v"]
     if fused:
-        bits = lambda t: t.view(torch.int16).numpy()  # noqa: E731
+        raw = torch.int32 if kr.dtype == torch.float32 else torch.int16
+        bits = lambda t: t.view(raw).numpy()  # noqa: E731
         put = lambda pool, rows: torch.from_numpy(kv_append(bits(pool), bits(rows), slots.numpy()))  # noqa: E731
         kb, vb = put(kr, b["k_new"]), put(vr, b["v_new"])
-        assert torch.equal(k.cpu().view(torch.int16), kb) and torch.equal(v.cpu().view(torch.int16), vb)
+        assert torch.equal(k.cpu().view(raw), kb) and torch.equal(v.cpu().view(raw), vb)
         kr, vr = kb.view(kr.dtype), vb.view(vr.dtype)
     ref = oracle_gather(b["q"], kr, vr, b["tables"], b["ctx"], b["ql"], d ** -0.5)
-    torch.testing.assert_close(out.cpu(), ref, atol=TOL, rtol=TOL)
+    torch.testing.assert_close(out.cpu(), ref, atol=TOL[out.dtype], rtol=TOL[out.dtype])
 
 
 def _split_bytes(b):
@@ -79,7 +81,10 @@ def _split_bytes(b):
     (64, 8, 2, 3, torch.bfloat16), (64, 64, 1, 4, torch.float16), (64, 16, 2, 6, torch.float16),
     (80, 8, 3, 1, torch.bfloat16), (80, 32, 1, 8, torch.float16), (96, 16, 2, 2, torch.bfloat16),
     (112, 128, 1, 3, torch.float16), (128, 32, 2, 4, torch.bfloat16), (128, 8, 1, 16, torch.float16),
-    (128, 16, 1, 71, torch.bfloat16), (128, 16, 2, 3, torch.float16)])
+    (128, 16, 1, 71, torch.bfloat16), (128, 16, 2, 3, torch.float16),
+    (32, 8, 2, 3, torch.float32), (48, 16, 1, 5, torch.float32), (64, 16, 2, 1, torch.float32),
+    (80, 32, 1, 8, torch.float32), (96, 64, 2, 2, torch.float32), (112, 8, 1, 1, torch.float32),
+    (128, 16, 1, 71, torch.float32), (128, 32, 2, 4, torch.float32)])
 @pytest.mark.parametrize("lengths", [EDGES, DECODE], ids=["prompts", "decode"])
 @pytest.mark.parametrize("fused", [False, True], ids=["plain", "append"])
 def test_shapes_groups_and_block_sizes(d, bs, kv, group, dtype, lengths, fused):
@@ -98,6 +103,15 @@ def test_split_contexts(d, bs, kv, group, dtype, fused):
     # A decode batch of long contexts (a decode kernel's where one takes the shape).
     lone = _batch([(c, 1) for c, _ in LONG], dtype=dtype, d=d, bs=bs, kv=kv, group=group, seed=9 + d)
     _check(lone, fused=fused)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [64, 65, 200])
+def test_fp32_prompts_over_sequence_counts(n):
+    """Tiles found across lanes, several sequences a lane, prompts of no token among them."""
+    lengths = [(20 + (13 * i) % 90, (7 * i) % 19) for i in range(n)]
+    lengths[0], lengths[n // 2], lengths[n - 1] = (1500, 33), (40, 40), (17, 16)
+    _check(_batch(lengths, dtype=torch.float32, d=64, bs=16, kv=1, group=3, seed=n), fused=False)
 
 
 @pytest.mark.gpu
