@@ -18,11 +18,12 @@ graph for batch size B reads the first B entries of each segment and the first B
 table rows, so every graph shares the one buffer and the one copy.
 
 Attention is captured with the widest context a W-block table allows
-(max_context_len = W * block_size): the grid covers every partition a sequence can
-have, workgroups past a sequence's own context exit at once, and the split-KV
-workspace is sized for it. A sequence's output depends only on its own context and
-the GEMMs see the same M = B as the eager step, so a replay computes bit for bit what
-the eager step computes.
+(max_context_len = W * block_size): it chooses the kernel and sizes the split-KV
+workspace; the kernels read the real lengths and cut the contexts by them. The GEMMs see
+the same M = B as the eager step, so a replay computes bit for bit what the eager step
+computes wherever the eager step's longest context chooses the same kernel (always at
+GPT-2's 1024 positions in 16 bits; fp32 steps of 27 or more sequences may round
+differently, within the kernels' own error).
 
 Every capture is checked before it is instantiated: its nodes are counted by type
 through libpagedkv (pkv_graph_node_counts) and a graph holding a memset node is
