@@ -61,7 +61,7 @@ int fill_common(AttnParams& p, const char* what, void* out, int64_t out_st, int6
 }
 
 // Layout: [merge counters, kMergeCounterBytes][ml][o] when any context spans more than
-// one partition; empty otherwise.
+// one partition or the persistent MFMA kernel may run; empty otherwise.
 // Behind the counters two layouts share the space: the split contexts' partials
 // ([ml][o] per (sequence, head, 256-token partition)) and the persistent MFMA kernel's
 // ([prefix table][ml][o], partials per (workgroup, side, wave, head)); the workspace
@@ -96,7 +96,12 @@ DecodeWorkspace decode_workspace(int64_t num_seqs, int64_t num_heads, int64_t nu
             w.mfma_o_bytes = round256(slots * head_dim * 4);
         }
     }
-    if (w.max_parts == 1) w.cnt_bytes = w.ml_bytes = w.o_bytes = 0;  // single partition: no partials
+    if (w.max_parts == 1) {
+        // Single partition: no partials. The counters' room stays in front of the persistent
+        // kernel's layout, so that it never lies over counters another call relies on.
+        w.ml_bytes = w.o_bytes = 0;
+        if (w.mfma_pfx_bytes == 0) w.cnt_bytes = 0;
+    }
     return w;
 }
 
