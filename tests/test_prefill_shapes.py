@@ -44,9 +44,10 @@ def _batch(lengths, *, dtype, d, bs, kv, group, seed=0):
                 ql=torch.tensor([q for _, q in lengths]), k_new=rand(t, kv, d), v_new=rand(t, kv, d))
 
 
-def _check(b, *, fused, told=None):
+def _check(b, *, fused, told=None, scale=None):
     """told: other context lengths for the host copy, which only balances the launch."""
     d, bs = b["q"].shape[2], b["k"].shape[1]
+    scale = d ** -0.5 if scale is None else scale
     first = b["ctx"] - b["ql"]
     slots = torch.cat([b["tables"][i, torch.arange(int(f), int(f + n)) // bs] * bs
                        + torch.arange(int(f), int(f + n)) % bs for i, (f, n) in enumerate(zip(first, b["ql"]))])
@@ -54,7 +55,7 @@ def _check(b, *, fused, told=None):
     ctx = attach_host(b["ctx"].cuda(), b["ctx"] if told is None else told)
     ql = attach_host(b["ql"].cuda(), b["ql"])
     append = (b["k_new"].cuda(), b["v_new"].cuda(), slots.cuda()) if fused else None
-    out = paged_attention_hip_launch(b["q"].cuda(), k, v, b["tables"].cuda(), ctx, ql, d ** -0.5, append=append)
+    out = paged_attention_hip_launch(b["q"].cuda(), k, v, b["tables"].cuda(), ctx, ql, scale, append=append)
     torch.cuda.synchronize()
     kr, vr = b["k"], b["v"]
     if fused:
@@ -64,7 +65,7 @@ def _check(b, *, fused, told=None):
         kb, vb = put(kr, b["k_new"]), put(vr, b["v_new"])
         assert torch.equal(k.cpu().view(raw), kb) and torch.equal(v.cpu().view(raw), vb)
         kr, vr = kb.view(kr.dtype), vb.view(vr.dtype)
-    ref = oracle_gather(b["q"], kr, vr, b["tables"], b["ctx"], b["ql"], d ** -0.5)
+    ref = oracle_gather(b["q"], kr, vr, b["tables"], b["ctx"], b["ql"], scale)
     torch.testing.assert_close(out.cpu(), ref, atol=TOL[out.dtype], rtol=TOL[out.dtype])
 
 
@@ -89,6 +90,17 @@ def _split_bytes(b):
 @pytest.mark.parametrize("fused", [False, True], ids=["plain", "append"])
 def test_shapes_groups_and_block_sizes(d, bs, kv, group, dtype, lengths, fused):
     _check(_batch(lengths, dtype=dtype, d=d, bs=bs, kv=kv, group=group, seed=d + bs + group), fused=fused)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,bs,kv,group,dtype", [
+    (64, 16, 2, 1, torch.float16), (128, 16, 2, 4, torch.bfloat16), (48, 8, 2, 3, torch.float16),
+    (80, 32, 1, 8, torch.bfloat16), (64, 16, 1, 17, torch.float16), (128, 16, 2, 1, torch.float32),
+    (32, 8, 1, 3, torch.float32)])
+@pytest.mark.parametrize("scale", [0.0, -0.125])
+@pytest.mark.parametrize("lengths", [EDGES, DECODE, LONG], ids=["prompts", "decode", "long"])
+def test_scales_that_are_not_positive(d, bs, kv, group, dtype, scale, lengths):
+    _check(_batch(lengths, dtype=dtype, d=d, bs=bs, kv=kv, group=group, seed=d + 1), fused=True, scale=scale)
 
 
 @pytest.mark.gpu
