@@ -55,6 +55,12 @@ struct AttnParams {
     int* ws_pfx;
 };
 
+// Whether the byte offsets of rows 0 .. slots - 1 of a block fit the unsigned 32-bit per-lane
+// offsets of the tuned kernels (a negative slot stride does not: the generic kernel's case).
+inline bool slot_offsets_fit(const AttnParams& p, int slots, int itemsize) {
+    return p.ss >= 0 && p.ss <= 0x7fffffff && (slots * p.ss + p.head_dim) * itemsize <= 0xffffffffll;
+}
+
 // One-launch MFMA decode (attn_decode_split.hip): whether it takes these parameters (with
 // p.app_* set: including the fused append, whose source rows must be 16-byte aligned).
 bool decode_split_applies(const AttnParams& p, int dtype);

@@ -336,6 +336,7 @@ bool decode_f32_applies(const AttnParams& p) {
     if ((int64_t)p.num_seqs * p.num_kv_heads * p.max_parts * kDecodePart * 64 * 8 < kMinBytes) return false;
     if (p.num_kv_heads > 65535 || p.max_parts > 65535 || p.num_seqs > 65535) return false;
     if (p.max_parts > 1 && (!p.ws_o || !p.ws_ml)) return false;
+    if (!slot_offsets_fit(p, kBS, 4)) return false;
     // 16-byte chunk loads need 16-byte aligned rows.
     const uint64_t probe = (uint64_t)(uintptr_t)p.q | (uint64_t)(uintptr_t)p.k | (uint64_t)(uintptr_t)p.v |
                            (uint64_t)(p.q_st * 4) | (uint64_t)(p.q_sh * 4) | (uint64_t)(p.sb * 4) |

@@ -823,8 +823,7 @@ bool decode_mfma_applies(const AttnParams& p, int dtype, int64_t max_context_len
                            (uint64_t)(p.sb * 2) | (uint64_t)(p.ss * 2) | (uint64_t)(p.sh * 2) |
                            (uint64_t)(p.out_st * 2) | (uint64_t)(p.out_sh * 2);
     if (probe % 16) return false;
-    // Slot offsets inside a block in 32 bits.
-    if (kBS * p.ss * 2 >= ((int64_t)1 << 32)) return false;
+    if (!slot_offsets_fit(p, kBS, 2)) return false;
     return decode_mfma_max_grid() > 0;
 }
 

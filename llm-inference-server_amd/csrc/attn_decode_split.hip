@@ -845,8 +845,7 @@ static bool split_shape(const AttnParams& p, int dtype) {
     if (p.head_dim % 16 || p.head_dim < 32 || p.head_dim > 128) return false;
     // Units of a sequence are exact in fp32 (the run search divides in it).
     if ((int64_t)p.max_parts * kDecodePart >= ((int64_t)1 << 28)) return false;
-    // Offsets inside an 8-row half in 32 bits.
-    if (8 * p.ss * isz + p.head_dim * isz > 0xffffffffll || p.ss < 0) return false;
+    if (!slot_offsets_fit(p, 8, isz)) return false;   // inside an 8-row half
     // 16-byte rows, those of a fused append among them.
     uint64_t probe = (uint64_t)(uintptr_t)p.q | (uint64_t)(uintptr_t)p.k | (uint64_t)(uintptr_t)p.v |
                      (uint64_t)(p.q_st * isz) | (uint64_t)(p.q_sh * isz) | (uint64_t)(p.sb * isz) |

@@ -266,7 +266,7 @@ int launch_f32_attention(const AttnParams& p, hipStream_t stream) {
                            (uint64_t)(p.out_st * 4) | (uint64_t)(p.out_sh * 4);
     if (probe % 16) return PKV_EUNSUPPORTED;
     // Byte offsets inside a block fit the 32-bit-friendly range the DMA offsets assume.
-    if ((int64_t)kTile * p.ss * 4 > 0x7fffffff) return PKV_EUNSUPPORTED;
+    if (p.ss < 0 || (int64_t)kTile * p.ss * 4 > 0x7fffffff) return PKV_EUNSUPPORTED;
     if (!p.qsl) return PKV_EUNSUPPORTED;
     if (p.num_seqs == 0 || p.num_tokens == 0) return PKV_OK;
     return p.head_dim == 64 ? launch_d<64>(p, stream) : launch_d<128>(p, stream);

@@ -799,6 +799,8 @@ bool prefill_tuned(const AttnParams& p, int dtype) {
     if (p.block_shift < 3) return false;
     if (p.head_dim % 16 || p.head_dim < 32 || p.head_dim > 128) return false;
     if (dtype != PKV_FLOAT16 && dtype != PKV_BFLOAT16) return false;
+    // The kernel's offsets are unsigned (strides too large for 32 bits take its per-row path).
+    if (p.ss < 0) return false;
     // The kernel masks to -inf and takes the maximum before it scales: scale > 0 only.
     if (!(p.scale > 0.f)) return false;
     // The grid is one dimension, and row numbers of a sequence stay below 2^31.

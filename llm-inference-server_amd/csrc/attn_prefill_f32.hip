@@ -341,6 +341,8 @@ int launch_prefill_f32_mfma(const AttnParams& p, hipStream_t stream) {
     if (p.max_query_len <= 1) return PKV_EUNSUPPORTED;
     if (p.group != 1 && p.group != 2 && p.group != 4 && p.group != 8) return PKV_EUNSUPPORTED;
     if (p.num_blocks < 1) return PKV_EUNSUPPORTED;
+    // Unsigned offsets (strides too large for 32 bits take the per-row path).
+    if (p.ss < 0) return PKV_EUNSUPPORTED;
     // The kernel masks to -inf and takes the maximum before it scales: scale > 0 only.
     if (!(p.scale > 0.f)) return PKV_EUNSUPPORTED;
     // 16-byte rows: query, pool and output pointers and strides.

@@ -155,3 +155,32 @@ def test_split_workspace_is_host_arithmetic():
         for ctx in (2000, 8192, 131072):
             for q in (1, 40, 300):
                 assert need([ctx] * n, [q] * n) <= (130 << 20) + 8 * n * q * 32 + (1 << 20)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,bs,dtype", [(128, 16, torch.bfloat16), (80, 32, torch.float16), (64, 16, torch.float32)])
+@pytest.mark.parametrize("lengths", [EDGES, DECODE], ids=["prompts", "decode"])
+def test_slots_of_a_block_in_reverse_order(d, bs, dtype, lengths):
+    """A pool whose slot stride is negative (C ABI only: torch has no such strides)."""
+    b = _batch(lengths, dtype=dtype, d=d, bs=bs, kv=2, group=2, seed=d)
+    k, v = b["k"].flip(1).contiguous().cuda(), b["v"].flip(1).contiguous().cuda()
+    back = (bs - 1) * k.stride(1) * k.element_size()
+    q, tables, ctx = b["q"].cuda(), b["tables"].cuda(), b["ctx"].cuda()
+    out = torch.full_like(q, float("nan"))
+    code, L, s = native.dtype_code(dtype), native.lib(), torch.cuda.current_stream().cuda_stream
+    args = (out.data_ptr(), out.stride(0), out.stride(1), q.data_ptr(), q.stride(0), q.stride(1),
+            k.data_ptr() + back, v.data_ptr() + back, k.stride(0), -k.stride(1), k.stride(2), *k.shape,
+            tables.data_ptr(), tables.stride(0), tables.shape[1], ctx.data_ptr())
+    n, heads = len(lengths), q.shape[1]
+    if lengths is DECODE:
+        need = L.pkv_paged_attention_decode_workspace_bytes(n, heads, 2, d, 700)
+        ws = torch.zeros(need, dtype=torch.uint8, device="cuda")
+        rc = L.pkv_paged_attention_decode(*args, n, heads, 700, d ** -0.5, code, ws.data_ptr(), need, s)
+    else:
+        qsl = torch.tensor([0, *torch.cumsum(b["ql"], 0).tolist()]).cuda()
+        rc = L.pkv_paged_attention_prefill(*args, qsl.data_ptr(), n, heads, q.shape[0], int(b["ql"].max()), d ** -0.5,
+                                           code, s)
+    native.check(rc, "attention")
+    torch.cuda.synchronize()
+    ref = oracle_gather(b["q"], b["k"], b["v"], b["tables"], b["ctx"], b["ql"], d ** -0.5)
+    torch.testing.assert_close(out.cpu(), ref, atol=TOL[dtype], rtol=TOL[dtype])
