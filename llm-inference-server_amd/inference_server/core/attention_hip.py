@@ -132,6 +132,9 @@ def _batch_facts(context_lens: torch.Tensor, query_lens: torch.Tensor, block_siz
         if hit is not None and hit[0] == key:
             return hit[1]
     hctx, hql = _host_lengths(context_lens, query_lens)
+    if key is not None:
+        # Kept past this call: not the caller's tensors, which may be written to later.
+        hctx, hql = hctx.clone(), hql.clone()
     n = int(hctx.numel())
     facts = {
         "hctx": hctx,

@@ -32,6 +32,20 @@ def test_facts_are_shared_until_the_lengths_change():
     assert attention_hip._batch_facts(ctx, ql, 16, 4)["too_few_blocks"]
 
 
+def test_kept_lengths_are_not_the_callers_tensors():
+    """A host tensor of another step's values must not show through facts that an equal one
+    attached since still finds."""
+    hctx, hql = torch.tensor([20, 33]), torch.tensor([4, 1])
+    ctx, ql = _Lengths([20, 33]), _Lengths([4, 1])
+    ctx._pkv_host, ql._pkv_host = hctx, hql
+    first = attention_hip._batch_facts(ctx, ql, 16, 4)
+    ctx._pkv_host, ql._pkv_host = hctx.clone(), hql.clone()
+    hctx.copy_(torch.tensor([64, 1]))
+    hql.copy_(torch.tensor([1, 1]))
+    assert attention_hip._batch_facts(ctx, ql, 16, 4) is first
+    assert first["hctx"].tolist() == [20, 33] and first["hql"].tolist() == [4, 1]
+
+
 @pytest.mark.gpu
 def test_query_starts_follow_lengths_and_streams():
     """One upload per step and stream; lengths written in place make a new one (the same
