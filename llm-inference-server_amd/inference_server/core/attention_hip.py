@@ -152,15 +152,27 @@ def _batch_facts(context_lens: torch.Tensor, query_lens: torch.Tensor, block_siz
     return facts
 
 
-def _query_start(facts: dict, dev: torch.device, stream: int) -> torch.Tensor:
+_CAPTURED_ATTR = "_pkv_captured_qsl"
+
+
+def _query_start(facts: dict, context_lens: torch.Tensor, dev: torch.device, stream: int) -> torch.Tensor:
     """Device query_start_loc of a batch, uploaded once per step and stream. The upload
     leaves from pinned memory: a pageable one waits for everything queued on the stream,
     which cost a step one such wait per layer (3 GPT-2 prompts, 31 us a call of which the
     kernel is 12)."""
     capturing = torch.cuda.is_current_stream_capturing()
-    # A graph must not hold a buffer that lives as long as this step's length tensors:
-    # inside a capture the pageable upload is refused by the runtime.
-    qsl = None if capturing else facts["qsl"].get((dev, stream))
+    if capturing:
+        # A capture takes the one that a call before it uploaded (on any stream: whoever
+        # captures has joined the warm-up). It then lives as long as context_lens, which the
+        # graph reads too, not only until the facts change. Without one the upload below is
+        # refused by the runtime.
+        for (where, _), qsl in facts["qsl"].items():
+            if where == dev:
+                kept = getattr(context_lens, _CAPTURED_ATTR, ())
+                if not any(t is qsl for t in kept):
+                    setattr(context_lens, _CAPTURED_ATTR, (*kept, qsl))
+                return qsl
+    qsl = facts["qsl"].get((dev, stream))
     if qsl is None:
         hql = facts["hql"]
         host = torch.zeros(hql.numel() + 1, dtype=torch.long, pin_memory=not capturing)
@@ -289,7 +301,7 @@ def paged_attention_hip_launch(
 
     qsl = getattr(query_lens, _QSL_ATTR, None)
     if qsl is None:
-        qsl = _query_start(facts, dev, stream)
+        qsl = _query_start(facts, context_lens, dev, stream)
     # Workspace for split contexts (0 bytes: a batch that is not split).
     lens = (facts["hctx"].data_ptr(), facts["hql"].data_ptr())
     ws_bytes = L.pkv_paged_attention_prefill_workspace_bytes(n_seqs, n_heads, n_kv, head_dim, n_tok, *lens)

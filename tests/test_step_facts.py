@@ -72,3 +72,31 @@ def test_query_starts_follow_lengths_and_streams():
     hql.copy_(torch.tensor([2, 7]))
     ql.copy_(hql)
     check()
+
+
+@pytest.mark.gpu
+def test_a_warmed_prefill_call_can_be_captured():
+    """With host lengths attached and one call before the capture, the graph reads the
+    query_start_loc of that call, which outlives a change of the lengths' facts."""
+    g = torch.Generator().manual_seed(4)
+    k, v = (torch.randn(16, 16, 2, 64, generator=g).half().cuda() for _ in range(2))
+    tables = torch.arange(16).view(2, 8).cuda()
+    q = torch.randn(9, 4, 64, generator=g).half().cuda()
+    hctx, hql = torch.tensor([90, 70]), torch.tensor([7, 2])
+    ctx, ql = attach_host(hctx.cuda(), hctx.clone()), attach_host(hql.cuda(), hql.clone())
+    call = lambda: paged_attention_hip_launch(q, k, v, tables, ctx, ql, 0.125)  # noqa: E731
+    eager = call()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    # Other lengths through the same tensors' facts, and their memory handed out again.
+    attach_host(ql, torch.tensor([2, 7]))
+    call()
+    del call
+    spare = [torch.full((3,), -1, dtype=torch.long, device="cuda") for _ in range(64)]
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+    del spare
