@@ -72,6 +72,10 @@ const char* pkv_last_error(void);
  * kernels launch through. */
 int pkv_graph_node_counts(void* graph, int64_t* counts, int64_t num_types);
 
+/* *id = a number of the capture that `stream` is part of, another one for each capture, or
+ * 0 outside one. For callers that keep a workspace for the calls of one capture. */
+int pkv_stream_capture_id(hipStream_t stream, uint64_t* id);
+
 /* ------------------------------------------------------------------ attention
  * Paged attention over a block-major pool, the contract of the reference's
  * `paged_attention(query, k_pool, v_pool, block_tables, context_lens, query_lens,

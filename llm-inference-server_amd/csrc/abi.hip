@@ -55,3 +55,14 @@ extern "C" int pkv_graph_node_counts(void* graph, int64_t* counts, int64_t num_t
     }
     return PKV_OK;
 }
+
+extern "C" int pkv_stream_capture_id(hipStream_t stream, uint64_t* id) {
+    pkv::clear_error();
+    if (!id) return pkv::fail(PKV_EINVAL, "stream_capture_id: null pointer");
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long n = 0;
+    const hipError_t e = hipStreamGetCaptureInfo(stream, &status, &n);
+    if (e != hipSuccess) return pkv::fail(PKV_EHIP, "stream_capture_id: %s", hipGetErrorString(e));
+    *id = status == hipStreamCaptureStatusActive ? (uint64_t)n : 0;
+    return PKV_OK;
+}

@@ -65,6 +65,10 @@ def _host_lengths(context_lens: torch.Tensor, query_lens: torch.Tensor) -> tuple
     return hc.long().contiguous(), hq.long().contiguous()
 
 
+#: The merge counters at the front of a workspace, what must read zero (include/pagedkv.h).
+_COUNTER_BYTES = 256 * 1024
+
+
 class _Workspaces:
     """One attention workspace per (device, stream), grown on demand and reused across
     calls (split-KV decode and split prefill; a stream runs one call at a time). It is
@@ -73,14 +77,17 @@ class _Workspaces:
     them need no initialisation). A different stream gets its own buffer. Sizes are powers
     of two and a buffer that had to grow is kept, not freed: a graph captured on that
     stream earlier replays into it (the kept ones add up to less than the one in use).
-    Growth inside a capture is a temporary of that graph. After a call that did not
-    complete (a launch error, a reset device), `reset()` drops the buffers so the next call
-    gets a zero-filled one."""
+    A capture that finds none large enough gets one of its own, shared by its later calls
+    and cleared once, at its first call, by every replay (one fill node, not one a layer). After a call that did not complete (a
+    launch error, a reset device), `reset()` drops the buffers so the next call gets a
+    zero-filled one."""
 
     def __init__(self) -> None:
         self._lock = threading.Lock()
         self._bufs: dict[tuple[int, int], torch.Tensor] = {}
         self._kept: list[torch.Tensor] = []
+        # (capture id, buffer) of the capture under way on a stream.
+        self._captured: dict[tuple[int, int], tuple[int, torch.Tensor]] = {}
 
     def partials(self, device: torch.device, stream: int, nbytes: int) -> torch.Tensor:
         idx = device.index if device.index is not None else torch.cuda.current_device()
@@ -88,9 +95,16 @@ class _Workspaces:
         with self._lock:
             buf = self._bufs.get(key)
             if buf is None or buf.numel() < nbytes:
-                size = 1 << (max(nbytes, 1 << 16) - 1).bit_length()
                 if torch.cuda.is_current_stream_capturing():
-                    return torch.zeros(size, dtype=torch.uint8, device=device)
+                    capture = native.stream_capture_id(stream)
+                    held = self._captured.get(key)
+                    if held is None or held[0] != capture or held[1].numel() < nbytes:
+                        own = torch.empty(max(nbytes, 1 << 16), dtype=torch.uint8, device=device)
+                        own[:_COUNTER_BYTES].zero_()
+                        held = self._captured[key] = (capture, own)
+                    return held[1]
+                self._captured.pop(key, None)
+                size = 1 << (max(nbytes, 1 << 16) - 1).bit_length()
                 if buf is not None:
                     self._kept.append(buf)
                 buf = torch.zeros(size, dtype=torch.uint8, device=device)
@@ -102,6 +116,7 @@ class _Workspaces:
         with self._lock:
             self._bufs.clear()
             self._kept.clear()
+            self._captured.clear()
 
 
 _WORKSPACES = _Workspaces()

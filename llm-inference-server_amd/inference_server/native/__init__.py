@@ -34,6 +34,7 @@ SIGNATURES: dict[str, tuple] = {
     "pkv_abi_version": (_int, []),
     "pkv_last_error": (ctypes.c_char_p, []),
     "pkv_graph_node_counts": (_int, [_ptr, _ptr, _i64]),
+    "pkv_stream_capture_id": (_int, [_ptr, ctypes.POINTER(ctypes.c_uint64)]),
     "pkv_paged_attention_decode_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i64]),
     "pkv_paged_attention_decode": (
         _int,
@@ -212,6 +213,13 @@ def stream_handle(device: torch.device) -> int:
     if _raw_stream is not None:
         return _raw_stream(device.index if device.index is not None else torch.cuda.current_device())
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def stream_capture_id(stream: int) -> int:
+    """A number of the capture `stream` is part of, another for each; 0 outside one."""
+    out = ctypes.c_uint64()
+    check(lib().pkv_stream_capture_id(stream, ctypes.byref(out)), "pkv_stream_capture_id")
+    return out.value
 
 
 def require_gpu(t: torch.Tensor, what: str) -> None:

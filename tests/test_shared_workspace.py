@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from inference_server import native
-from inference_server.core.attention_hip import _WORKSPACES, paged_attention_hip_launch
+from inference_server.core.attention_hip import _WORKSPACES, attach_host, paged_attention_hip_launch
 from oracle.gather import paged_attention_gather as oracle_gather
 
 pytestmark = pytest.mark.gpu
@@ -64,3 +64,30 @@ def test_the_same_on_the_static_scratch():
         native.check(rc, "pkv_paged_attention_decode_noalloc")
         torch.cuda.synchronize()
         _check(b, out, rows)
+
+
+def test_a_capture_clears_one_workspace_for_all_its_calls():
+    """Captures on a stream without a workspace: one fill node each, whatever the calls, and
+    each capture its own (the second one is replayed first)."""
+    from inference_server.core.decode_graphs import node_census
+
+    b = [t.cuda() for t in _split()]
+    hosts = (_split()[4], _split()[5])
+    attach_host(b[4], hosts[0])
+    attach_host(b[5], hosts[1])
+    eager = paged_attention_hip_launch(*b, 128 ** -0.5)
+    stream, graphs = torch.cuda.Stream(), []
+    for _ in range(2):
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph, stream=stream):
+            outs = [paged_attention_hip_launch(*b, 128 ** -0.5) for _ in range(3)]
+        assert node_census(graph) == {"kernel": 3 + 1}
+        graph.instantiate()
+        graphs.append((graph, outs))
+    for _ in range(2):
+        for graph, outs in reversed(graphs):
+            for o in outs:
+                o.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(o, eager) for o in outs)
