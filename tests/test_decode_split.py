@@ -149,3 +149,27 @@ def test_rows_off_16_bytes_are_appended_by_the_append_kernel():
                                      torch.ones(n, dtype=torch.long).cuda(), 64 ** -0.5,
                                      append=(odd["k_new"], odd["v_new"], slots.cuda()))
     assert torch.equal(out.cpu(), plain)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("far", [16 * 8, 16 * 40 + 5])
+def test_the_largest_weight_is_not_rounded(dtype, far):
+    """Two keys that nearly cancel, the later one's weight against the first no number of the
+    pool dtype: rounded, it would leave nothing of the output. (2e-2 covers the output's own
+    rounding and exp2's.)"""
+    n, ctx = 12, far + 9
+    b = _batch([ctx] * n, dtype=dtype, d=64, bs=16, kv=1, group=1)
+    score = torch.tensor([1.0 + 0.34375 * i for i in range(n)]).to(dtype)     # all numbers of both dtypes
+    w = score.double().exp()
+    b["q"].zero_()[:, :, 0] = 8.0                                              # scores: K's first column
+    for i in range(n):
+        k, v = torch.zeros(ctx, 64), torch.zeros(ctx, 64)
+        k[:, 0] = -100.0
+        k[0, 0], k[far, 0] = 0.0, score[i]
+        v[0], v[far] = -w[i].to(dtype).float(), 1.0
+        pos = torch.arange(ctx)
+        at = b["tables"][i, pos // 16], pos % 16
+        b["k"][at], b["v"][at] = k.to(dtype)[:, None], v.to(dtype)[:, None]
+    want = (w - w.to(dtype).double()) / (1 + w)
+    out = _run(b, fused=False)[0].double()
+    torch.testing.assert_close(out, want[:, None, None].expand_as(out), rtol=2e-2, atol=1e-6)
