@@ -71,7 +71,7 @@ bool prompt_split_f32_applies(const AttnParams& p);
 int launch_prompt_split_f32(const AttnParams& p, hipStream_t stream);
 // Whether the batch's row tiles make at most two and a quarter rounds of the GPU there.
 bool prompt_split_f32_few(const AttnParams& p);
-// fp32 register kernel (attn_decode.hip): the shapes and sizes where it beats the kernel
+// fp32 register kernel (attn_decode.hip): the shapes where it beats the kernel
 // above; it appends nothing itself.
 bool decode_f32_applies(const AttnParams& p);
 int launch_decode_f32(const AttnParams& p, hipStream_t stream);

@@ -1,14 +1,16 @@
-// Paged decode attention for fp32 pools, block_size 16, head_dim 64, ungrouped heads, for
-// batches of much K/V: a partition kernel with K/V staged in registers, and a split-KV merge
-// kernel.
+// Paged decode attention for fp32 pools, block_size 16, head_dim 64, one or two query heads per
+// KV head: a partition kernel with K/V staged in registers, and a split-KV merge kernel.
 //
-// Bound: HBM and the arithmetic beside it. With one head a group the one-launch MFMA kernel
-// (attn_decode_split.hip) spends its fp32 matrix steps on 16 columns of which one counts;
-// here each product is computed once. Measured, us a call with the append launch, this kernel
-// first, 12 heads: 32 sequences of 16-1024 tokens 27.3 vs 29.0, 60 of 16-2000 73 vs 77; with
-// less K/V its second launch decides: 22 of 16-1000 24.7 vs 22.8, 32 of 16-300 24.5 vs 22.1.
-// Groups of 2 are even (64 of 16-1000 38.0 vs 38.5), larger ones lose (16 of 100-3000, groups
-// of 8, 26.8 vs 20.5).
+// Bound: HBM and the arithmetic beside it. With so few heads a group the one-launch MFMA kernel
+// (attn_decode_split.hip) spends its fp32 matrix steps on 16 columns of which one or two count;
+// here each product is computed once. Measured, us a call replayed from a graph, this kernel
+// first, 12 heads: 8 sequences of 16-500 tokens 8.3 vs 11.3, 16 of 500-1000 18.2 vs 20.7, 32 of
+// 16-1000 22.7 vs 23.7, 64 of 200-3000 114 vs 129, 22 of 16-1000 18.8 vs 18.8; issued eagerly
+// its second launch can cost the host more than that (22 of 16-1000 with the append 24.7 vs
+// 22.8), but a rule on sizes would have an eager step and its captured form, which is told the
+// longest context its tables allow, run different kernels. Groups of 2, 6 KV heads: 64 of
+// 500-2000 46 vs 57; of 4 the other is even or faster (8 of 16-1000 10.7 vs 9.6), of 8 faster
+// (200 of 500-2000 68 vs 61).
 //
 //  * Work unit = (KV head, 256-token partition, sequence): one 256-thread workgroup of 4
 //    wave64s, 64 tokens (4 blocks) per wave.
@@ -95,11 +97,11 @@ __global__ __launch_bounds__(kWaves * 64) void paged_decode_kernel(const AttnPar
     Vec16 q[G][CPL];
     {
         const char* qrow = reinterpret_cast<const char*>(p.q) + ((int64_t)seq * p.q_st + (int64_t)kvh * G * p.q_sh) * ISZ;
-        const uint32_t q_head_bytes = (uint32_t)(p.q_sh * ISZ);
+        const int64_t q_head_bytes = p.q_sh * ISZ;
 #pragma unroll
         for (int g = 0; g < G; ++g)
 #pragma unroll
-            for (int i = 0; i < CPL; ++i) q[g][i] = load16(qrow + (g * q_head_bytes + (uint32_t)((i * KLPT + kj) * 16)));
+            for (int i = 0; i < CPL; ++i) q[g][i] = load16(qrow + g * q_head_bytes + (i * KLPT + kj) * 16);
     }
     const char* kblk[kBPW];
     const char* vblk[kBPW];
@@ -326,14 +328,10 @@ int launch_g(const AttnParams& p, dim3 grid, hipStream_t stream) {
     return check_launch("paged decode combine");
 }
 
-// K/V (at the batch's longest context) from which this kernel is the faster one (see above).
-constexpr int64_t kMinBytes = (int64_t)160 << 20;
-
 }  // namespace
 
 bool decode_f32_applies(const AttnParams& p) {
-    if (p.block_size != kBS || p.head_dim != 64 || p.group != 1) return false;
-    if ((int64_t)p.num_seqs * p.num_kv_heads * p.max_parts * kDecodePart * 64 * 8 < kMinBytes) return false;
+    if (p.block_size != kBS || p.head_dim != 64 || (p.group != 1 && p.group != 2)) return false;
     if (p.num_kv_heads > 65535 || p.max_parts > 65535 || p.num_seqs > 65535) return false;
     if (p.max_parts > 1 && (!p.ws_o || !p.ws_ml)) return false;
     if (!slot_offsets_fit(p, kBS, 4)) return false;
@@ -346,7 +344,8 @@ bool decode_f32_applies(const AttnParams& p) {
 
 int launch_decode_f32(const AttnParams& p, hipStream_t stream) {
     if (!decode_f32_applies(p)) return PKV_EUNSUPPORTED;
-    return launch_g<64, 1>(p, dim3((unsigned)p.num_kv_heads, (unsigned)p.max_parts, (unsigned)p.num_seqs), stream);
+    const dim3 grid((unsigned)p.num_kv_heads, (unsigned)p.max_parts, (unsigned)p.num_seqs);
+    return p.group == 1 ? launch_g<64, 1>(p, grid, stream) : launch_g<64, 2>(p, grid, stream);
 }
 
 }  // namespace pkv

@@ -151,6 +151,19 @@ def test_rows_off_16_bytes_are_appended_by_the_append_kernel():
     assert torch.equal(out.cpu(), plain)
 
 
+#: Around the edges of a block, a wave's 64 tokens and a 256-token partition, up to 5 partitions.
+REGISTER_EDGES = [1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257, 271, 320, 321, 511, 512, 513,
+                  576, 767, 768, 769, 1000, 1023, 1024, 1025, 1279, 1280]
+
+
+@pytest.mark.parametrize("kv,group", [(12, 1), (3, 2)])
+@pytest.mark.parametrize("ctx", [REGISTER_EDGES, REGISTER_EDGES[:15]], ids=["partitions", "one partition"])
+@pytest.mark.parametrize("fused", [False, True], ids=["plain", "append"])
+def test_fp32_register_kernel(kv, group, ctx, fused):
+    """attn_decode.hip: fp32, head_dim 64, groups of 1 and 2."""
+    _check(_batch(ctx, dtype=torch.float32, d=64, bs=16, kv=kv, group=group, seed=group), fused=fused)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("far", [16 * 8, 16 * 40 + 5])
 def test_the_largest_weight_is_not_rounded(dtype, far):
