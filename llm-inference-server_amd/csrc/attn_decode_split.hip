@@ -307,6 +307,16 @@ __device__ __forceinline__ int wave_scan(int x, int lane) {
 __device__ __forceinline__ int wave_total(int x, int lane) {
     return __builtin_amdgcn_readlane(wave_scan(x, lane), 63);
 }
+// The largest of the lanes' x >= 0.
+__device__ __forceinline__ int wave_max(int x) {
+    auto up = [](int a, int b) { return a > b ? a : b; };
+    x = up(x, dpp_shr<0x111>(x));
+    x = up(x, dpp_shr<0x112>(x));
+    x = up(x, dpp_shr<0x114>(x));
+    x = up(x, dpp_shr<0x118>(x));
+    return up(up(__builtin_amdgcn_readlane(x, 15), __builtin_amdgcn_readlane(x, 31)),
+              up(__builtin_amdgcn_readlane(x, 47), __builtin_amdgcn_readlane(x, 63)));
+}
 
 // Context length as every decode kernel clamps it: never past the table row or the
 // partials the workspace was sized for (neither binds for valid input).
@@ -319,6 +329,19 @@ __device__ __forceinline__ int decode_ctx(const AttnParams& p, int seq) {
     return c > 0 ? (int)c : 0;
 }
 
+// How a launch cuts its contexts (lengths in units). The host gives what the shape decides; the
+// lengths decide the rest on the device, so that a sequence's result does not depend on the
+// bound that the launch was given for them: a captured step, told the longest context its
+// tables allow, computes what the eager step computes.
+enum CutMode { kCutNone, kCutRuns };
+struct Cut {
+    int mode;
+    int min_run;                              // a run is never shorter
+    int whole;                                // a batch of no longer context is not cut
+    int slots, slots2, slots2_from;           // runs of one KV head that the GPU holds (0: do not
+                                              // cut); slots2 where the longest context reaches slots2_from
+};
+
 // The `at`-th run of one KV head's batch, numbered sequence by sequence; seq < 0: none.
 struct Pick {
     int seq, ctx, split, n_splits;
@@ -326,8 +349,8 @@ struct Pick {
 
 // Every wave by itself, lane l holding the contexts of sequences PER l .. PER l + PER - 1.
 template <int PER>
-__device__ __forceinline__ Pick pick_run(const AttnParams& p, int lane, int at, int min_run, int slots) {
-    int units_of[PER], cl[PER], units = 0;
+__device__ __forceinline__ Pick pick_run(const AttnParams& p, int lane, int at, const Cut& cut) {
+    int units_of[PER], cl[PER], units = 0, longest = 0;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const int s = lane * PER + i;
@@ -337,14 +360,22 @@ __device__ __forceinline__ Pick pick_run(const AttnParams& p, int lane, int at, 
     for (int i = 0; i < PER; ++i) {
         units_of[i] = (cl[i] + kUnit - 1) / kUnit;
         units += units_of[i];
+        longest = units_of[i] > longest ? units_of[i] : longest;
     }
+    // In whole partials, as the host rounds the bound.
+    constexpr int PART = kDecodePart / kUnit;
+    longest = (wave_max(longest) + PART - 1) / PART * PART;
+    const int slots = longest <= cut.whole ? 0 : longest >= cut.slots2_from ? cut.slots2 : cut.slots;
     // The shortest run with which one KV head's runs fit its share of the GPU's slots: from
     // the even share of those left when every sequence's last run is half empty, up in
     // growing steps (mostly none or one).
     const int total = wave_total(units, lane);
-    const int even = slots - p.num_seqs / 2;  // slots >= num_seqs
-    int run = (total + even - 1) / even;
-    run = run > min_run ? run : min_run;
+    int run = 1 << 30;                        // none is cut
+    if (slots > 0) {
+        const int even = slots - p.num_seqs / 2;  // slots >= num_seqs
+        run = (total + even - 1) / even;
+        run = run > cut.min_run ? run : cut.min_run;
+    }
     int n_of[PER], mine = 0;
     for (int step = (run + 15) >> 4;; run += step, step += (step + 1) >> 1) {
         mine = 0;
@@ -426,7 +457,7 @@ constexpr int wgs_per_cu(int row_bytes, int NW) {
 // f / G, head f % G, each with its own causal bound; no split and no append. Else they are
 // the G heads of a sequence's one token.
 template <typename T, int D, int NW, bool PROMPT>
-__global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnParams p, int min_run, int slots) {
+__global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnParams p, const Cut cut) {
     using C = Contract<T, D>;
     constexpr int ISZ = (int)sizeof(T);
     constexpr int ROWB = D * ISZ;             // bytes per (token, head) row
@@ -464,13 +495,12 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
         // Keys visible to the tile's last token.
         ctx = pos0 + (int)((uint32_t)(row0 + rows - 1) / (uint32_t)G) + 1;
         if (ctx <= 0) return;
-    } else if (slots == 0) {                         // one workgroup per (sequence, KV head)
+    } else if (cut.mode == kCutNone) {               // one workgroup per (sequence, KV head)
         seq = at;
         ctx = __builtin_amdgcn_readfirstlane(decode_ctx(p, seq));
         if (ctx == 0) return;
     } else {
-        const Pick pick = p.num_seqs <= 64 ? pick_run<1>(p, lane, at, min_run, slots)
-                                           : pick_run<kScanPer>(p, lane, at, min_run, slots);
+        const Pick pick = p.num_seqs <= 64 ? pick_run<1>(p, lane, at, cut) : pick_run<kScanPer>(p, lane, at, cut);
         if (pick.seq < 0) return;
         seq = pick.seq;
         ctx = pick.ctx;
@@ -775,29 +805,35 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
 template <typename T, int D, int NW>
 int launch_nw(const AttnParams& p, hipStream_t stream) {
     const int64_t pairs = (int64_t)p.num_seqs * p.num_kv_heads;
-    int64_t fits = (int64_t)kCus * wgs_per_cu(D * (int)sizeof(T), NW);
-    // Many pairs of long contexts: runs for two rounds, or the longest context would be
-    // walked whole (250 sequences of 512-8192 tokens, 8/2 heads, bf16: 219 -> 189 us; 60 of
-    // 16-2000, 12 heads of 64, fp32: 84 -> 72); with less to read the second round's start and
-    // merges cost more than it evens out (64 of 16-2048, 12 heads of 64, fp16: 24 -> 25.5;
-    // 120 of 1-1000, 32/8 heads, fp16: 49 -> 55).
-    const int64_t units = (int64_t)p.max_parts * (kDecodePart / kUnit);
-    if ((2 * pairs > fits && pairs * units * kUnit * D * 2 * (int64_t)sizeof(T) > ((int64_t)1 << 30)) ||
-        (pairs >= fits && units >= 24 * NW))
-        fits *= 2;
+    const int64_t fits = (int64_t)kCus * wgs_per_cu(D * (int)sizeof(T), NW);
+    const int64_t units = (int64_t)p.max_parts * (kDecodePart / kUnit);   // longest context's bound
+    Cut cut{};
     // At least 4 units a wave and run (and a workspace slot's tokens); contexts of up to 8
     // units a wave are not worth the merge (12 layers of a GPT-2 decode step captured for
     // 1024 tokens, 8 sequences, fp16: 161.5 -> 158.2 us with the projections).
-    const int min_run = NW * 4 > kDecodePart / kUnit ? NW * 4 : kDecodePart / kUnit;
+    cut.min_run = NW * 4 > kDecodePart / kUnit ? NW * 4 : kDecodePart / kUnit;
+    cut.whole = NW * 8;
     // No split either where the pairs fill the GPU by themselves, or where the counters or
     // the scan do not reach.
-    int slots = 0;
-    if (units > NW * 8 && p.ws_cnt && p.num_seqs <= kMaxScanSeqs && pairs < fits &&
-        p.num_seqs * units < ((int64_t)1 << 31))
-        slots = (int)(fits / p.num_kv_heads);
-    const int64_t grid = slots > 0 ? (int64_t)(slots > p.num_seqs ? slots : p.num_seqs) * p.num_kv_heads : pairs;
+    if (p.ws_cnt && p.num_seqs <= kMaxScanSeqs && p.num_seqs * units < ((int64_t)1 << 31)) {
+        // Many pairs of long contexts: runs for two rounds, or the longest context would be
+        // walked whole (250 sequences of 512-8192 tokens, 8/2 heads, bf16: 219 -> 189 us; 60 of
+        // 16-2000, 12 heads of 64, fp32: 84 -> 72); with less to read the second round's start and
+        // merges cost more than it evens out (64 of 16-2048, 12 heads of 64, fp16: 24 -> 25.5;
+        // 120 of 1-1000, 32/8 heads, fp16: 49 -> 55).
+        int64_t from = 0x7fffffff;
+        if (2 * pairs > fits) from = ((int64_t)1 << 30) / (pairs * kUnit * D * 2 * (int64_t)sizeof(T)) + 1;
+        if (pairs >= fits && from > 24 * NW) from = 24 * NW;
+        cut.slots2_from = (int)from;
+        cut.slots = pairs < fits ? (int)(fits / p.num_kv_heads) : 0;
+        cut.slots2 = pairs < 2 * fits ? (int)(2 * fits / p.num_kv_heads) : 0;
+    }
+    const int slots = units >= cut.slots2_from ? cut.slots2 : cut.slots;
+    if (units > cut.whole && slots > 0) cut.mode = kCutRuns;
+    const int64_t grid =
+        cut.mode == kCutRuns ? (int64_t)(slots > p.num_seqs ? slots : p.num_seqs) * p.num_kv_heads : pairs;
     if (grid > 0x7fffffff) return PKV_EUNSUPPORTED;
-    paged_decode_split_kernel<T, D, NW, false><<<dim3((unsigned)grid), NW * 64, 0, stream>>>(p, min_run, slots);
+    paged_decode_split_kernel<T, D, NW, false><<<dim3((unsigned)grid), NW * 64, 0, stream>>>(p, cut);
     return check_launch("paged decode attention (split)");
 }
 
@@ -840,7 +876,7 @@ int64_t prompt_tiles(const AttnParams& p) { return p.num_tokens * p.group / kUni
 template <int D>
 int launch_prompt(const AttnParams& p, hipStream_t stream) {
     const unsigned grid = (unsigned)(prompt_tiles(p) * p.num_kv_heads);
-    paged_decode_split_kernel<float, D, 4, true><<<dim3(grid), 256, 0, stream>>>(p, 0, 0);
+    paged_decode_split_kernel<float, D, 4, true><<<dim3(grid), 256, 0, stream>>>(p, Cut{});
     return check_launch("paged prompt attention (split)");
 }
 

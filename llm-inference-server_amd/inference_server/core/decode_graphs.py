@@ -18,12 +18,13 @@ graph for batch size B reads the first B entries of each segment and the first B
 table rows, so every graph shares the one buffer and the one copy.
 
 Attention is captured with the widest context a W-block table allows
-(max_context_len = W * block_size): it chooses the kernel and sizes the split-KV
-workspace; the kernels read the real lengths and cut the contexts by them. The GEMMs see
-the same M = B as the eager step, so a replay computes bit for bit what the eager step
-computes wherever the eager step's longest context chooses the same kernel (always at
-GPT-2's 1024 positions in 16 bits; fp32 steps of 27 or more sequences may round
-differently, within the kernels' own error).
+(max_context_len = W * block_size): it sizes the split-KV workspace and the grid; the
+kernels read the real lengths and cut the contexts by them alone. The GEMMs see the same
+M = B as the eager step, so a replay computes bit for bit what the eager step computes,
+but for two choices that go by that bound, both of large batches: the persistent 16-bit
+kernel (512 MiB of K/V at the bound: 171 sequences of GPT-2's 1024 positions) and
+workgroups of two waves (four rounds of (sequence, KV head) pairs of at most 512 tokens:
+4096 pairs in 16 bits, 2048 in fp32 at heads of 64, half of that at 128).
 
 Every capture is checked before it is instantiated: its nodes are counted by type
 through libpagedkv (pkv_graph_node_counts) and a graph holding a memset node is

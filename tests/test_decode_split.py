@@ -11,7 +11,8 @@ import pytest
 import torch
 
 from inference_server import native
-from inference_server.core.attention_hip import paged_attention_hip_launch
+from inference_server.core.attention_hip import attach_host, paged_attention_hip_launch
+from inference_server.core.decode_graphs import capture_step
 from oracle.gather import paged_attention_gather as oracle_gather
 
 pytestmark = pytest.mark.gpu
@@ -162,6 +163,45 @@ REGISTER_EDGES = [1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 
 def test_fp32_register_kernel(kv, group, ctx, fused):
     """attn_decode.hip: fp32, head_dim 64, groups of 1 and 2."""
     _check(_batch(ctx, dtype=torch.float32, d=64, bs=16, kv=kv, group=group, seed=group), fused=fused)
+
+
+def _captured(b, width, bound):
+    """The call captured with `bound` as the longest context, replayed on the real lengths."""
+    n = len(b["ctx"])
+    tables = torch.zeros(n, width, dtype=torch.long)
+    tables[:, :b["tables"].shape[1]] = b["tables"]
+    ctx, ones = b["ctx"].cuda(), torch.ones(n, dtype=torch.long)
+    attach_host(ctx, torch.full((n,), bound))
+    args = (b["q"].cuda(), b["k"].cuda(), b["v"].cuda(), tables.cuda(), ctx, attach_host(ones.cuda(), ones),
+            b["q"].shape[2] ** -0.5)
+    graph, out, census = capture_step(lambda: paged_attention_hip_launch(*args), torch.device("cuda", 0),
+                                      torch.cuda.Stream(), None, "decode")
+    out.fill_(float("nan"))
+    graph.replay()
+    torch.cuda.synchronize()
+    return out.cpu(), census
+
+
+@pytest.mark.parametrize("n,dtype,kv,group,d,bs,lo,hi,bound", [
+    (24, torch.float32, 12, 1, 64, 16, 40, 500, 1024), (8, torch.float32, 6, 2, 64, 16, 40, 300, 1024),
+    (32, torch.float32, 4, 4, 64, 16, 40, 500, 1024), (8, torch.float32, 8, 1, 128, 16, 40, 250, 2048),
+    (64, torch.float16, 12, 1, 64, 16, 40, 500, 1024), (43, torch.float16, 12, 1, 64, 16, 40, 512, 1024),
+    (8, torch.float16, 12, 1, 64, 16, 17, 700, 1024), (64, torch.bfloat16, 8, 4, 128, 16, 30, 250, 1024),
+    (8, torch.bfloat16, 8, 4, 128, 16, 30, 520, 4096), (20, torch.float16, 1, 3, 80, 32, 30, 520, 4096),
+    (130, torch.float16, 3, 1, 64, 16, 30, 600, 15000), (130, torch.float16, 3, 1, 64, 32, 30, 11000, 15000)])
+def test_a_captured_call_computes_the_eager_one(n, dtype, kv, group, d, bs, lo, hi, bound):
+    """Bit for bit, whatever longest context the capture was told: what is cut, and where, comes
+    from the lengths."""
+    ctx = [lo + i % 7 for i in range(n)]
+    for i in range(5):
+        ctx[(i * n) // 5] = hi - i
+    b = _batch(ctx, dtype=dtype, d=d, bs=bs, kv=kv, group=group, seed=n)
+    eager = _run(b, fused=False)[0]
+    out, census = _captured(b, -(-bound // bs), bound)
+    assert torch.equal(out, eager)
+    # One launch, but for the fp32 register kernel and its merge.
+    registers = dtype == torch.float32 and d == 64 and group <= 2
+    assert census == {"kernel": 2 if registers else 1}
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
