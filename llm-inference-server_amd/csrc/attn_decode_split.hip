@@ -808,11 +808,17 @@ int launch_nw(const AttnParams& p, hipStream_t stream) {
     const int64_t fits = (int64_t)kCus * wgs_per_cu(D * (int)sizeof(T), NW);
     const int64_t units = (int64_t)p.max_parts * (kDecodePart / kUnit);   // longest context's bound
     Cut cut{};
-    // At least 4 units a wave and run (and a workspace slot's tokens); contexts of up to 8
-    // units a wave are not worth the merge (12 layers of a GPT-2 decode step captured for
-    // 1024 tokens, 8 sequences, fp16: 161.5 -> 158.2 us with the projections).
-    cut.min_run = NW * 4 > kDecodePart / kUnit ? NW * 4 : kDecodePart / kUnit;
-    cut.whole = NW * 8;
+    // Units a wave that a run has at least (and a workspace slot's tokens), and that a context
+    // may have before it is worth the merge: 2 and 4 where a unit is dear, fp32 products and
+    // rows of 160 bytes up, else 3 and 6. Replayed from graphs, us a call, 2 and 4 vs 3 and 6
+    // vs 4 and 8: 32/8 heads of 128, bf16, 4 sequences of 16-1000 tokens 9.9 / - / 13.6, 16 of
+    // them 11.1 / - / 14.8; fp32, 16/4 heads of 64, 8 of 16-1000 9.6 / - / 16.5; over 40 batches
+    // of 1-64 sequences of 300-8000 tokens (geometric mean, relative): 8/4 heads of 80 0.93 /
+    // 0.94 / 1.02, 16/4 of 96 0.95 / 0.97 / 1.04, 12 heads of 64, fp16, 1.02 / 1.01 / 1.04, 8/4
+    // of 64 1.04 / 1.03 / 1.05.
+    constexpr bool kDear = sizeof(T) == 4 || D >= 80;
+    cut.min_run = NW * (kDear ? 2 : 3) > kDecodePart / kUnit ? NW * (kDear ? 2 : 3) : kDecodePart / kUnit;
+    cut.whole = NW * (kDear ? 4 : 6);
     // No split either where the pairs fill the GPU by themselves, or where the counters or
     // the scan do not reach.
     if (p.ws_cnt && p.num_seqs <= kMaxScanSeqs && p.num_seqs * units < ((int64_t)1 << 31)) {
