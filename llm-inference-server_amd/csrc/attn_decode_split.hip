@@ -15,7 +15,8 @@
 //    length (no less than 4 units a wave) with which all runs fit the GPU at once, and finds
 //    its own (sequence, split) by a wave scan, no barrier. The grid is bounded by the GPU, not
 //    by the longest context a captured graph must serve, and holds next to no empty
-//    workgroups; a sequence's runs are of even lengths.
+//    workgroups; a sequence's runs are of even lengths. Batches that fill the GPU by their
+//    pairs alone have only their outlying long contexts cut (pick_long).
 //  * Streaming: per wave a two-slot ring of units in LDS (K and V, 16 rows of one KV head),
 //    filled by nontemporal LDS DMA; a unit's K and V^T fragments are read into registers
 //    first and the slot refilled with the unit after next at once. Waits are explicit vmcnt
@@ -333,13 +334,14 @@ __device__ __forceinline__ int decode_ctx(const AttnParams& p, int seq) {
 // lengths decide the rest on the device, so that a sequence's result does not depend on the
 // bound that the launch was given for them: a captured step, told the longest context its
 // tables allow, computes what the eager step computes.
-enum CutMode { kCutNone, kCutRuns };
+enum CutMode { kCutNone, kCutRuns, kCutLong };
 struct Cut {
     int mode;
     int min_run;                              // a run is never shorter
     int whole;                                // a batch of no longer context is not cut
     int slots, slots2, slots2_from;           // runs of one KV head that the GPU holds (0: do not
                                               // cut); slots2 where the longest context reaches slots2_from
+    int long_from;                            // kCutLong: only contexts from here on are cut
 };
 
 // The `at`-th run of one KV head's batch, numbered sequence by sequence; seq < 0: none.
@@ -410,6 +412,48 @@ __device__ __forceinline__ Pick pick_run(const AttnParams& p, int lane, int at, 
             }
         return r;
     }
+}
+
+// Batches that fill the GPU by themselves (or exceed the scan above): only contexts that would
+// outlast the rest of the launch are cut, into runs of twice a slot's share of the batch. The
+// first num_seqs picks are the sequences' first runs, which read nothing but their own length
+// unless it is a long one; the others are the further runs of the long ones, at most half as
+// many as one KV head has slots. us a call before and now, 8/2 heads of 128, bf16, one context
+// of 8192 tokens among 600 of 50-150: 92 -> 30, among 1100: 97 -> 41; fp32, one of 4096 among
+// 400: 125 -> 61; 600 short ones alone 17.3 -> 17.1.
+__device__ __forceinline__ Pick pick_long(const AttnParams& p, int lane, int at, const Cut& cut) {
+    auto units_at = [&](int s) { return (decode_ctx(p, s) + kUnit - 1) / kUnit; };
+    if (at < p.num_seqs) {
+        const int ctx = __builtin_amdgcn_readfirstlane(decode_ctx(p, at));
+        if (ctx == 0) return Pick{-1, 0, 0, 0};
+        if ((ctx + kUnit - 1) / kUnit < cut.long_from) return Pick{at, ctx, 0, 1};
+    }
+    int sum = 0;
+#pragma unroll 4
+    for (int s = lane; s < p.num_seqs; s += 64) sum += units_at(s);
+    const int share = (wave_total(sum, lane) + cut.slots - 1) / cut.slots;
+    const int run = 2 * share > cut.min_run ? 2 * share : cut.min_run;
+    auto runs_of = [&](int units) { return units >= cut.long_from ? (units + run - 1) / run : 1; };
+    if (at < p.num_seqs) {
+        const int ctx = __builtin_amdgcn_readfirstlane(decode_ctx(p, at));
+        return Pick{at, ctx, 0, runs_of((ctx + kUnit - 1) / kUnit)};
+    }
+    int left = at - p.num_seqs;
+    for (int s0 = 0; s0 < p.num_seqs; s0 += 64) {
+        const int s = s0 + lane;
+        const int ctx = s < p.num_seqs ? decode_ctx(p, s) : 0;
+        const int more = runs_of((ctx + kUnit - 1) / kUnit) - 1;
+        const int incl = wave_scan(more, lane);
+        const uint64_t found = __builtin_amdgcn_ballot_w64(left < incl);
+        if (found) {
+            const int src = __builtin_ctzll(found);
+            const int n = __builtin_amdgcn_readlane(more, src);
+            return Pick{s0 + src, __builtin_amdgcn_readlane(ctx, src),
+                        left - (__builtin_amdgcn_readlane(incl, src) - n) + 1, n + 1};
+        }
+        left -= __builtin_amdgcn_readlane(incl, 63);
+    }
+    return Pick{-1, 0, 0, 0};
 }
 
 // Prompts: the `at`-th tile of 16 query rows of one KV head's batch, numbered sequence by
@@ -500,7 +544,9 @@ __global__ __launch_bounds__(NW * 64) void paged_decode_split_kernel(const AttnP
         ctx = __builtin_amdgcn_readfirstlane(decode_ctx(p, seq));
         if (ctx == 0) return;
     } else {
-        const Pick pick = p.num_seqs <= 64 ? pick_run<1>(p, lane, at, cut) : pick_run<kScanPer>(p, lane, at, cut);
+        const Pick pick = cut.mode == kCutLong ? pick_long(p, lane, at, cut)
+                          : p.num_seqs <= 64   ? pick_run<1>(p, lane, at, cut)
+                                               : pick_run<kScanPer>(p, lane, at, cut);
         if (pick.seq < 0) return;
         seq = pick.seq;
         ctx = pick.ctx;
@@ -819,9 +865,11 @@ int launch_nw(const AttnParams& p, hipStream_t stream) {
     constexpr bool kDear = sizeof(T) == 4 || D >= 80;
     cut.min_run = NW * (kDear ? 2 : 3) > kDecodePart / kUnit ? NW * (kDear ? 2 : 3) : kDecodePart / kUnit;
     cut.whole = NW * (kDear ? 4 : 6);
-    // No split either where the pairs fill the GPU by themselves, or where the counters or
-    // the scan do not reach.
-    if (p.ws_cnt && p.num_seqs <= kMaxScanSeqs && p.num_seqs * units < ((int64_t)1 << 31)) {
+    // Where the pairs fill the GPU by themselves, or the scan does not reach, contexts of less
+    // than 32 units a wave are not cut; none are where the counters do not reach.
+    cut.long_from = NW * 32;
+    const bool can = p.ws_cnt && p.num_seqs * units < ((int64_t)1 << 31);
+    if (can && p.num_seqs <= kMaxScanSeqs) {
         // Many pairs of long contexts: runs for two rounds, or the longest context would be
         // walked whole (250 sequences of 512-8192 tokens, 8/2 heads, bf16: 219 -> 189 us; 60 of
         // 16-2000, 12 heads of 64, fp32: 84 -> 72); with less to read the second round's start and
@@ -835,9 +883,16 @@ int launch_nw(const AttnParams& p, hipStream_t stream) {
         cut.slots2 = pairs < 2 * fits ? (int)(2 * fits / p.num_kv_heads) : 0;
     }
     const int slots = units >= cut.slots2_from ? cut.slots2 : cut.slots;
-    if (units > cut.whole && slots > 0) cut.mode = kCutRuns;
-    const int64_t grid =
-        cut.mode == kCutRuns ? (int64_t)(slots > p.num_seqs ? slots : p.num_seqs) * p.num_kv_heads : pairs;
+    int64_t grid = pairs;
+    if (units > cut.whole && slots > 0) {
+        cut.mode = kCutRuns;
+        grid = (int64_t)(slots > p.num_seqs ? slots : p.num_seqs) * p.num_kv_heads;
+    } else if (can && units >= cut.long_from && cut.slots == 0 && cut.slots2 == 0) {
+        cut.mode = kCutLong;
+        cut.slots = (int)(fits / p.num_kv_heads > 1 ? fits / p.num_kv_heads : 1);
+        cut.min_run = cut.long_from / 2;
+        grid = ((int64_t)p.num_seqs + cut.slots / 2) * p.num_kv_heads;
+    }
     if (grid > 0x7fffffff) return PKV_EUNSUPPORTED;
     paged_decode_split_kernel<T, D, NW, false><<<dim3((unsigned)grid), NW * 64, 0, stream>>>(p, cut);
     return check_launch("paged decode attention (split)");

@@ -99,11 +99,14 @@ def test_run_search_over_sequence_counts(n, dtype, fused):
 
 
 @pytest.mark.parametrize("n,kv,d,long", [
-    (350, 3, 32, 2200),      # as many pairs as the GPU holds: unsplit, 34 units a wave
+    (350, 3, 32, 2200),      # more pairs than the GPU holds, long contexts: runs for two rounds
+    (350, 3, 32, 1300),      # the same, none long enough: unsplit
     (1030, 1, 64, 300),      # more sequences than the search takes
+    (1100, 1, 64, 5000),     # the same, with contexts that would outlast the others
+    (600, 2, 128, 8192),     # two rounds of pairs, likewise
     (700, 6, 64, 90),        # many rounds of pairs: two waves a workgroup
-    (40, 3, 128, 9000)],     # runs of several chunks of block ids
-    ids=["unsplit", "many", "rounds", "long"])
+    (40, 3, 128, 9000)],     # a few long contexts, cut into short runs
+    ids=["two rounds", "unsplit", "many", "many, outliers", "outliers", "rounds", "long"])
 def test_unsplit_and_long_runs(n, kv, d, long):
     ctx = [1 + (29 * i) % 70 for i in range(n)]
     ctx[1], ctx[n // 2], ctx[n - 1] = long, long - 7, long + 13
@@ -187,7 +190,8 @@ def _captured(b, width, bound):
     (32, torch.float32, 4, 4, 64, 16, 40, 500, 1024), (8, torch.float32, 8, 1, 128, 16, 40, 250, 2048),
     (64, torch.float16, 12, 1, 64, 16, 40, 500, 1024), (43, torch.float16, 12, 1, 64, 16, 40, 512, 1024),
     (8, torch.float16, 12, 1, 64, 16, 17, 700, 1024), (64, torch.bfloat16, 8, 4, 128, 16, 30, 250, 1024),
-    (8, torch.bfloat16, 8, 4, 128, 16, 30, 520, 4096), (20, torch.float16, 1, 3, 80, 32, 30, 520, 4096),
+    (8, torch.bfloat16, 8, 4, 128, 16, 30, 520, 4096), (300, torch.bfloat16, 6, 2, 128, 16, 30, 3000, 8192),
+    (20, torch.float16, 1, 3, 80, 32, 30, 520, 4096),
     (130, torch.float16, 3, 1, 64, 16, 30, 600, 15000), (130, torch.float16, 3, 1, 64, 32, 30, 11000, 15000)])
 def test_a_captured_call_computes_the_eager_one(n, dtype, kv, group, d, bs, lo, hi, bound):
     """Bit for bit, whatever longest context the capture was told: what is cut, and where, comes
