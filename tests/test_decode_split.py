@@ -114,6 +114,28 @@ def test_unsplit_and_long_runs(n, kv, d, long):
            rows=[0, 1, 2, n // 2, n - 2, n - 1])
 
 
+@pytest.mark.parametrize("n,ctx,dtype,kv,group,d,bs", [
+    (8, 42000, torch.float16, 8, 1, 64, 16),         # runs of ~44 units a wave
+    (6, 50000, torch.bfloat16, 4, 2, 80, 32),        # ~38
+    (6, 60000, torch.float32, 2, 4, 128, 16),        # ~45
+    (1030, 4800, torch.float16, 1, 2, 64, 8)],       # past the search, none outlying: 75, uncut
+    ids=["fp16", "bf16", "fp32", "uncut"])
+@pytest.mark.parametrize("fused", [False, True], ids=["plain", "append"])
+def test_waves_of_more_units_than_they_hold_block_ids_of(n, ctx, dtype, kv, group, d, bs, fused):
+    """A wave holds the block ids of 32 units: these take the next ones and start their ring
+    anew. Sequences share blocks, but for the one that holds their new token."""
+    g = torch.Generator().manual_seed(n)
+    ctxs = [ctx + (13 * i) % 97 for i in range(n)]
+    need = [-(-c // bs) for c in ctxs]
+    shared = 600
+    tables = torch.randint(0, shared, (n, max(need) + 1), generator=g)
+    tables[torch.arange(n), torch.tensor(need) - 1] = shared + torch.randperm(n, generator=g)
+    rand = lambda *s: torch.randn(*s, generator=g).to(dtype)  # noqa: E731
+    b = dict(q=2 * rand(n, kv * group, d), k=rand(shared + n, bs, kv, d), v=rand(shared + n, bs, kv, d), tables=tables,
+             ctx=torch.tensor(ctxs), k_new=rand(n, kv, d), v_new=rand(n, kv, d))
+    _check(b, fused=fused, rows=[0, n // 2, n - 1])
+
+
 def test_contexts_of_zero_write_nothing_and_split_nothing():
     b = _batch([2500, 40, 17], dtype=torch.float16, d=128, bs=16, kv=2, group=4, seed=5)
     ref, _, _, _ = _run(b, fused=False)
