@@ -139,6 +139,7 @@ int launch_prefill_attention(const AttnParams& p, int dtype, hipStream_t stream)
 // batch's contexts itself (one load per sequence, replacing its own context and query
 // start loads); batches of more than kPrefillSortSeqs sequences keep index order.
 constexpr int kPrefillSortSeqs = 256;   // one sequence per thread
+constexpr int kPrefillWaveSeqs = 16;
 
 struct PrefillSeq {
     int seq;
@@ -209,11 +210,15 @@ __device__ __forceinline__ int split_count(int n_tiles, int splits, int split_ti
     return n < 1 ? 1 : (n < splits ? n : splits);
 }
 
-// This workgroup's item (256 threads, all of them call it: it holds two barriers). False:
+// This workgroup's item (256 threads, all of them call it: it may hold two barriers). False:
 // none. The hardware hands workgroup L to XCD L % 8 and each XCD has its own L2: items are
 // numbered row tile fastest, then split, then sequence (longest context first, as above),
 // then KV head, and XCD x takes the x-th contiguous eighth, so the workgroups that re-read
 // one sequence's K/V share an L2. Row tiles run last-first (the longest causal range first).
+// Every workgroup pays for this search before its first load, so it takes one LDS read a
+// sequence, in the waves that hold sequences only, and none in batches of up to 16 (three
+// reads a sequence before: 200 prompts of 1-8 tokens behind up to 500, 12 heads of 64, fp16,
+// 67 -> 52 us a call; 200 of 1-30 behind up to 200 55 -> 39; 8 of 16-500 17.4 -> 16.3).
 template <int ROWS, int KEYS>
 __device__ __forceinline__ bool prefill_item(const AttnParams& p, int block_size, PrefillItem& r) {
     const int t = (int)threadIdx.x;
@@ -238,70 +243,118 @@ __device__ __forceinline__ bool prefill_item(const AttnParams& p, int block_size
         r.ctx = (int)(c < cap ? c : cap);
         return r.row_tile * ROWS < r.q_len * (int)G;
     }
-    __shared__ int s_ctx[kPrefillSortSeqs];
-    __shared__ uint32_t s_tiles[kPrefillSortSeqs];   // row tiles
-    __shared__ uint32_t s_items[kPrefillSortSeqs];   // row tiles x splits
-    __shared__ PrefillItem s_pick;
-    __shared__ int s_found;
+    // Small batches: every wave for itself, without LDS or a barrier.
+    const bool in_wave = p.num_seqs <= kPrefillWaveSeqs;
+    const int lane = t & 63, s = in_wave ? lane : t;
     int64_t q_first = 0;
-    int q_len = 0, ctx = 0;
+    int q_len = 0, ctx = 0, key = -1;
     uint32_t tiles = 0, items = 0;
-    if (t < p.num_seqs) {
-        const int64_t c = p.ctx_lens[t];
-        q_first = p.qsl ? p.qsl[t] : t;
-        q_len = p.qsl ? (int)(p.qsl[t + 1] - q_first) : 1;
+    if (s < p.num_seqs) {
+        const int64_t c = p.ctx_lens[s];
+        q_first = p.qsl ? p.qsl[s] : s;
+        q_len = p.qsl ? (int)(p.qsl[s + 1] - q_first) : 1;
         ctx = (int)(c < cap ? c : cap);
         tiles = q_len > 0 ? ((uint32_t)q_len * G + ROWS - 1) / ROWS : 0;
         items = tiles * (uint32_t)split_count((ctx + KEYS - 1) / KEYS, p.splits, p.split_tiles);
-        s_ctx[t] = ctx;
-        s_tiles[t] = tiles;
-        s_items[t] = items;
+        // Longest context first, ties by index (contexts of 2^23 tokens count as tied).
+        const int k = ctx < 0 ? 0 : ctx < (1 << 23) ? ctx : (1 << 23) - 1;
+        key = k << 8 | (255 - s);
     }
-    if (t == 0) s_found = 0;
-    __syncthreads();
-    if (t < p.num_seqs) {
-        uint32_t before = 0, total = 0, tiles_before = 0, tiles_total = 0;
+    uint32_t before = 0, total = 0, tiles_before = 0, tiles_total = 0;
+    const bool cut = p.splits > 1;            // else a row tile is an item
+    if (in_wave) {
         for (int u = 0; u < p.num_seqs; ++u) {
-            const int cu = s_ctx[u];
-            const bool first = cu > ctx || (cu == ctx && u < t);
-            total += s_items[u];
-            tiles_total += s_tiles[u];
-            before += first ? s_items[u] : 0;
-            tiles_before += first ? s_tiles[u] : 0;
+            const bool first = __builtin_amdgcn_readlane(key, u) > key;
+            const uint32_t iu = (uint32_t)__builtin_amdgcn_readlane((int)items, u);
+            total += iu;
+            before += first ? iu : 0;
+            if (cut) {
+                const uint32_t tu = (uint32_t)__builtin_amdgcn_readlane((int)tiles, u);
+                tiles_total += tu;
+                tiles_before += first ? tu : 0;
+            }
         }
-        int splits = p.splits;
-        if (splits > 1 && (total * (uint32_t)p.num_kv_heads + 7) / 8 > gridDim.x / 8) {
+    }
+    // Whether this workgroup's item is the sequence's; then r is its item (but seq, q_len, ctx
+    // and q_first).
+    auto mine = [&]() {
+        r.splits = p.splits;
+        if (cut && (total * (uint32_t)p.num_kv_heads + 7) / 8 > gridDim.x / 8) {
             // Longer contexts than the grid was sized for: unsplit.
-            splits = 1;
+            r.splits = 1;
             total = tiles_total;
             before = tiles_before;
             items = tiles;
         }
         const uint32_t n_items = total * (uint32_t)p.num_kv_heads;
         const uint32_t item = xcd * ((n_items + 7) / 8) + at;
-        if (at < (n_items + 7) / 8 && item < n_items) {
-            const uint32_t kvh = item / total;
-            const uint32_t in_head = item - kvh * total;
-            if (in_head >= before && in_head - before < items) {
-                const uint32_t in_seq = in_head - before;
-                const uint32_t split = in_seq / tiles;
-                s_pick = PrefillItem{t, (int)kvh, (int)split, (int)(tiles - 1 - (in_seq - split * tiles)), q_len, ctx,
-                                     splits, q_first};
+        if (at >= (n_items + 7) / 8 || item >= n_items) return false;
+        const uint32_t kvh = item / total;
+        const uint32_t in_seq = item - kvh * total - before;     // wraps below the sequence's first
+        if (in_seq >= items) return false;
+        r.kvh = (int)kvh;
+        r.split = (int)(in_seq / tiles);
+        r.row_tile = (int)(tiles - 1 - in_seq % tiles);
+        return true;
+    };
+    bool found;
+    if (in_wave) {
+        const uint64_t lanes = __builtin_amdgcn_ballot_w64(mine());
+        found = lanes != 0;
+        const int src = found ? __builtin_ctzll(lanes) : 0;
+        r = PrefillItem{src,
+                        __builtin_amdgcn_readlane(r.kvh, src),
+                        __builtin_amdgcn_readlane(r.split, src),
+                        __builtin_amdgcn_readlane(r.row_tile, src),
+                        __builtin_amdgcn_readlane(q_len, src),
+                        __builtin_amdgcn_readlane(ctx, src),
+                        __builtin_amdgcn_readlane(r.splits, src),
+                        readlane64(q_first, src)};
+    } else {
+        __shared__ uint4 s_seq[kPrefillSortSeqs];   // one LDS read a step of the loop below
+        __shared__ PrefillItem s_pick;
+        __shared__ int s_found;
+        if (t == 0) s_found = 0;
+        if (t < p.num_seqs) s_seq[t] = make_uint4((uint32_t)key, items, tiles, 0u);
+        __syncthreads();
+        if (t < p.num_seqs) {
+            if (cut) {
+#pragma unroll 4
+                for (int u = 0; u < p.num_seqs; ++u) {
+                    const uint4 o = s_seq[u];
+                    const bool first = (int)o.x > key;
+                    total += o.y;
+                    tiles_total += o.z;
+                    before += first ? o.y : 0;
+                    tiles_before += first ? o.z : 0;
+                }
+            } else {
+#pragma unroll 4
+                for (int u = 0; u < p.num_seqs; ++u) {
+                    const uint2 o = *reinterpret_cast<const uint2*>(&s_seq[u]);
+                    total += o.y;
+                    before += (int)o.x > key ? o.y : 0;
+                }
+            }
+            if (mine()) {
+                s_pick = PrefillItem{t, r.kvh, r.split, r.row_tile, q_len, ctx, r.splits, q_first};
                 s_found = 1;
             }
         }
+        __syncthreads();
+        found = s_found != 0;
+        r = s_pick;
     }
-    __syncthreads();
-    if (!s_found) return false;
+    if (!__builtin_amdgcn_readfirstlane((int)found)) return false;
     // Uniform: into scalar registers.
-    r.seq = __builtin_amdgcn_readfirstlane(s_pick.seq);
-    r.kvh = __builtin_amdgcn_readfirstlane(s_pick.kvh);
-    r.split = __builtin_amdgcn_readfirstlane(s_pick.split);
-    r.row_tile = __builtin_amdgcn_readfirstlane(s_pick.row_tile);
-    r.q_len = __builtin_amdgcn_readfirstlane(s_pick.q_len);
-    r.ctx = __builtin_amdgcn_readfirstlane(s_pick.ctx);
-    r.splits = __builtin_amdgcn_readfirstlane(s_pick.splits);
-    r.q_first = readlane64(s_pick.q_first, 0);
+    r.seq = __builtin_amdgcn_readfirstlane(r.seq);
+    r.kvh = __builtin_amdgcn_readfirstlane(r.kvh);
+    r.split = __builtin_amdgcn_readfirstlane(r.split);
+    r.row_tile = __builtin_amdgcn_readfirstlane(r.row_tile);
+    r.q_len = __builtin_amdgcn_readfirstlane(r.q_len);
+    r.ctx = __builtin_amdgcn_readfirstlane(r.ctx);
+    r.splits = __builtin_amdgcn_readfirstlane(r.splits);
+    r.q_first = readlane64(r.q_first, 0);
     return true;
 }
 

@@ -127,6 +127,23 @@ def test_fp32_prompts_over_sequence_counts(n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [15, 16, 17, 64, 65, 200, 256, 257])
+@pytest.mark.parametrize("split", [False, True], ids=["whole", "split"])
+def test_prompts_over_sequence_counts(n, split):
+    """Items found within a wave and through LDS, on grids that are not a multiple of 8 items,
+    with prompts of no token among them; with and without long contexts to split (257
+    sequences never are)."""
+    lengths = [(20 + (13 * i) % 90, (7 * i) % 19) for i in range(n)]
+    lengths[0], lengths[n // 2], lengths[n - 1] = (1500 if split else 150, 33), (40, 40), (3000 if split else 17, 1)
+    b = _batch(lengths, dtype=torch.float16, d=64, bs=16, kv=1, group=3, seed=n)
+    assert (_split_bytes(b) > 0) == (split and n <= 256)
+    _check(b, fused=True)
+    if split:       # the host's lengths only balance the launch: a grid without room for the splits
+        told = torch.where(b["ctx"] > 1000, torch.tensor(1100), b["ctx"])
+        _check(b, fused=False, told=told)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("told", [[1100] * 6, [3000, 40, 70, 5, 43, 2]], ids=["shorter", "one long"])
 def test_split_contexts_longer_than_told_are_attended_whole(told):
     b = _batch(LONG, dtype=torch.bfloat16, d=128, bs=16, kv=2, group=4, seed=11)
