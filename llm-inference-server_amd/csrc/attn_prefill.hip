@@ -742,11 +742,6 @@ SplitPlan prefill_split_plan(int64_t num_seqs, int64_t num_heads, int64_t num_kv
     if (num_seqs < 1 || num_seqs > kPrefillSortSeqs || num_tokens < 1 || num_kv_heads < 1 || head_dim < 1) return plan;
     const int64_t group = num_heads / num_kv_heads;
     const int64_t slots = head_dim >= 112 ? 512 : head_dim >= 80 ? 768 : 1024;
-    // Without the lengths (a decode call): contexts spread evenly up to the bound.
-    auto tiles_of = [&](int64_t i) {
-        return ceil_div(ctx ? ctx[i] : max_context_len * (2 * i + 1) / (2 * num_seqs), kKT);
-    };
-    auto rows_of = [&](int64_t i) { return (qlen ? qlen[i] : 1) * group; };
     auto launch_us = [&](int64_t wgs, int64_t longest, int64_t work) {
         const float full = wgs < slots ? (float)wgs / slots : 1.f;
         const float tile = kTileAlone + (kTileFull - kTileAlone) * full;
@@ -755,37 +750,68 @@ SplitPlan prefill_split_plan(int64_t num_seqs, int64_t num_heads, int64_t num_kv
         const float all = (work * tile + wgs * kStart) / slots + 0.5f * one;
         return all > one ? all : one;
     };
-    int64_t wgs = 0, work = 0, longest = ctx ? 0 : ceil_div(max_context_len, kKT);
+    // Per sequence with work: key tiles, workgroups unsplit, query rows of all KV heads.
+    static_assert(kPrefillSortSeqs % 4 == 0, "");
+    double tiles[kPrefillSortSeqs], per_split[kPrefillSortSeqs], rows_of[kPrefillSortSeqs];
+    int live = 0;
+    int64_t wgs = 0, work = 0, longest = ctx ? 0 : (max_context_len + kKT - 1) / kKT;
     for (int64_t i = 0; i < num_seqs; ++i) {
-        const int64_t t = tiles_of(i), w = ceil_div(rows_of(i), kRows) * num_kv_heads;
-        if (t <= 0 || w <= 0) continue;
+        // Without the lengths (a decode call): contexts spread evenly up to the bound.
+        const int64_t c = ctx ? ctx[i] : max_context_len * (2 * i + 1) / (2 * num_seqs);
+        const int64_t r = (qlen ? qlen[i] : 1) * group;
+        if (c <= 0 || r <= 0) continue;
+        const int64_t t = c < ((int64_t)1 << 36) ? (c + kKT - 1) / kKT : (int64_t)1 << 30;
+        const int64_t w = (r + kRows - 1) / kRows * num_kv_heads;
         wgs += w;
         work += w * t;
         longest = longest > t ? longest : t;
         if (wgs >= 2 * slots) return plan;       // the GPU is full, and stays so
+        tiles[live] = (double)t;
+        per_split[live] = (double)w;
+        rows_of[live++] = (double)(r * num_kv_heads);
     }
     if (longest * kKT <= kSplitMinContext) return plan;
+    for (int i = live; i % 4; ++i) {             // nothing, for the loop below
+        tiles[i] = 1.0;
+        per_split[i] = rows_of[i] = 0.0;
+    }
     const int64_t rows = num_tokens * num_heads;
     float best = kWorth * launch_us(wgs, longest, work);
     for (const int64_t run : kRuns) {
         if (run >= longest) break;
         const int64_t splits = ceil_div(longest, run);
         if (rows * splits * (head_dim + 2) * 4 > kMaxBytes) continue;
-        int64_t n = 0, parts = 0, top = 0;
-        for (int64_t i = 0; i < num_seqs; ++i) {
-            const int64_t t = tiles_of(i), w = ceil_div(rows_of(i), kRows) * num_kv_heads;
-            if (t <= 0 || w <= 0) continue;
-            const int64_t s = ceil_div(t, run);
-            n += w * s;
-            top = top > ceil_div(t, s) ? top : ceil_div(t, s);
-            if (s > 1) parts += rows_of(i) * num_kv_heads * s;
-        }
-        const float us = launch_us(n, top, work) + kMerge + parts * (head_dim + 2) * 4 / kBytesPerUs;
+        // The least that it can take, from the sums alone: mostly enough to pass on.
+        const int64_t least = ceil_div(work, run) > wgs ? ceil_div(work, run) : wgs;
+        if (launch_us(least, ceil_div(longest, splits), work) + kMerge >= best) continue;
+        // In doubles and four sums, for the host's vector units (22 run lengths over 256
+        // sequences: 30-50 us in 64-bit integers); all are whole numbers below 2^53.
+        const double inv = 1.0 / (double)run, above = (double)run - 0.5;
+        auto splits_of = [&](double t) { return (double)(int32_t)((t + above) * inv); };
+        double ns[4] = {}, ps[4] = {};
+        for (int i = 0; i < live; i += 4)
+            for (int j = 0; j < 4; ++j) {
+                // ceil(tiles / run): the half keeps the product off whole numbers.
+                const double s = splits_of(tiles[i + j]);
+                ns[j] += per_split[i + j] * s;
+                ps[j] += s > 1 ? rows_of[i + j] * s : 0.0;
+            }
+        const double n = ns[0] + ns[1] + ns[2] + ns[3], parts = ps[0] + ps[1] + ps[2] + ps[3];
+        // The longest of the even splits, rounded up; no split is longer than the run.
+        double top = 0;
+        for (int i = 0; i < live && top <= (double)run - 1.0; ++i)
+            if (tiles[i] > top) {
+                const double even = tiles[i] / splits_of(tiles[i]);
+                top = even > top ? even : top;
+            }
+        top += 1.0 - 1e-9;
+        const float us = launch_us((int64_t)n, (int64_t)top, work) + kMerge +
+                         (int64_t)parts * (head_dim + 2) * 4 / kBytesPerUs;
         if (us >= best) continue;
         best = us;
         plan.splits = (int)splits;
         plan.split_tiles = (int)run;
-        plan.items = ctx ? n : wgs * splits;     // lengths unknown: room for all of them at the bound
+        plan.items = ctx ? (int64_t)n : wgs * splits;     // lengths unknown: room for all of them at the bound
     }
     if (plan.splits == 1) return plan;
     auto round256 = [](int64_t b) { return ceil_div(b, 256) * 256; };

@@ -10,7 +10,9 @@ of the shapes without a decode kernel run through it too.
 from __future__ import annotations
 
 import ctypes
+import random
 
+import numpy as np
 import pytest
 import torch
 
@@ -201,3 +203,52 @@ def test_slots_of_a_block_in_reverse_order(d, bs, dtype, lengths):
     torch.cuda.synchronize()
     ref = oracle_gather(b["q"], b["k"], b["v"], b["tables"], b["ctx"], b["ql"], d ** -0.5)
     torch.testing.assert_close(out.cpu(), ref, atol=TOL[dtype], rtol=TOL[dtype])
+
+
+def _planned_bytes(ctx, ql, heads, kv, d):
+    """The workspace of the cheapest run length in the launch model of csrc/attn_prefill.hip,
+    computed sequence by sequence in whole numbers."""
+    up = lambda a, b: -(-a // b)  # noqa: E731
+    group, slots = heads // kv, 512 if d >= 112 else 768 if d >= 80 else 1024
+    live = [(up(c, 64), up(q * group, 128) * kv, q * heads) for c, q in zip(ctx, ql) if c > 0 and q > 0]
+    f = np.float32
+
+    def us(wgs, longest, work):
+        tile = f(1.1) + (f(1.9) - f(1.1)) * (f(wgs) / f(slots) if wgs < slots else f(1))
+        one = f(longest) * tile + f(6)
+        return one if wgs <= slots else max(one, (f(work) * tile + f(wgs) * f(6)) / f(slots) + f(0.5) * one)
+
+    wgs, work, longest = sum(w for _, w, _ in live), sum(t * w for t, w, _ in live), max(t for t, _, _ in live)
+    if len(ctx) > 256 or wgs >= 2 * slots or longest * 64 <= 1024:
+        return 0
+    rows, splits, best = sum(ql) * heads, 1, f(0.85) * us(wgs, longest, work)
+    for run in (4, 5, 6, 8, 10, 12, 14, 17, 20, 24, 28, 34, 40, 48, 56, 68, 80, 96, 112, 136, 160, 192):
+        if run >= longest:
+            break
+        n = up(longest, run)
+        if rows * n * (d + 2) * 4 > 128 << 20:
+            continue
+        s = [up(t, run) for t, _, _ in live]
+        parts = sum(r * m for (_, _, r), m in zip(live, s) if m > 1)
+        cost = us(sum(w * m for (_, w, _), m in zip(live, s)), max(up(t, m) for (t, _, _), m in zip(live, s)), work)
+        cost = cost + f(4) + f(parts * (d + 2) * 4) / f(4.5e6)
+        if cost < best:
+            best, splits = cost, n
+    r256 = lambda b: up(b, 256) * 256  # noqa: E731
+    return 0 if splits == 1 else 256 * 1024 + r256(rows * 4) + r256(rows * splits * 8) + r256(rows * splits * d * 4)
+
+
+def test_split_plan_is_the_cheapest_run_length():
+    size = native.lib().pkv_paged_attention_prefill_workspace_bytes
+    rng, split = random.Random(7), 0
+    for _ in range(600):
+        n, kv, d = rng.choice([1, 2, 3, 5, 16, 64, 101, 256]), rng.choice([1, 2, 4, 8]), rng.choice([32, 80, 128])
+        heads, q, hi = kv * rng.choice([1, 3, 4, 17]), rng.choice([1, 4, 40, 300]), rng.choice([1500, 8192, 131072])
+        ql = [rng.randint(n > 1, q) for _ in range(n)]
+        ql[0] = max(ql[0], 1)
+        ctx = [max(m, rng.randint(1, hi)) for m in ql]
+        arr = lambda v: (ctypes.c_int64 * n)(*v)  # noqa: E731
+        need = size(n, heads, kv, d, sum(ql), arr(ctx), arr(ql))
+        assert need == _planned_bytes(ctx, ql, heads, kv, d), (n, heads, kv, d, ql, ctx)
+        split += need > 0
+    assert split > 200
