@@ -269,6 +269,9 @@ int64_t pkv_paged_attention_prefill_workspace_bytes(int64_t num_seqs, int64_t nu
                                                     int64_t head_dim, int64_t num_tokens,
                                                     const int64_t* host_context_lens,
                                                     const int64_t* host_query_lens);
+/* 1 if pools of this block size, head_dim and dtype can have their contexts split at all
+ * (the size above does not know them), else 0: no workspace is of use. At most 128 MiB are. */
+int pkv_paged_attention_prefill_can_split(int64_t block_size, int64_t head_dim, int dtype);
 int pkv_paged_attention_prefill_split(
     void* out, int64_t out_stride_t, int64_t out_stride_h,
     const void* query, int64_t q_stride_t, int64_t q_stride_h,

@@ -78,6 +78,8 @@ int launch_decode_f32(const AttnParams& p, hipStream_t stream);
 // True when launch_prefill_attention runs the MFMA kernel for these parameters (with
 // p.app_* set: including the fused append, whose source rows must be 16-byte aligned).
 bool prefill_tuned(const AttnParams& p, int dtype);
+// What it asks of the shape alone.
+bool prefill_shape(int64_t block_size, int64_t head_dim, int dtype);
 
 // How the prefill MFMA kernel cuts a batch's contexts (splits = 1: it does not), and the
 // workspace that takes: runs of at most split_tiles 64-key tiles, at most `splits` of them

@@ -475,6 +475,10 @@ extern "C" int64_t pkv_paged_attention_prefill_workspace_bytes(int64_t num_seqs,
     return plan.splits > 1 ? kMergeCounterBytes + plan.total() : 0;
 }
 
+extern "C" int pkv_paged_attention_prefill_can_split(int64_t block_size, int64_t head_dim, int dtype) {
+    return prefill_shape(block_size, head_dim, dtype) ? 1 : 0;
+}
+
 extern "C" int pkv_paged_attention_prefill_split(
     void* out, int64_t out_stride_t, int64_t out_stride_h, const void* query, int64_t q_stride_t,
     int64_t q_stride_h, void* k_pool, void* v_pool, int64_t pool_stride_block, int64_t pool_stride_slot,

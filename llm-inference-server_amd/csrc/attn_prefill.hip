@@ -736,7 +736,7 @@ SplitPlan prefill_split_plan(int64_t num_seqs, int64_t num_heads, int64_t num_kv
                              int64_t num_tokens, const int64_t* ctx, const int64_t* qlen, int64_t max_context_len) {
     constexpr float kStart = 6.f, kTileAlone = 1.1f, kTileFull = 1.9f, kMerge = 4.f, kBytesPerUs = 4.5e6f;
     constexpr float kWorth = 0.85f;              // the gain that a split has to promise
-    constexpr int64_t kMaxBytes = 128 << 20;
+    constexpr int64_t kMaxBytes = 128 << 20;     // of workspace, the counters' room and roundings included
     static const int kRuns[] = {4, 5, 6, 8, 10, 12, 14, 17, 20, 24, 28, 34, 40, 48, 56, 68, 80, 96, 112, 136, 160, 192};
     SplitPlan plan{1, 0x7fffffff, 0, 0, 0, 0};
     if (num_seqs < 1 || num_seqs > kPrefillSortSeqs || num_tokens < 1 || num_kv_heads < 1 || head_dim < 1) return plan;
@@ -780,7 +780,7 @@ SplitPlan prefill_split_plan(int64_t num_seqs, int64_t num_heads, int64_t num_kv
     for (const int64_t run : kRuns) {
         if (run >= longest) break;
         const int64_t splits = ceil_div(longest, run);
-        if (rows * splits * (head_dim + 2) * 4 > kMaxBytes) continue;
+        if (kMergeCounterBytes + 3 * 256 + rows * 4 + rows * splits * (head_dim + 2) * 4 > kMaxBytes) continue;
         // The least that it can take, from the sums alone: mostly enough to pass on.
         const int64_t least = ceil_div(work, run) > wgs ? ceil_div(work, run) : wgs;
         if (launch_us(least, ceil_div(longest, splits), work) + kMerge >= best) continue;
@@ -821,10 +821,14 @@ SplitPlan prefill_split_plan(int64_t num_seqs, int64_t num_heads, int64_t num_kv
     return plan;
 }
 
+bool prefill_shape(int64_t block_size, int64_t head_dim, int dtype) {
+    if (block_size < 8 || (block_size & (block_size - 1))) return false;
+    if (head_dim % 16 || head_dim < 32 || head_dim > 128) return false;
+    return dtype == PKV_FLOAT16 || dtype == PKV_BFLOAT16;
+}
+
 bool prefill_tuned(const AttnParams& p, int dtype) {
-    if (p.block_shift < 3) return false;
-    if (p.head_dim % 16 || p.head_dim < 32 || p.head_dim > 128) return false;
-    if (dtype != PKV_FLOAT16 && dtype != PKV_BFLOAT16) return false;
+    if (!prefill_shape(p.block_size, p.head_dim, dtype)) return false;
     // The kernel's offsets are unsigned (strides too large for 32 bits take its per-row path).
     if (p.ss < 0) return false;
     // The kernel masks to -inf and takes the maximum before it scales: scale > 0 only.

@@ -162,6 +162,7 @@ def _batch_facts(context_lens: torch.Tensor, query_lens: torch.Tensor, block_siz
         "all_decode": bool((hql == 1).all()),
         "max_ctx": longest,
         "max_q": int(hql.max()) if hql.size else 0,
+        "split_ws": {},  # split prefill's workspace bytes by shape, planned on first use
         "qsl": {},  # device query_start_loc by (device, stream), built on first prefill use
     }
     if key is not None:
@@ -319,9 +320,16 @@ def paged_attention_hip_launch(
     qsl = getattr(query_lens, _QSL_ATTR, None)
     if qsl is None:
         qsl = _query_start(facts, context_lens, dev, stream)
-    # Workspace for split contexts (0 bytes: a batch that is not split).
+    # Workspace for split contexts (0 bytes: a batch that is not split), planned by a step's
+    # first layer.
     lens = (facts["hctx"].data_ptr(), facts["hql"].data_ptr())
-    ws_bytes = L.pkv_paged_attention_prefill_workspace_bytes(n_seqs, n_heads, n_kv, head_dim, n_tok, *lens)
+    shape = (n_heads, n_kv, head_dim, block_size, dt)
+    ws_bytes = facts["split_ws"].get(shape)
+    if ws_bytes is None:
+        ws_bytes = 0
+        if L.pkv_paged_attention_prefill_can_split(block_size, head_dim, dt):
+            ws_bytes = L.pkv_paged_attention_prefill_workspace_bytes(n_seqs, n_heads, n_kv, head_dim, n_tok, *lens)
+        facts["split_ws"][shape] = ws_bytes
     ws_ptr, ws_size = None, 0
     if ws_bytes:
         ws = _WORKSPACES.partials(dev, stream, ws_bytes)

@@ -101,6 +101,7 @@ SIGNATURES: dict[str, tuple] = {
          _ptr],
     ),
     "pkv_paged_attention_prefill_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i64, _ptr, _ptr]),
+    "pkv_paged_attention_prefill_can_split": (_int, [_i64, _i64, _int]),
     "pkv_paged_attention_prefill_split": (
         _int,
         [_ptr, _i64, _i64,

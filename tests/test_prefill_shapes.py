@@ -17,7 +17,7 @@ import pytest
 import torch
 
 from inference_server import native
-from inference_server.core.attention_hip import attach_host, paged_attention_hip_launch
+from inference_server.core.attention_hip import _WORKSPACES, attach_host, paged_attention_hip_launch
 from oracle.gather import paged_attention_gather as oracle_gather
 from oracle.kvops import kv_append
 
@@ -120,6 +120,19 @@ def test_split_contexts(d, bs, kv, group, dtype, fused):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,bs,grows", [(torch.float32, 16, 0), (torch.bfloat16, 12, 0), (torch.bfloat16, 16, 1)])
+def test_only_batches_that_can_split_grow_the_workspace(dtype, bs, grows):
+    b = _batch([(6000, 30)], dtype=dtype, d=64, bs=bs, kv=1, group=4)
+    torch.cuda.synchronize()
+    _WORKSPACES.reset()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        _check(b, fused=False)
+    held = [key for key in _WORKSPACES._bufs if key[1] == stream.cuda_stream]
+    assert len(held) == grows
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n", [64, 65, 200])
 def test_fp32_prompts_over_sequence_counts(n):
     """Tiles found across lanes, several sequences a lane, prompts of no token among them."""
@@ -205,6 +218,14 @@ def test_slots_of_a_block_in_reverse_order(d, bs, dtype, lengths):
     torch.testing.assert_close(out.cpu(), ref, atol=TOL[dtype], rtol=TOL[dtype])
 
 
+def test_shapes_that_cannot_be_split_take_no_workspace():
+    can = native.lib().pkv_paged_attention_prefill_can_split
+    fp16, bf16, fp32 = native.PKV_FLOAT16, native.PKV_BFLOAT16, native.PKV_FLOAT32
+    assert all(can(bs, d, t) for bs in (8, 16, 128) for d in (32, 48, 128) for t in (fp16, bf16))
+    assert not any(can(16, d, fp32) for d in (32, 64, 128))
+    assert not any(can(bs, 64, fp16) for bs in (0, 1, 4, 6, 24, 48)) and not any(can(16, d, bf16) for d in (8, 40, 144))
+
+
 def _planned_bytes(ctx, ql, heads, kv, d):
     """The workspace of the cheapest run length in the launch model of csrc/attn_prefill.hip,
     computed sequence by sequence in whole numbers."""
@@ -226,7 +247,7 @@ def _planned_bytes(ctx, ql, heads, kv, d):
         if run >= longest:
             break
         n = up(longest, run)
-        if rows * n * (d + 2) * 4 > 128 << 20:
+        if 256 * 1024 + 3 * 256 + rows * 4 + rows * n * (d + 2) * 4 > 128 << 20:
             continue
         s = [up(t, run) for t, _, _ in live]
         parts = sum(r * m for (_, _, r), m in zip(live, s) if m > 1)
@@ -250,5 +271,6 @@ def test_split_plan_is_the_cheapest_run_length():
         arr = lambda v: (ctypes.c_int64 * n)(*v)  # noqa: E731
         need = size(n, heads, kv, d, sum(ql), arr(ctx), arr(ql))
         assert need == _planned_bytes(ctx, ql, heads, kv, d), (n, heads, kv, d, ql, ctx)
+        assert need <= 128 << 20
         split += need > 0
     assert split > 200
