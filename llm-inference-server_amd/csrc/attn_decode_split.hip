@@ -856,15 +856,17 @@ int launch_nw(const AttnParams& p, hipStream_t stream) {
     Cut cut{};
     // Units a wave that a run has at least (and a workspace slot's tokens), and that a context
     // may have before it is worth the merge: 2 and 4 where a unit is dear, fp32 products and
-    // rows of 160 bytes up, else 3 and 6. Replayed from graphs, us a call, 2 and 4 vs 3 and 6
-    // vs 4 and 8: 32/8 heads of 128, bf16, 4 sequences of 16-1000 tokens 9.9 / - / 13.6, 16 of
-    // them 11.1 / - / 14.8; fp32, 16/4 heads of 64, 8 of 16-1000 9.6 / - / 16.5; over 40 batches
-    // of 1-64 sequences of 300-8000 tokens (geometric mean, relative): 8/4 heads of 80 0.93 /
-    // 0.94 / 1.02, 16/4 of 96 0.95 / 0.97 / 1.04, 12 heads of 64, fp16, 1.02 / 1.01 / 1.04, 8/4
-    // of 64 1.04 / 1.03 / 1.05.
+    // rows of 160 bytes up, else 3 and 8. Replayed from graphs, us a call, 2 and 4 vs 4 and 8:
+    // 32/8 heads of 128, bf16, 4 sequences of 16-1000 tokens 9.9 vs 13.6, 16 of them 11.1 vs
+    // 14.8; fp32, 16/4 heads of 64, 8 of 16-1000 9.6 vs 16.5. Over 40 batches of 1-64 sequences
+    // of 300-8000 tokens (geometric means, relative), 2 and 4 / 3 and 6 / 3 and 8: 8/4 heads of
+    // 80 0.93 / 0.94 / 1.01, 16/4 of 96 0.95 / 0.97 / 1.02, 12 heads of 64, fp16, 1.02 / 1.01 /
+    // 1.03, 8/4 of 64 1.04 / 1.03 / 1.04; but a step captured for GPT-2's 1024 positions is
+    // told of no longer context than 8 units a wave and spares the search at that bound (12
+    // layers of 8 sequences 161 vs 166 us with 6).
     constexpr bool kDear = sizeof(T) == 4 || D >= 80;
     cut.min_run = NW * (kDear ? 2 : 3) > kDecodePart / kUnit ? NW * (kDear ? 2 : 3) : kDecodePart / kUnit;
-    cut.whole = NW * (kDear ? 4 : 6);
+    cut.whole = NW * (kDear ? 4 : 8);
     // Where the pairs fill the GPU by themselves, or the scan does not reach, contexts of less
     // than 32 units a wave are not cut; none are where the counters do not reach.
     cut.long_from = NW * 32;
