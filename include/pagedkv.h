@@ -132,11 +132,17 @@ int64_t pkv_paged_attention_decode_workspace_bytes(int64_t num_seqs, int64_t num
  * and at most 1024 sequences, run the persistent MFMA kernel (equal runs of 16-key
  * blocks per workgroup, then a small merge kernel for the sequences the runs cut);
  * fp32 batches with one or two heads of 64 a KV head (block size 16) run the register kernel
- * and its merge kernel; any other batch of head_dims 32..128 (multiples of 16), groups up to 16 and
- * power-of-two block sizes from 8 runs the one-launch MFMA kernel (contexts cut into runs
- * that fit the GPU, merged in place), 16-bit groups above 16 the prefill kernel, the rest
- * the generic kernel. All launch on the same stream; calls that overlap in time (different
- * streams) need distinct workspaces. */
+ * and its merge kernel; any other batch of head_dims 32..128 (multiples of 16), groups up
+ * to 16 and power-of-two block sizes from 8 runs the one-launch MFMA kernel (contexts cut
+ * into runs that fit the GPU, merged in place), 16-bit groups above 16 the prefill kernel,
+ * the rest the generic kernel.
+ * The persistent and the one-launch kernel cut a context by all lengths of the batch, so the
+ * rounding of a sequence's output can change with the batch that it is in. It does not
+ * change from call to call, nor with max_context_len but where that chooses the persistent
+ * kernel, or the one-launch kernel's workgroups of two waves (at least four rounds of
+ * (sequence, KV head) pairs, 512 tokens at most).
+ * All launch on the same stream; calls that overlap in time (different streams) need
+ * distinct workspaces. */
 int pkv_paged_attention_decode(
     void* out, int64_t out_stride_t, int64_t out_stride_h,
     const void* query, int64_t q_stride_t, int64_t q_stride_h,
@@ -260,7 +266,8 @@ int pkv_paged_attention_prefill_append(
  * else the append of pkv_paged_attention_prefill_append. host_context_lens /
  * host_query_lens: the lengths in HOST memory, int64 [num_seqs], read during the call;
  * they only decide whether and how to split (a context longer than told is still attended
- * to whole); NULL means no split. workspace: at least
+ * to whole), and so the rounding of an output, which can change with the batch that a
+ * sequence is in; NULL means no split. workspace: at least
  * pkv_paged_attention_prefill_workspace_bytes() bytes for the same sizes and lengths, else
  * (or NULL) the batch is not split. Its first 256 KiB are never touched and the rest needs
  * no initialisation, so one buffer can serve this call and the decode calls on a stream;

@@ -1,6 +1,8 @@
 // fp32 paged attention on 16-key tiles (one block each) over a float32 pool with block
-// size 16 and head_dim 64 or 128: prefill-entry batches of 1-token rows, and prefill
-// batches the fp32 MFMA kernel (attn_prefill_f32.hip) declines. Replaces, for float32 pools, the reference's ragged loop and batched decode
+// size 16 and head_dim 64 or 128: what both fp32 MFMA kernels decline, prefill-entry batches
+// of more sequences than the 16-row form of attn_decode_split.hip searches (1024) that
+// attn_prefill_f32.hip does not take either (1-token rows, scales that are not positive).
+// Replaces, for float32 pools, the reference's ragged loop and batched decode
 // (inference_server/core/attention.py:130-187) where the only other kernel walks the
 // keys one at a time.
 //

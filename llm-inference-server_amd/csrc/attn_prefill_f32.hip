@@ -334,10 +334,11 @@ int launch_d(const AttnParams& p, hipStream_t stream) {
 
 int launch_prefill_f32_mfma(const AttnParams& p, hipStream_t stream) {
     if (!p.qsl || p.app_k || p.block_size != kBS || (p.head_dim != 64 && p.head_dim != 128)) return PKV_EUNSUPPORTED;
-    // Batches of 1-token rows only stay on the tiled fp32 kernel: a 32-query tile would
-    // carry one query (64 rows of ctx 100-2000, d64: 341 vs 222 us). Any longer row and
-    // the tiles pay (8 x 128-token prefills + 56 one-token rows: 360 vs 835 us; config 1's
-    // 8 prompts: 24 vs 51 us; 16 x 512-token chunks at d128, GQA 4: 2.46 vs 13.5 ms).
+    // Batches of 1-token rows only go to the 16-row form of attn_decode_split.hip (or, past its
+    // 1024 sequences, to the tiled kernel): a 32-query tile would carry one query (64 rows of ctx
+    // 100-2000, d64: 341 us here, 222 on the tiled kernel). Any longer row and the tiles pay
+    // against the tiled kernel (8 x 128-token prefills + 56 one-token rows: 360 vs 835 us; 16 x
+    // 512-token chunks at d128, GQA 4: 2.46 vs 13.5 ms).
     if (p.max_query_len <= 1) return PKV_EUNSUPPORTED;
     if (p.group != 1 && p.group != 2 && p.group != 4 && p.group != 8) return PKV_EUNSUPPORTED;
     if (p.num_blocks < 1) return PKV_EUNSUPPORTED;

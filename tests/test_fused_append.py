@@ -10,9 +10,8 @@ pool and output. Decode cases cover both partition lengths the launch picks, hea
 boundaries. Prefill cases cover fresh prompts, chunks onto a cached prefix that ends
 inside a block, mixed prefill + decode batches, GQA groups that split a KV head over
 several workgroups, and new slots that hold NaN before the call (a read of a slot this
-launch is still writing would show). fp32, odd-stride sources and GQA groups with no
-tuned instance (3, 6) take the separate append launch inside the call. The executor's steps are checked eager and replayed
-from graphs.
+launch is still writing would show). Rows off 16 bytes, and fp32 prompts, take the separate
+append launch inside the call. The executor's steps are checked eager and replayed from graphs.
 """
 
 from __future__ import annotations
@@ -73,9 +72,9 @@ CASES = [
     (64, 8, 4, 128, 3000, torch.bfloat16, (1, 192, 193, 768, 769)), # long partitions
     (40, 4, 1, 64, 5000, torch.float16, (2, 191, 192, 1536, 1537)),
     (8, 2, 2, 64, 700, torch.bfloat16, ()),
-    (5, 2, 4, 128, 600, torch.float32, (1, 100)),                    # fp32: append launch first
-    (6, 2, 3, 128, 900, torch.bfloat16, (1, 300)),                   # group 3: no tuned instance
-    (5, 2, 6, 64, 700, torch.float16, (2, 257)),                     # group 6: no tuned instance
+    (5, 2, 4, 128, 600, torch.float32, (1, 100)),                    # fp32
+    (6, 2, 3, 128, 900, torch.bfloat16, (1, 300)),                   # groups that are no power of two
+    (5, 2, 6, 64, 700, torch.float16, (2, 257)),  
 ]
 
 
