@@ -342,7 +342,7 @@ def config1_fp32(steps: int, warmup: int) -> dict:
         "causal_flops": w.flops,
         "decode_algorithmic_bytes": w.decode_bytes,
         "note": "GPT-2 shape fp32 (12 heads, d64, block 16): config 1's 8 prompts prefilled in one call "
-                "and one decode step over them 16 tokens later, both on the one-launch fp32 MFMA kernel",
+                "(one-launch fp32 MFMA kernel) and one decode step over them 16 tokens later (register kernel)",
     }
 
 

@@ -39,12 +39,13 @@
 // Numerics follow the reference gather path (core/attention.py:130-153) as the persistent
 // kernel does: scores rounded to the pool dtype before and after the scale, softmax in fp32,
 // probabilities exp2(s - m) rounded to the pool dtype before P·V, fp32 accumulation, one
-// rounding of the output. Keys at or beyond context_lens are never loaded. m is the maximum of the unit itself in 16 bits: its largest
-// weight is then 1, which rounds to itself, and the unit's product is scaled to the running
-// maximum (raised lazily, past 2^8 only) in fp32. Against 64 bits, before that (weights against
-// the running maximum) and now: 12 layers of a GPT-2 step 4.30e-4 -> 4.16e-4, 64 GPT-2
-// sequences 8.45e-4 -> 8.34e-4, 24/8 heads of 128 in blocks of 32 1.439e-3 -> 1.432e-3; it
-// costs 0-0.3 us a call (8 GPT-2 sequences of 16-1000 tokens 8.3 -> 8.7 us).
+// rounding of the output. Keys at or beyond context_lens are never loaded.
+// m is the maximum of the unit itself in 16 bits: its largest weight is then 1, which rounds to
+// itself, and the unit's product is scaled to the running maximum (raised lazily, past 2^8
+// only) in fp32. Against 64 bits, before that (weights against the running maximum) and now:
+// 12 layers of a GPT-2 step 4.30e-4 -> 4.16e-4, 64 GPT-2 sequences 8.45e-4 -> 8.34e-4, 24/8
+// heads of 128 in blocks of 32 1.439e-3 -> 1.432e-3; it costs 0-0.3 us a call (8 GPT-2
+// sequences of 16-1000 tokens 8.3 -> 8.7 us).
 #include "attention.h"
 
 namespace pkv {
@@ -870,7 +871,9 @@ int launch_nw(const AttnParams& p, hipStream_t stream) {
     // Where the pairs fill the GPU by themselves, or the scan does not reach, contexts of less
     // than 32 units a wave are not cut; none are where the counters do not reach.
     cut.long_from = NW * 32;
-    const bool can = p.ws_cnt && p.num_seqs * units < ((int64_t)1 << 31);
+    // (Up to 2^30 units a batch: the search's run, which starts there where none is cut, then
+    // ends at once and stays far inside 32 bits.)
+    const bool can = p.ws_cnt && p.num_seqs * units <= ((int64_t)1 << 30);
     if (can && p.num_seqs <= kMaxScanSeqs) {
         // Many pairs of long contexts: runs for two rounds, or the longest context would be
         // walked whole (250 sequences of 512-8192 tokens, 8/2 heads, bf16: 219 -> 189 us; 60 of

@@ -79,9 +79,9 @@ class _Workspaces:
     of two and a buffer that had to grow is kept, not freed: a graph captured on that
     stream earlier replays into it (the kept ones add up to less than the one in use).
     A capture that finds none large enough gets one of its own, shared by its later calls
-    and cleared once, at its first call, by every replay (one fill node, not one a layer). After a call that did not complete (a
-    launch error, a reset device), `reset()` drops the buffers so the next call gets a
-    zero-filled one."""
+    and cleared once, at its first call, by every replay (one fill node, not one a layer).
+    After a call that did not complete (a launch error, a reset device), `reset()` drops the
+    buffers so the next call gets a zero-filled one."""
 
     def __init__(self) -> None:
         self._lock = threading.Lock()

@@ -74,7 +74,7 @@ CASES = [
     (8, 2, 2, 64, 700, torch.bfloat16, ()),
     (5, 2, 4, 128, 600, torch.float32, (1, 100)),                    # fp32
     (6, 2, 3, 128, 900, torch.bfloat16, (1, 300)),                   # groups that are no power of two
-    (5, 2, 6, 64, 700, torch.float16, (2, 257)),  
+    (5, 2, 6, 64, 700, torch.float16, (2, 257)),
 ]
 
 
