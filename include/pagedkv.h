@@ -132,7 +132,8 @@ int64_t pkv_paged_attention_decode_workspace_bytes(int64_t num_seqs, int64_t num
  * and at most 1024 sequences, run the persistent MFMA kernel (equal runs of 16-key
  * blocks per workgroup, then a small merge kernel for the sequences the runs cut);
  * fp32 batches with one or two heads of 64 a KV head (block size 16) run the register kernel
- * and its merge kernel; any other batch of head_dims 32..128 (multiples of 16), groups up
+ * (256-token partitions, merged in place, in large batches by a second kernel to the same
+ * bits); any other batch of head_dims 32..128 (multiples of 16), groups up
  * to 16 and power-of-two block sizes from 8 runs the one-launch MFMA kernel (contexts cut
  * into runs that fit the GPU, merged in place), 16-bit groups above 16 the prefill kernel,
  * the rest the generic kernel.

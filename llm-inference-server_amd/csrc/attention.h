@@ -72,8 +72,9 @@ int launch_prompt_split_f32(const AttnParams& p, hipStream_t stream);
 // Whether the batch's row tiles make at most two and a quarter rounds of the GPU there.
 bool prompt_split_f32_few(const AttnParams& p);
 // fp32 register kernel (attn_decode.hip): the shapes where it beats the kernel
-// above; it appends nothing itself.
+// above; and whether it takes the fused append of p.app_* (16-byte source rows, small batches).
 bool decode_f32_applies(const AttnParams& p);
+bool decode_f32_appends(const AttnParams& p);
 int launch_decode_f32(const AttnParams& p, hipStream_t stream);
 // True when launch_prefill_attention runs the MFMA kernel for these parameters (with
 // p.app_* set: including the fused append, whose source rows must be 16-byte aligned).

@@ -1,16 +1,16 @@
 // Paged decode attention for fp32 pools, block_size 16, head_dim 64, one or two query heads per
-// KV head: a partition kernel with K/V staged in registers, and a split-KV merge kernel.
+// KV head: a partition kernel with K/V staged in registers, which appends the new rows and
+// merges the partitions itself or, in large batches, leaves both to launches of their own.
 //
-// Bound: HBM and the arithmetic beside it. With so few heads a group the one-launch MFMA kernel
-// (attn_decode_split.hip) spends its fp32 matrix steps on 16 columns of which one or two count;
-// here each product is computed once. Measured, us a call replayed from a graph, this kernel
-// first, 12 heads: 8 sequences of 16-500 tokens 8.3 vs 11.3, 16 of 500-1000 18.2 vs 20.7, 32 of
-// 16-1000 22.7 vs 23.7, 64 of 200-3000 114 vs 129, 22 of 16-1000 18.8 vs 18.8; issued eagerly
-// its second launch can cost the host more than that (22 of 16-1000 with the append 24.7 vs
-// 22.8), but a rule on sizes would have an eager step and its captured form, which is told the
-// longest context its tables allow, run different kernels. Groups of 2, 6 KV heads: 64 of
-// 500-2000 46 vs 57; of 4 the other is even or faster (8 of 16-1000 10.7 vs 9.6), of 8 faster
-// (200 of 500-2000 68 vs 61).
+// Bound: HBM and the arithmetic beside it, the start and the merge in small batches. With so few
+// heads a group the one-launch MFMA kernel (attn_decode_split.hip) spends its fp32 matrix steps
+// on 16 columns of which one or two count; here each product is computed once. Measured, us a
+// call replayed from a graph, this kernel first, 12 heads: 8 sequences of 16-500 tokens 8.4 vs
+// 14.2, 16 of 500-1000 17.4 vs 22.8, 22 of 16-1000 19.4 vs 22.9, 64 of 200-3000 106 vs 129.
+// Groups of 2, 6 KV heads: 64 of 500-2000 48 vs 59; of 4 the other is even or faster (8 of
+// 16-1000 10.7 vs 9.6), of 8 faster (200 of 500-2000 68 vs 61). A rule on sizes would have an
+// eager step and its captured form, which is told the longest context its tables allow, run
+// different kernels.
 //
 //  * Work unit = (KV head, 256-token partition, sequence): one 256-thread workgroup of 4
 //    wave64s, 64 tokens (4 blocks) per wave.
@@ -18,8 +18,9 @@
 //    with readlane), then all K loads of the 4 blocks at once, the scores, then all V loads
 //    at once, issued before the softmax so they are in flight while it runs.
 //  * Split-KV: a sequence that fits one partition is finished in place; otherwise each
-//    partition writes its partial (max, denominator, unnormalised output) and the second
-//    kernel on the same stream merges them with the log-sum-exp rule.
+//    partition writes its partial (max, denominator, unnormalised output), and the last
+//    workgroup of the (sequence, KV head) to end, or a second kernel on the same stream, merges
+//    them in order with the log-sum-exp rule.
 // Keys at or beyond context_lens are never loaded.
 #include <type_traits>
 
@@ -45,7 +46,68 @@ __device__ __forceinline__ float chunk_dot(const Vec16& k, const Vec16& q, float
 __device__ __forceinline__ Vec16 kv_load16(const void* ptr) { return load16_stream(ptr); }
 __device__ __forceinline__ uint2 kv_load8(const void* ptr) { return load8_stream(ptr); }
 
-template <int D, int G>
+// A pair of a partial. FUSED: agent-scope accesses, written through to where every XCD's
+// agent-scope loads read (the merging workgroup may run behind another L2); else another
+// launch reads what one wrote.
+template <bool FUSED>
+__device__ __forceinline__ void put_pair(float* at, float x, float y) {
+    uint64_t* to = reinterpret_cast<uint64_t*>(at);
+    const uint64_t v = (uint64_t)__builtin_bit_cast(uint32_t, y) << 32 | __builtin_bit_cast(uint32_t, x);
+    if constexpr (FUSED) __hip_atomic_store(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *to = v;
+}
+template <bool FUSED>
+__device__ __forceinline__ float2 get_pair(float* at) {
+    uint64_t* from = reinterpret_cast<uint64_t*>(at);
+    uint64_t v;
+    if constexpr (FUSED) v = __hip_atomic_load(from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else v = *from;
+    return make_float2(__builtin_bit_cast(float, (uint32_t)v), __builtin_bit_cast(float, (uint32_t)(v >> 32)));
+}
+
+// Merge of a (KV head, sequence)'s partitions by one wave, each lane two adjacent head_dim
+// elements of one head: the online log-sum-exp rule over them in order, CH at a time.
+template <int D, int G, bool FUSED>
+__device__ __forceinline__ void merge_partitions(const AttnParams& p, int seq, int kvh, int n_parts) {
+    constexpr int CH = 16;                    // partitions whose loads are in flight together
+    static_assert(D % 2 == 0 && G * D / 2 <= 64, "one wave");
+    const int lane = lane_id();
+    if (lane >= G * D / 2) return;
+    const int head = kvh * G + 2 * lane / D, d = 2 * lane % D;
+    const int64_t base = ((int64_t)seq * p.num_heads + head) * p.max_parts;
+    float* ml = p.ws_ml + base * 2;
+    float* o = p.ws_o + base * D + d;
+    float M = kNegInf, L = 0.f, O0 = 0.f, O1 = 0.f;
+    for (int pt0 = 0; pt0 < n_parts; pt0 += CH) {
+        float2 mlv[CH], ov[CH];
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            const bool in = pt0 + j < n_parts;
+            mlv[j] = in ? get_pair<FUSED>(ml + (pt0 + j) * 2) : make_float2(kNegInf, 0.f);
+            ov[j] = in ? get_pair<FUSED>(o + (int64_t)(pt0 + j) * D) : make_float2(0.f, 0.f);
+        }
+        float Mc = M;
+#pragma unroll
+        for (int j = 0; j < CH; ++j) Mc = fmaxf(Mc, mlv[j].x);
+        const float rescale = M == kNegInf ? 0.f : fast_exp2(M - Mc);
+        L *= rescale;
+        O0 *= rescale;
+        O1 *= rescale;
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            const float sc = mlv[j].x == kNegInf ? 0.f : fast_exp2(mlv[j].x - Mc);
+            L += sc * mlv[j].y;
+            O0 += sc * ov[j].x;
+            O1 += sc * ov[j].y;
+        }
+        M = Mc;
+    }
+    float* orow = reinterpret_cast<float*>(p.out) + (int64_t)seq * p.out_st + (int64_t)head * p.out_sh;
+    orow[d] = O0 / L;
+    orow[d + 1] = O1 / L;
+}
+
+template <int D, int G, bool FUSED>
 __global__ __launch_bounds__(kWaves * 64) void paged_decode_kernel(const AttnParams p) {
     using T = float;
     constexpr int ISZ = (int)sizeof(T);
@@ -114,12 +176,28 @@ __global__ __launch_bounds__(kWaves * 64) void paged_decode_kernel(const AttnPar
         vblk[b] = vbase + id * block_bytes;
     }
 
+    // ------------------------------------------------------------ fused append
+    // The new token is the context's last key: the wave that holds it takes its row from the
+    // caller (its pool slot is not read in this launch) and stores it, lanes 0 .. CHUNKS-1 the
+    // K row, CHUNKS .. 2 CHUNKS-1 the V row.
+    const bool has_new = FUSED && p.app_slots && ctx - 1 >= wstart && ctx - 1 < wstart + kTPW;
+    const int new_tok = has_new ? ctx - 1 - wstart : -1;
+    const char* knew = reinterpret_cast<const char*>(p.app_k) + ((int64_t)seq * p.app_st + (int64_t)kvh * p.app_sh) * ISZ;
+    const char* vnew = reinterpret_cast<const char*>(p.app_v) + ((int64_t)seq * p.app_st + (int64_t)kvh * p.app_sh) * ISZ;
+    static_assert(2 * CHUNKS <= 64, "one piece per lane");
+    Vec16 new_piece = Vec16{{0u, 0u, 0u, 0u}};
+    int64_t new_slot = -1;
+    if (has_new && lane < 2 * CHUNKS) {
+        new_slot = p.app_slots[seq];
+        new_piece = load16((lane < CHUNKS ? knew : vnew) + lane % CHUNKS * 16);
+    }
+
     // ------------------------------------------------------------ K, scores, V issue
-    // Fast path (wave-uniform): all 64 tokens inside the context and all 4 block ids
-    // inside the pool. Its loads are unconditional and nothing is zero-filled; the other
+    // Fast path (wave-uniform): all 64 tokens inside the context and in the pool, all 4 block
+    // ids inside it. Its loads are unconditional and nothing is zero-filled; the other
     // waves (at most the last two of a sequence) predicate every load and zero what they
     // skip, which costs ~15% more VALU instructions.
-    bool full = wstart + kTPW <= ctx;
+    bool full = wstart + kTPW <= ctx && !has_new;
 #pragma unroll
     for (int b = 0; b < kBPW; ++b) full = full && live[b];
     // K: each load instruction reads 8 tokens x one whole 128-byte line of their rows.
@@ -135,10 +213,10 @@ __global__ __launch_bounds__(kWaves * 64) void paged_decode_kernel(const AttnPar
 #pragma unroll
             for (int gr = 0; gr < KGRP; ++gr) {
                 if (FULL || live[b]) {
+                    const char* row = kblk[b] + (k_lane_off + (uint32_t)(gr * 8) * slot_bytes);
+                    if (!FULL && b * kBS + gr * 8 + ktok == new_tok) row = knew + kj * 16;
 #pragma unroll
-                    for (int i = 0; i < CPL; ++i)
-                        kv[b][gr][i] = kv_load16(kblk[b] + (k_lane_off + (uint32_t)(gr * 8) * slot_bytes +
-                                                            (uint32_t)(i * KLPT * 16)));
+                    for (int i = 0; i < CPL; ++i) kv[b][gr][i] = kv_load16(row + i * KLPT * 16);
                 } else {
 #pragma unroll
                     for (int i = 0; i < CPL; ++i) kv[b][gr][i] = Vec16{{0u, 0u, 0u, 0u}};
@@ -169,7 +247,8 @@ __global__ __launch_bounds__(kWaves * 64) void paged_decode_kernel(const AttnPar
                 vv[st] = kv_load8(vblk[b] + off);
             } else {
                 vv[st] = make_uint2(0u, 0u);
-                if (live[b] && wstart + t_rel < ctx) vv[st] = kv_load8(vblk[b] + off);
+                if (live[b] && wstart + t_rel < ctx)
+                    vv[st] = kv_load8(t_rel == new_tok ? vnew + vchunk * 8 : vblk[b] + off);
             }
         }
     };
@@ -212,6 +291,10 @@ __global__ __launch_bounds__(kWaves * 64) void paged_decode_kernel(const AttnPar
     for (int g = 0; g < G; ++g)
 #pragma unroll
         for (int e = 0; e < EPV; ++e) acc[g][e] = fold_lanes<VLPT>(acc[g][e]);
+    if (has_new && (uint64_t)new_slot < (uint64_t)p.num_blocks * kBS) {
+        const int64_t dst = new_slot / kBS * block_bytes + new_slot % kBS * (int64_t)slot_bytes + lane % CHUNKS * 16;
+        store16(const_cast<char*>(lane < CHUNKS ? kbase : vbase) + dst, new_piece);
+    }
     if (vslot == 0) {
 #pragma unroll
         for (int g = 0; g < G; ++g)
@@ -228,103 +311,79 @@ __global__ __launch_bounds__(kWaves * 64) void paged_decode_kernel(const AttnPar
     lds_barrier();
 
     // ------------------------------------------------------------ merge the waves
-    const int head0 = kvh * G;
-    for (int idx = (int)threadIdx.x; idx < G * D; idx += kWaves * 64) {
-        const int g = idx / D, d = idx - g * D;
+    // In the first wave, two adjacent head_dim elements a lane.
+    if (wave != 0) return;
+    static_assert(G * D / 2 <= 64, "one wave");
+    if (lane < G * D / 2) {
+        const int g = 2 * lane / D, d = 2 * lane % D;
         float M = kNegInf;
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) M = fmaxf(M, s_ml[w][g][0]);
-        float L = 0.f, O = 0.f;
+        float L = 0.f, O0 = 0.f, O1 = 0.f;
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
             const float mw = s_ml[w][g][0];
             const float sc = mw == kNegInf ? 0.f : fast_exp2(mw - M);
             L += sc * s_ml[w][g][1];
-            O += sc * s_acc[w][g][d];
+            O0 += sc * s_acc[w][g][d];
+            O1 += sc * s_acc[w][g][d + 1];
         }
+        const int head = kvh * G + g;
         if (n_parts == 1) {
-            T* orow = reinterpret_cast<T*>(p.out) + (int64_t)seq * p.out_st + (int64_t)(head0 + g) * p.out_sh;
-            orow[d] = from_f32<T>(O / L);
+            float* orow = reinterpret_cast<float*>(p.out) + (int64_t)seq * p.out_st + (int64_t)head * p.out_sh;
+            orow[d] = O0 / L;
+            orow[d + 1] = O1 / L;
         } else {
-            const int64_t slot = ((int64_t)seq * p.num_heads + head0 + g) * p.max_parts + part;
-            p.ws_o[slot * D + d] = O;
-            if (d == 0) {
-                p.ws_ml[slot * 2] = M;
-                p.ws_ml[slot * 2 + 1] = L;
-            }
+            const int64_t slot = ((int64_t)seq * p.num_heads + head) * p.max_parts + part;
+            put_pair<FUSED>(p.ws_o + slot * D + d, O0, O1);
+            if (d == 0) put_pair<FUSED>(p.ws_ml + slot * 2, M, L);
         }
     }
+    if (!FUSED || n_parts == 1) return;
+
+    // ------------------------------------------------------------ merge the partitions
+    // By the last workgroup of the (sequence, KV head) to get here, which returns the counter
+    // to zero for the next call. The stores above are all this wave's: s_waitcnt vmcnt(0) holds
+    // it until each is acknowledged from the agent's coherence point, before the counter moves.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    uint32_t* cnt = p.ws_cnt + ((int64_t)seq * p.num_kv_heads + kvh);
+    uint32_t arrived = 0;
+    if (lane == 0) arrived = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane(arrived) != (uint32_t)(n_parts - 1)) return;
+    if (lane == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    merge_partitions<D, G, true>(p, seq, kvh, n_parts);
 }
 
-// Split-KV merge, launched after the partition kernel on the same stream (stream
-// order is the only synchronisation: no fences, no atomics). One workgroup per
-// (KV head, sequence) merges the partitions' (max, denominator, output) with the
-// log-sum-exp rule; sequences that fit one PART-token partition were finished by the
-// partition kernel and are skipped.
-// Threads of a merge workgroup: the G * D / 2 element pairs of one KV head, in whole
-// waves, at most 256 (one wave for a head_dim-64 group of one).
-template <int G, int D>
-constexpr int kCombineThreads = (G * D / 2 + 63) / 64 * 64 < 256 ? (G * D / 2 + 63) / 64 * 64 : 256;
-
+// The same merge as a launch of its own, one wave per (KV head, sequence).
 template <int D, int G>
-__global__ __launch_bounds__((kCombineThreads<G, D>)) void paged_decode_combine_kernel(const AttnParams p) {
-    using T = float;
-    constexpr int PART = kDecodePart;
+__global__ __launch_bounds__(64) void paged_decode_combine_kernel(const AttnParams p) {
     const int kvh = (int)blockIdx.x;
     const int seq = (int)blockIdx.y;
     int64_t ctx64 = p.ctx_lens[seq];
     ctx64 = ctx64 < (int64_t)p.table_width * kBS ? ctx64 : (int64_t)p.table_width * kBS;
     ctx64 = ctx64 < (int64_t)p.max_parts * kDecodePart ? ctx64 : (int64_t)p.max_parts * kDecodePart;
-    const int n_parts = (int)((ctx64 + PART - 1) / PART);
-    if (n_parts <= 1) return;
-    const int head0 = kvh * G;
-    constexpr int CH = 16;  // partitions whose loads are in flight together
-    static_assert(D % 2 == 0, "pairs of head_dim elements");
-    // Each thread merges two adjacent head_dim elements (8-byte loads), so G * D <= 512
-    // (every shape the partition kernels take) is one pass of dependent loads.
-    for (int idx = (int)threadIdx.x; idx < G * D / 2; idx += kCombineThreads<G, D>) {
-        const int g = (2 * idx) / D, d = 2 * idx - g * D;
-        const int64_t base = ((int64_t)seq * p.num_heads + head0 + g) * p.max_parts;
-        const float2* ml = reinterpret_cast<const float2*>(p.ws_ml) + base;
-        const float2* o = reinterpret_cast<const float2*>(p.ws_o + base * D + d);
-        // Online log-sum-exp over the partitions, CH at a time.
-        float M = kNegInf, L = 0.f, O0 = 0.f, O1 = 0.f;
-        for (int pt0 = 0; pt0 < n_parts; pt0 += CH) {
-            float2 mlv[CH], ov[CH];
-#pragma unroll
-            for (int j = 0; j < CH; ++j) {
-                const bool in = pt0 + j < n_parts;
-                mlv[j] = in ? ml[pt0 + j] : make_float2(kNegInf, 0.f);
-                ov[j] = in ? o[(int64_t)(pt0 + j) * (D / 2)] : make_float2(0.f, 0.f);
-            }
-            float Mc = M;
-#pragma unroll
-            for (int j = 0; j < CH; ++j) Mc = fmaxf(Mc, mlv[j].x);
-            const float rescale = M == kNegInf ? 0.f : fast_exp2(M - Mc);
-            L *= rescale;
-            O0 *= rescale;
-            O1 *= rescale;
-#pragma unroll
-            for (int j = 0; j < CH; ++j) {
-                const float sc = mlv[j].x == kNegInf ? 0.f : fast_exp2(mlv[j].x - Mc);
-                L += sc * mlv[j].y;
-                O0 += sc * ov[j].x;
-                O1 += sc * ov[j].y;
-            }
-            M = Mc;
-        }
-        T* orow = reinterpret_cast<T*>(p.out) + (int64_t)seq * p.out_st + (int64_t)(head0 + g) * p.out_sh;
-        orow[d] = from_f32<T>(O0 / L);
-        orow[d + 1] = from_f32<T>(O1 / L);
-    }
+    const int n_parts = (int)((ctx64 + kDecodePart - 1) / kDecodePart);
+    if (n_parts > 1) merge_partitions<D, G, false>(p, seq, kvh, n_parts);
 }
+
+// Workgroups, at the bound of the launch, up to which it appends and merges by itself. us a call
+// against three launches (append, partitions, merge), with the append, 12 heads, eager and
+// replayed: 2 sequences of 4-1107 tokens 18.1 -> 13.6, 10.1 -> 8.0; 8 of 16-500 18.5 -> 13.5, 10.9
+// -> 8.4; 32 of 16-1024 25.4 -> 21.7, 24.8 -> 22.0. Above, the waves that stay for the merge cost
+// more than the launches: 64 of 200-3000 replayed, 9216 workgroups, 108.9 -> 115.7; 200 of
+// 500-2000 272 -> 280. Both forms compute the same bits, whichever a captured step's bound takes.
+constexpr int64_t kFusedWgs = 2048;
+
+bool fused_size(const AttnParams& p) { return (int64_t)p.num_seqs * p.num_kv_heads * p.max_parts <= kFusedWgs; }
 
 template <int D, int G>
 int launch_g(const AttnParams& p, dim3 grid, hipStream_t stream) {
-    paged_decode_kernel<D, G><<<grid, kWaves * 64, 0, stream>>>(p);
+    const bool fused = fused_size(p) && (p.max_parts == 1 ? p.app_slots != nullptr : p.ws_cnt != nullptr);
+    if (fused) paged_decode_kernel<D, G, true><<<grid, kWaves * 64, 0, stream>>>(p);
+    else paged_decode_kernel<D, G, false><<<grid, kWaves * 64, 0, stream>>>(p);
     int rc = check_launch("paged decode attention");
-    if (rc || p.max_parts == 1) return rc;
-    paged_decode_combine_kernel<D, G><<<dim3(grid.x, grid.z), kCombineThreads<G, D>, 0, stream>>>(p);
+    if (rc || fused || p.max_parts == 1) return rc;
+    paged_decode_combine_kernel<D, G><<<dim3(grid.x, grid.z), 64, 0, stream>>>(p);
     return check_launch("paged decode combine");
 }
 
@@ -340,6 +399,12 @@ bool decode_f32_applies(const AttnParams& p) {
                            (uint64_t)(p.q_st * 4) | (uint64_t)(p.q_sh * 4) | (uint64_t)(p.sb * 4) |
                            (uint64_t)(p.ss * 4) | (uint64_t)(p.sh * 4);
     return probe % 16 == 0;
+}
+
+bool decode_f32_appends(const AttnParams& p) {
+    if (!fused_size(p) || (p.max_parts > 1 && !p.ws_cnt)) return false;
+    return (((uint64_t)(uintptr_t)p.app_k | (uint64_t)(uintptr_t)p.app_v | (uint64_t)(p.app_st * 4) |
+             (uint64_t)(p.app_sh * 4)) % 16) == 0;
 }
 
 int launch_decode_f32(const AttnParams& p, hipStream_t stream) {

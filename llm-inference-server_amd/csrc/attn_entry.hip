@@ -186,12 +186,13 @@ int decode_impl(void* out, int64_t out_stride_t, int64_t out_stride_h, const voi
         p.app_st = app->st;
         p.app_sh = app->sh;
         p.app_slots = app->slots;
-        // The fp32 register kernel reads the pool only. The MFMA kernels write the rows themselves: the persistent one by 4-byte copies
+        // The tuned kernels write the rows themselves: the persistent one by 4-byte copies
         // (even strides, 4-byte aligned sources), the others from 16-byte rows. Any other
         // kernel gets the append launch first.
-        const bool fuse = mfma ? app->st % 2 == 0 && app->sh % 2 == 0 &&
-                                     ((uintptr_t)app->k_new | (uintptr_t)app->v_new) % 4 == 0
-                               : !f32_regs && (decode_split_applies(p, dtype) || prefill_tuned(p, dtype));
+        const bool fuse = mfma       ? app->st % 2 == 0 && app->sh % 2 == 0 &&
+                                           ((uintptr_t)app->k_new | (uintptr_t)app->v_new) % 4 == 0
+                          : f32_regs ? decode_f32_appends(p)
+                                     : decode_split_applies(p, dtype) || prefill_tuned(p, dtype);
         if (!fuse && (rc = append_first())) return rc;
     }
     if (mfma) {

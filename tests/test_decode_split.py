@@ -182,12 +182,26 @@ REGISTER_EDGES = [1, 15, 16, 17, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 
                   576, 767, 768, 769, 1000, 1023, 1024, 1025, 1279, 1280]
 
 
-@pytest.mark.parametrize("kv,group", [(12, 1), (3, 2)])
+@pytest.mark.parametrize("kv,group", [(12, 1), (3, 2), (16, 1), (14, 2)])   # the last two past 2048 workgroups
 @pytest.mark.parametrize("ctx", [REGISTER_EDGES, REGISTER_EDGES[:15]], ids=["partitions", "one partition"])
 @pytest.mark.parametrize("fused", [False, True], ids=["plain", "append"])
 def test_fp32_register_kernel(kv, group, ctx, fused):
     """attn_decode.hip: fp32, head_dim 64, groups of 1 and 2."""
     _check(_batch(ctx, dtype=torch.float32, d=64, bs=16, kv=kv, group=group, seed=group), fused=fused)
+
+
+def test_fp32_register_kernel_appends_rows_off_16_bytes():
+    """By the append launch, in front of the same kernel: the same bits."""
+    b = _batch(REGISTER_EDGES, dtype=torch.float32, d=64, bs=16, kv=3, group=1)
+    out, k, v, slots = _run(b, fused=True)
+    kd, vd = b["k"].cuda(), b["v"].cuda()
+    odd = [torch.empty(t.numel() + 1, device="cuda")[1:].view(t.shape).copy_(t) for t in (b["k_new"], b["v_new"])]
+    assert all(t.data_ptr() % 16 for t in odd)
+    got = paged_attention_hip_launch(b["q"].cuda(), kd, vd, b["tables"].cuda(), b["ctx"].cuda(),
+                                     torch.ones(len(slots), dtype=torch.long).cuda(), 0.125, append=(*odd, slots.cuda()))
+    assert torch.equal(got.cpu(), out)
+    assert torch.equal(torch.nan_to_num(kd.cpu()), torch.nan_to_num(k))
+    assert torch.equal(torch.nan_to_num(vd.cpu()), torch.nan_to_num(v))
 
 
 def _captured(b, width, bound):
@@ -208,7 +222,7 @@ def _captured(b, width, bound):
 
 
 @pytest.mark.parametrize("n,dtype,kv,group,d,bs,lo,hi,bound", [
-    (24, torch.float32, 12, 1, 64, 16, 40, 500, 1024), (8, torch.float32, 6, 2, 64, 16, 40, 300, 1024),
+    (24, torch.float32, 12, 1, 64, 16, 40, 500, 1024), (24, torch.float32, 12, 1, 64, 16, 40, 500, 4096), (8, torch.float32, 6, 2, 64, 16, 40, 300, 1024),
     (32, torch.float32, 4, 4, 64, 16, 40, 500, 1024), (8, torch.float32, 8, 1, 128, 16, 40, 250, 2048),
     (64, torch.float16, 12, 1, 64, 16, 40, 500, 1024), (43, torch.float16, 12, 1, 64, 16, 40, 512, 1024),
     (8, torch.float16, 12, 1, 64, 16, 17, 700, 1024), (64, torch.bfloat16, 8, 4, 128, 16, 30, 250, 1024),
@@ -225,9 +239,9 @@ def test_a_captured_call_computes_the_eager_one(n, dtype, kv, group, d, bs, lo, 
     eager = _run(b, fused=False)[0]
     out, census = _captured(b, -(-bound // bs), bound)
     assert torch.equal(out, eager)
-    # One launch, but for the fp32 register kernel and its merge.
+    # One launch, but for the fp32 register kernel's merge at a bound of more than 2048 workgroups.
     registers = dtype == torch.float32 and d == 64 and group <= 2
-    assert census == {"kernel": 2 if registers else 1}
+    assert census == {"kernel": 2 if registers and n * kv * -(-bound // 256) > 2048 else 1}
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
